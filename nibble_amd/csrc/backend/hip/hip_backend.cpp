@@ -163,13 +163,14 @@ void HipBackend::reserve(const ReserveParams& rp) {
   if (floats < 0) throw Error("reserve: invalid n_heads " + str(rp.n_heads));
   const int64_t ws_floats = std::max(floats, nbhs_attn_prefill_workspace_bound(cu_count_));
   // Quantized activations of up to max_rows rows of width up to max_width: the largest companion-format buffer
-  // over the quantized types (their row-major and residue-major forms have one size).
+  // over the quantized types (for the K types, of their two forms).
   int64_t acts = 0;
   if (rp.max_rows > 0)
     for (const int t : {2, 6, 7, 8, 12, 13, 14}) {
       const int64_t be = nbh_quant::block_elems(t), w = rp.max_width / be * be;
       if (w > 0) {
-        const int64_t b = nbhs_quant_act_bytes(t, rp.max_rows, w);
+        const int64_t b = nbh_quant::is_k(t) ? nbhs_quant_act_rm_bytes(t, rp.max_rows, w)  // the larger form
+                                             : nbhs_quant_act_bytes(t, rp.max_rows, w);
         if (b < 0) throw Error("reserve: activation scratch for max_rows=" + str(rp.max_rows) + " max_width=" +
                                str(rp.max_width) + " is too large");
         acts = std::max(acts, b);
@@ -482,15 +483,15 @@ void HipBackend::matmul_multi(std::span<const Tensor* const> ws, const float* x,
   const bool fuse = n <= 4 && reinterpret_cast<uintptr_t>(x) % 16 == 0 && in % 4 == 0;
   int done_act = -1;
   for (const int t : types) {
-    // the tiled kernels from more than 16 rows on (K types: 8, Q6_K: 4), whose K-type activations are in
-    // residue-major order
+    // the tiled kernels from more than 16 rows on (K types: 8, Q6_K: 4), whose K-type activations take a form of
+    // their own
     const int64_t min_rows =
         t == nbh_quant::kQ6_K ? kQ6KTiledMinRows : nbh_quant::is_k(t) ? kKTiledMinRows : kGemvMaxRows;
     const bool tiled = n > min_rows;
     const bool rm = tiled && nbh_quant::is_k(t);
     const int act_key = 2 * nbh_quant::act_of(t) + (rm ? 1 : 0);
     if (!fuse && act_key != done_act) {
-      const int64_t ab = nbhs_quant_act_bytes(t, n, in);
+      const int64_t ab = rm ? nbhs_quant_act_rm_bytes(t, n, in) : nbhs_quant_act_bytes(t, n, in);
       if (ab < 0) throw Error("matmul: invalid quantized shape");
       ensure(acts_buf_, acts_buf_bytes_, size_t(ab));
       check(rm ? nbhs_quantize_acts_rm(t, x, n, in, acts_buf_, stream_)

@@ -23,6 +23,7 @@
 // launch (into LDS, once per wave and block), with the same bits as the standalone quantizer.
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
 
 #include "backend/hip/kernel_timing.h"
 #include "kernels/quant_layout.h"
@@ -58,6 +59,11 @@ __device__ __forceinline__ float opaque(float v) {
   asm volatile("" : "+v"(v));
   return v;
 }
+
+typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
+typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
+typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
+typedef float floatx4_t __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ int sdot4(uint32_t a, uint32_t b, int c) {
   return __builtin_amdgcn_sdot4(int(a), int(b), c, false);
@@ -114,9 +120,8 @@ __device__ __forceinline__ int nearest_int(float f) {
 
 // One wave per 256-element super-block; lane l = 8k + w holds elements 32k + w + 8i (i < 4) of sub-block k: the four
 // elements of residue word w, which it stores as word w of the sub-block (residue order, quant_layout.h).
-// RM: the super-block's quants in residue-major order instead (byte 32 w + 4 k + i = element 32 k + w + 8 i), so
-// that residue w's 32 quants - the ones that feed the reference's integer lane w - are contiguous (the order
-// qgemm_k_kernel reads).
+// RM: the tiled K kernels' operand form instead (quant_layout.h, kActQ8_K16): 16 times each quant as fp16, residue
+// by residue, and each sub-block's sum of its quants as two fp16 digits.
 template <bool RM>
 __global__ __launch_bounds__(64) void quantize_q8k_kernel(const float* __restrict__ x, int64_t in,
                                                           int8_t* __restrict__ qs, float* __restrict__ dq,
@@ -142,24 +147,40 @@ __global__ __launch_bounds__(64) void quantize_q8k_kernel(const float* __restric
     if (oa > amax || (oa == amax && oi < idx)) amax = oa, mx = om, idx = oi;
   }
   nan = __builtin_amdgcn_ballot_w64(nan) != 0;
-  uint32_t word = 0;
-  int b0 = 0, b1 = 0;  // this lane's share of the sub-block's two 16-sums (elements w, w + 8 | w + 16, w + 24)
+  int q[4] = {0, 0, 0, 0};
   float d = 0.f;
   if (amax != 0.f) {
     const float iscale = __fdiv_rn(-127.f, mx);
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const float sv = __fmul_rn(iscale, v[e]);
-      const int q = sv != sv ? 0 : nearest_int(fminf(127.f, fmaxf(-127.f, sv)));
-      if (e < 2) b0 += q; else b1 += q;
-      word |= uint32_t(q & 0xFF) << (8 * e);
+      q[e] = sv != sv ? 0 : nearest_int(fminf(127.f, fmaxf(-127.f, sv)));
     }
     d = __fdiv_rn(1.f, iscale);
   }
+  // the sub-block's two 16-sums (elements w, w + 8 | w + 16, w + 24 of each lane)
+  int b0 = q[0] + q[1], b1 = q[2] + q[3];
 #pragma unroll
   for (int m = 1; m < 8; m <<= 1) b0 += __shfl_xor(b0, m, 64), b1 += __shfl_xor(b1, m, 64);
-  reinterpret_cast<uint32_t*>(qs + i * 256)[RM ? 8 * w + k : lane] = word;
-  if (w == 0) bsums[i * 16 + 2 * k] = int16_t(b0), bsums[i * 16 + 2 * k + 1] = int16_t(b1);
+  if constexpr (RM) {
+    // chunk k / 2 of residue w: sub-block k's elements (0, 2) at halves 2 (k % 2), (1, 3) at 4 + 2 (k % 2)
+    _Float16* o = reinterpret_cast<_Float16*>(qs) + i * 256 + 32 * w + 8 * (k >> 1) + 2 * (k & 1);
+    *reinterpret_cast<half2_t*>(o) = half2_t{_Float16(16 * q[0]), _Float16(16 * q[2])};
+    *reinterpret_cast<half2_t*>(o + 4) = half2_t{_Float16(16 * q[1]), _Float16(16 * q[3])};
+    if (w == 0) {
+      _Float16* bs = reinterpret_cast<_Float16*>(bsums) + i * 16;
+      const int sum = b0 + b1;
+      const int at = (k & 4) | ((k & 1) << 1) | ((k >> 1) & 1);  // 0, 2, 1, 3 of each four
+      bs[at] = _Float16(sum & 63);
+      bs[8 + at] = _Float16(sum >> 6);
+    }
+  } else {
+    uint32_t word = 0;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) word |= uint32_t(q[e] & 0xFF) << (8 * e);
+    reinterpret_cast<uint32_t*>(qs + i * 256)[lane] = word;
+    if (w == 0) bsums[i * 16 + 2 * k] = int16_t(b0), bsums[i * 16 + 2 * k + 1] = int16_t(b1);
+  }
   if (lane == 0) dq[i] = nan ? __builtin_nanf("") : d;
 }
 
@@ -637,6 +658,7 @@ struct QGemmBatch {  // weights of one type sharing one input; tile0[i]: first r
 
 // Staged quant words as a native vector type (a uint4 copy is a memcpy that keeps the staging share in scratch).
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 typedef int i32x4_t __attribute__((ext_vector_type(4)));  // an integer MFMA result
 
 template <int T, int TJ, int WRT = 64>
@@ -853,299 +875,418 @@ hipError_t launch_legacy(LegacyTile tile, unsigned tiles, int64_t n, hipStream_t
   return nbhs_timing::launch(NBHS_K_QGEMM, qgemm_legacy_kernel<T, 2, 32>, grid, dim3(256), s, B, A, n);
 }
 
-// qgemm_k_kernel: the tiled matmul for the K types on the int8 matrix cores (v_mfma_i32_16x16x32_i8).
+// The tiled K matmuls, on the fp16 matrix cores (v_mfma_f32_16x16x32_f16).
 // The reference's integer lane w of a super-block is aux[w] = sum over the 32 elements e of residue w (four per
-// sub-block) of s(e) * q(e) * a(e), with the sub-block scale s varying along it. s * q is split into slices small
-// enough that each slice's per-element product fits int8, each slice is one exact integer MFMA over the residue
-// (K = 32), and aux[w] = sum_i c_i C_i, exactly:
-//   Q4_K: s = 8 s1 + s0 (s0, s1 < 8), q < 16                        -> s0 q, s1 q            (c = 1, 8)
-//   Q5_K: s = 16 s2 + 4 s1 + s0 (each < 4), q < 32                   -> s0 q, s1 q, s2 q      (c = 1, 4, 16)
-//   Q6_K: s signed 8-bit per 16 elements = 16 s1 + s0 (s0 < 16, -8 <= s1 < 8), q - 32 = 8 u1 + u0 (u0 < 8,
-//         -4 <= u1 < 4)                                              -> s1 u1, s1 u0, s0 u1, s0 u0 (c = 128, 16, 8, 1)
+// sub-block) of s(e) * q(e) * a(e), with the sub-block scale s varying along it. One MFMA contracts exactly a
+// residue. Its A operand is s q / 16, its B operand 16 a (|a| <= 127), both exact in fp16: s q is at most 63 * 31 for
+// Q4_K and Q5_K; for Q6_K s (q - 32) is taken as two operands, s n / 16 for the low nibble n and s (h - 2) for the
+// two high bits h, whose MFMAs share an accumulator. Every product and every partial sum is an integer below 2^24
+// (at most 32 * 4096 * 127), so the fp32 accumulator holds float(aux[w]) exactly, whatever the order: no integer
+// slices to combine and no conversion on the VALU, which the float sums bound (per output and residue a product and
+// an addition are left; the int8 form it replaces took two or more MFMAs and four or more VALU operations).
+// The minimum term's sumi = sum_k m_k b_k (b_k: the sub-block's quant sum, |b_k| <= 4064, m_k <= 63) is one
+// v_mfma_f32_16x16x16_f16 over b_k = 64 (b_k >> 6) + (b_k & 63) against (m_k, 64 m_k), likewise exact.
 // The float arithmetic that follows is the reference's per output and block: d = fp16(d_w) * d_a, sums[w] +=
 // d * aux[w], for Q4_K / Q5_K acc -= (fp16(dmin_w) * d_a) * sumi, result acc + sums[0] + ... + sums[7] - the same
 // operations in the same order as qgemv_kernel, so the same bits.
-// A workgroup (4 waves) takes 64 weight rows and 32 activation rows; each wave 16 weight rows against both 16-row
-// activation groups. Per super-block the raw weight words (quants, high bits), the sub-block scales and minimums
-// (taken out of their packing once, at staging), d / dmin widened, and the activation rows (residue-major Q8_K
-// quants, d, the sub-block sums of the 16-sums) are staged in LDS with 16-byte loads, the next super-block's share
-// of each thread loaded into registers while the current one is computed. A lane (weight row ml, k group kg of the
-// MFMA operand layout) builds its slice operands for residue w from its row's quant word 8 kg + w (the elements of
-// residue w in sub-blocks 2 kg and 2 kg + 1) and the two sub-blocks' scales; the result layout gives it weight rows
-// 4 kg + v (v < 4) of activation row ml of each group: 8 outputs and their 9 float accumulators per lane.
+// An A operand is built in registers from a row's raw words: and / or place a nibble pair in the mantissa of an fp16
+// constant C (C + n ulp(C)), and one packed multiply-add with (s', -C s') leaves s q / 16 exactly.
 template <int T>
-constexpr int k_slices() { return T == kQ4_K ? 2 : T == kQ5_K ? 3 : 4; }
-constexpr int kKTileRows = 64, kKTileActs = 32;
+constexpr int k_slices() { return T == kQ6_K ? 2 : 1; }
 
-typedef uint16_t u16x2_t __attribute__((ext_vector_type(2)));
+// (w & mask) | base as an fp16 pair. The constant base sits in a vector register, so that the pair is one and / or
+// instruction (which takes at most one scalar operand).
+__device__ __forceinline__ half2_t magic(uint32_t w, uint32_t mask, uint32_t base) {
+  asm("" : "+v"(base));
+  return __builtin_bit_cast(half2_t, (w & mask) | base);
+}
+__device__ __forceinline__ half8_t join(half2_t a, half2_t b, half2_t c, half2_t d) {
+  return half8_t{a[0], a[1], b[0], b[1], c[0], c[1], d[0], d[1]};
+}
+__device__ __forceinline__ half2_t pk_fma(half2_t a, half2_t b, half2_t c) { return __builtin_elementwise_fma(a, b, c); }
 
-// Bytes b of the result hold lo16(x_b * y_b) & 0xFF for the four bytes of a word, with x_b, y_b small signed
-// values given as 16-bit lanes: ex / ox the even / odd bytes' x, sy the y of bytes 0 and 1 (lane 0) and of bytes 2
-// and 3 (lane 1). Every product here fits int8, so its low byte is its two's complement.
-__device__ __forceinline__ uint32_t byte_products(u16x2_t ex, u16x2_t ox, u16x2_t sy) {
-  const u16x2_t pe = ex * sy, po = ox * sy;
-  return (__builtin_bit_cast(uint32_t, pe) & 0x00FF00FFu) | ((__builtin_bit_cast(uint32_t, po) & 0x00FF00FFu) << 8);
+// The constants of a lane's two sub-blocks (2 kg and 2 kg + 1), from their staged words (k_scale_words).
+template <int T>
+struct KScales {
+  half2_t s[2], c[2];  // Q4_K / Q5_K: s' and -C s', splat. Q6_K: the two 16-element scales and -64 times them
+  half2_t c6[2];       // Q6_K: -6 times the scales
+  __device__ __forceinline__ void set(uint32_t w0, uint32_t w1) {
+    const uint32_t w[2] = {w0, w1};
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      const half2_t v = __builtin_bit_cast(half2_t, w[b]);
+      if constexpr (T == kQ6_K) {
+        s[b] = v;
+        c[b] = v * half2_t{-64, -64};
+        c6[b] = v * half2_t{-6, -6};
+      } else {
+        s[b] = half2_t{v[0], v[0]};
+        c[b] = half2_t{v[1], v[1]};
+      }
+    }
+  }
+};
+
+// The A operand(s) of residue w for a lane's k group kg (sub-blocks 2 kg, 2 kg + 1), as 8 halves in the order
+// (sub-block 2 kg: elements 0, 2), (2 kg + 1: 0, 2), (2 kg: 1, 3), (2 kg + 1: 1, 3) - the order of kActQ8_K16.
+// Q4_K / Q5_K: q0 the row's quant word 8 kg + w (low nibbles sub-block 2 kg, high nibbles 2 kg + 1), h the high-bit
+// word w. Q6_K: q0, q1 the quant words 16 (kg / 2) + w and + 8, of which nibble kg % 2 belongs to sub-blocks 2 kg and
+// 2 kg + 1; h the word 8 (kg / 2) + w, their bits from 4 (kg % 2) on.
+template <int T>
+__device__ __forceinline__ void k_operand(uint32_t q0, uint32_t q1, uint32_t h, int kg, const KScales<T>& k,
+                                          half8_t (&a)[k_slices<T>()]) {
+  if constexpr (T == kQ6_K) {
+    const int sh = 4 * (kg & 1);
+    const uint32_t w0 = q0 >> sh, w1 = q1 >> sh, t = h >> sh;
+    constexpr uint32_t M = 0x000F000Fu, C = 0x54005400u;  // 64 + n / 16
+    a[0] = join(pk_fma(magic(w0, M, C), k.s[0], k.c[0]), pk_fma(magic(w1, M, C), k.s[1], k.c[1]),
+                pk_fma(magic(w0 >> 8, M, C), k.s[0], k.c[0]), pk_fma(magic(w1 >> 8, M, C), k.s[1], k.c[1]));
+    constexpr uint32_t H = 0x03000300u, D = 0x44004400u;  // 4 + h
+    a[1] = join(pk_fma(magic(t << 8, H, D), k.s[0], k.c6[0]), pk_fma(magic(t << 6, H, D), k.s[1], k.c6[1]),
+                pk_fma(magic(t, H, D), k.s[0], k.c6[0]), pk_fma(magic(t >> 2, H, D), k.s[1], k.c6[1]));
+  } else {
+    constexpr uint32_t L = 0x000F000Fu, G = 0x00F000F0u, C = 0x64006400u;  // 1024 + n, 1024 + 16 n
+    const uint32_t q8 = q0 >> 8;
+    uint32_t h0 = C, h1 = C, h2 = C, h3 = C;
+    asm("" : "+v"(h0));
+    if constexpr (T == kQ5_K) {  // bits 2 kg, 2 kg + 1 of each byte of h: bit 4 of n
+      const uint32_t t = h >> (2 * kg), b = h0;
+      h0 = ((t << 4) & 0x00100010u) | b;
+      h1 = ((t << 7) & 0x01000100u) | b;
+      h2 = ((t >> 4) & 0x00100010u) | b;
+      h3 = ((t >> 1) & 0x01000100u) | b;
+    } else {
+      h1 = h2 = h3 = h0;
+    }
+    a[0] = join(pk_fma(__builtin_bit_cast(half2_t, (q0 & L) | h0), k.s[0], k.c[0]),
+                pk_fma(__builtin_bit_cast(half2_t, (q0 & G) | h1), k.s[1], k.c[1]),
+                pk_fma(__builtin_bit_cast(half2_t, (q8 & L) | h2), k.s[0], k.c[0]),
+                pk_fma(__builtin_bit_cast(half2_t, (q8 & G) | h3), k.s[1], k.c[1]));
+  }
 }
 
+// The words KScales takes, of sub-blocks 2 kg and 2 kg + 1, from a row's 16 scale bytes: Q6_K the pairs of 16-element
+// scales as fp16; Q4_K / Q5_K (s / 16, -64 s) for the even sub-block, whose nibbles k_operand reads as 1024 + n, and
+// (s / 256, -4 s) for the odd one (1024 + 16 n).
+template <int T>
+__device__ __forceinline__ void k_scale_words(const u32x4_t& sc, int kg, uint32_t (&w)[2]) {
+  if constexpr (T == kQ6_K) {
+    const uint32_t lo = kg & 1 ? sc[1] : sc[0], hi = kg & 1 ? sc[3] : sc[2], b = kg & 2 ? hi : lo;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      w[i] = __builtin_bit_cast(uint32_t, half2_t{_Float16(int(int8_t((b >> (16 * i)) & 0xFFu))),
+                                                  _Float16(int(int8_t((b >> (16 * i + 8)) & 0xFFu)))});
+  } else {  // ggml get_scale_min_k4 (quant.cpp:52-61), four sub-blocks to a word
+    const uint32_t hi = kg >= 2 ? ~0u : 0u;
+    const uint32_t d4 = (((sc[2] & 0x0F0F0F0Fu) | ((sc[0] >> 2) & 0x30303030u)) & hi) | (sc[0] & 0x3F3F3F3Fu & ~hi);
+    const int sh = 16 * (kg & 1);
+    const float s0 = float((d4 >> sh) & 0xFFu), s1 = float((d4 >> (sh + 8)) & 0xFFu);
+    w[0] = __builtin_bit_cast(uint32_t, half2_t{_Float16(s0 * 0.0625f), _Float16(s0 * -64.f)});
+    w[1] = __builtin_bit_cast(uint32_t, half2_t{_Float16(s1 * 0.00390625f), _Float16(s1 * -4.f)});
+  }
+}
+
+// The A operand of a minimum term (Q4_K / Q5_K) for k group kg, in the order of the sum digits (kActQ8_K16): minimums
+// 4 (kg % 2) + 0, 2, 1, 3 against the low digits (kg < 2), 64 times them against the high ones.
+__device__ __forceinline__ half4_t k_min_operand(const u32x4_t& sc, int kg) {
+  const uint32_t hi = kg & 1 ? ~0u : 0u;
+  const uint32_t m4 =
+      ((((sc[2] >> 4) & 0x0F0F0F0Fu) | ((sc[1] >> 2) & 0x30303030u)) & hi) | (sc[1] & 0x3F3F3F3Fu & ~hi);
+  const _Float16 f = kg < 2 ? _Float16(1) : _Float16(64), c = _Float16(1024);
+  const half2_t f2 = {f, f}, c2 = {c, c};
+  const half2_t a = (magic(m4, 0x00FF00FFu, 0x64006400u) - c2) * f2, b = (magic(m4 >> 8, 0x00FF00FFu, 0x64006400u) - c2) * f2;
+  return half4_t{a[0], a[1], b[0], b[1]};
+}
+
+__device__ __forceinline__ void buffer_load_lds16(__amdgpu_buffer_rsrc_t rsrc, void* lds_wave_base, uint32_t voff,
+                                                  uint32_t soff) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, lds_wave_base, 16, voff, soff, 0, 0);
+#endif
+}
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc_of(const void* p, int64_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, int(bytes), 0x00020000);
+}
+// s_waitcnt with at most n vector loads outstanding and every LDS operation done
+constexpr int vm_lds_wait(int n) { return (n & 15) | (7 << 4) | (0 << 8) | ((n >> 4) << 14); }
+
+// qgemm_k_kernel: 64 weight rows x 32 activation rows per workgroup, 16 x 32 per wave. Operands travel global -> LDS
+// by direct-to-LDS buffer loads (rows past the ends read as zeros and are never stored; 16-byte chunks XOR-swizzled by
+// row, so fragment reads are conflict-free): the activation rows in half super-blocks (four residues, 256 bytes a
+// row) through a 3-stage ring, the raw quants and high bits a super-block ahead. The small planes of the next
+// super-block (scales, d and dmin; the activation rows' d and sum digits) are loaded into registers, each by one wave
+// and each value by one lane, during this super-block and stored to LDS at its end: the L1's rate of lane requests, not
+// bytes, bounded the kernel when every lane loaded the values that it uses (Q4_K, 17408 weight rows x 512 activation
+// rows, K = 2048: 123 us, 118 without the sums; this form 95). What bounds it now is VALU issue (271 operations per
+// wave and super-block, 128 of them the sums) with three waves per SIMD between the loads' latencies. Tiles of 16 x 64
+// and 32 x 32 per wave share an operand build among more sums but take two waves per SIMD and spill: 109 us.
+// Against the int8-slice kernel it replaces: Q4_K QKV (3072 rows x 512, K = 2048) 49 -> 20 us, Q6_K 67 -> 25.
 template <int T>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void qgemm_k_kernel(QGemmBatch B, QA A,
                                                                                              int64_t n) {
   static_assert(T == kQ4_K || T == kQ5_K || T == kQ6_K, "K types");
   constexpr int NS = k_slices<T>();
-  constexpr int WR = kKTileRows, AR = kKTileActs;
-  constexpr int QS = 33;                                 // words per staged quant row (32 and one of padding)
-  constexpr int HW = T == kQ5_K ? 8 : T == kQ6_K ? 16 : 0;  // high-bit words per row
-  constexpr int HS = HW + 1;
-  constexpr int AS = 68;                                 // words per staged activation row (64 and 4 of padding)
-  __shared__ uint32_t wq[WR * QS];
-  __shared__ uint32_t wh[HW > 0 ? WR * HS : 1];
-  __shared__ int wsc[WR][8], wmn[WR][8];                 // Q4_K / Q5_K: 6-bit scale and minimum per sub-block
-  __shared__ uint32_t wsq[WR][4];                        // Q6_K: the 16 int8 scales
-  __shared__ float wdm[WR][2];
-  __shared__ __align__(16) uint32_t aq[AR * AS];
-  __shared__ float ad[AR];
-  __shared__ int abs_[AR][8];                            // sum of the 16-sums of each sub-block (Q4_K / Q5_K)
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  constexpr int WN = 2, AR = 16 * WN;               // activation row groups per wave, activation rows per workgroup
+  constexpr int HB = T == kQ6_K ? 64 : T == kQ5_K ? 32 : 0;  // high-bit bytes per row and super-block
+  constexpr int kALoads = AR / 16;                  // direct-to-LDS loads per wave of an activation stage,
+  constexpr int kQLoads = 2 + (HB > 0 ? 1 : 0);     // and of a super-block's quants and high bits
+  // one object per stage: an LDS read then never waits for the loads into another stage
+  __shared__ __align__(16) uint8_t ring0[AR * 256], ring1[AR * 256], ring2[AR * 256];
+  __shared__ __align__(16) uint8_t quants0[64 * (128 + HB)], quants1[64 * (128 + HB)];  // by super-block parity
+  __shared__ __align__(16) u32x4_t scales[2][64];
+  __shared__ __align__(16) float wd[2][64], wm[2][64], ad[2][AR];
+  __shared__ __align__(16) half4_t digits[2][AR][4];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int ml = lane & 15, kg = lane >> 4;
   int wi = 0;
   for (int i = 1; i < B.n_w; ++i)
     if (int(blockIdx.x) >= B.tile0[i]) wi = i;
   const QW W = B.w[wi];
   float* __restrict__ y = B.y[wi];
-  const int64_t row0 = int64_t(int(blockIdx.x) - B.tile0[wi]) * WR, t0 = int64_t(blockIdx.y) * AR;
-  // A thread's share of one super-block: 2 quant u32x4 (64 rows x 128 bytes), its high-bit part, the scales and
-  // d / dmin of one row (threads < 64), 2 activation u32x4 (32 rows x 256 bytes) and one row's d and 16-sums
-  // (threads < 32). Rows and activation rows past the ends load clamped (staged, never stored).
+  const int64_t row0 = int64_t(int(blockIdx.x) - B.tile0[wi]) * 64, t0 = int64_t(blockIdx.y) * AR;
+  const int wrows = int(W.rows - row0 < 64 ? W.rows - row0 : 64), arows = int(n - t0 < AR ? n - t0 : AR);
+  const int nb = int(W.nb);
+  const __amdgpu_buffer_rsrc_t ra = rsrc_of(A.qs + t0 * nb * 512, int64_t(arows) * nb * 512);
+  const __amdgpu_buffer_rsrc_t rq = rsrc_of(W.q + row0 * nb * 128, int64_t(wrows) * nb * 128);
+  const __amdgpu_buffer_rsrc_t rh = rsrc_of(HB ? W.h + row0 * nb * HB : W.q, int64_t(wrows) * nb * HB);
+  // Load u of the activation rows fills rows 4 (4 u + wave) .. + 3: lane -> (row, position), and the lane loads the
+  // chunk that position holds (position p of row r: chunk p ^ (r % 16)).
+  uint32_t aoff[kALoads];
+#pragma unroll
+  for (int u = 0; u < kALoads; ++u) {
+    const int r = 4 * (4 * u + wave) + (lane >> 4);
+    aoff[u] = uint32_t(r) * uint32_t(nb) * 512 + 16 * ((lane & 15) ^ (r & 15));
+  }
+  // quants: position p of row r holds chunk p ^ (r / 2 % 8)
+  uint32_t qoff[2];
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int r = 8 * (4 * u + wave) + (lane >> 3);
+    qoff[u] = uint32_t(r) * uint32_t(nb) * 128 + 16 * ((lane & 7) ^ ((r >> 1) & 7));
+  }
+  // high bits: Q6_K four chunks per row (position p: chunk p ^ (r / 4 % 4)), Q5_K two (p ^ (r / 8 % 2))
+  const int hr = HB == 64 ? 16 * wave + (lane >> 2) : 16 * wave + (lane >> 1);
+  const uint32_t hoff = uint32_t(hr) * uint32_t(nb) * HB +
+                        16 * (HB == 64 ? (lane & 3) ^ ((hr >> 2) & 3) : (lane & 1) ^ ((hr >> 3) & 1));
+  auto ring = [&](auto st_c) __attribute__((always_inline)) {
+    constexpr int st = decltype(st_c)::value % 3;
+    return st == 0 ? ring0 : st == 1 ? ring1 : ring2;
+  };
+  auto quants = [&](auto p_c) __attribute__((always_inline)) { return decltype(p_c)::value % 2 == 0 ? quants0 : quants1; };
+  auto fetch = [&](int t, auto st_c) __attribute__((always_inline)) {  // stage t: half t % 2 of super-block t / 2
+#pragma unroll
+    for (int u = 0; u < kALoads; ++u)
+      buffer_load_lds16(ra, ring(st_c) + (4 * u + wave) * 1024, aoff[u], uint32_t(t) * 256);
+  };
+  auto fetch_quants = [&](int sb, auto p_c) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+      buffer_load_lds16(rq, quants(p_c) + (4 * u + wave) * 1024, qoff[u], uint32_t(sb) * 128);
+    if constexpr (HB > 0) {
+      if (lane < HB) buffer_load_lds16(rh, quants(p_c) + 64 * 128 + wave * (16 * HB), hoff, uint32_t(sb) * HB);
+    }
+  };
+  // This lane's share of a super-block's small planes: wave 0 the scales of weight row `lane`, wave 1 its d and dmin,
+  // wave 2 16 bytes of the activation rows' sum digits, wave 3 d of activation row `lane`. Rows past the ends read as
+  // zeros.
+  const __amdgpu_buffer_rsrc_t rs = rsrc_of(W.s + row0 * nb * 16, int64_t(wrows) * nb * 16),
+                               rd = rsrc_of(W.d + row0 * nb, int64_t(wrows) * nb * 2),
+                               rm = rsrc_of(T == kQ6_K ? W.d : W.m + row0 * nb, int64_t(wrows) * nb * 2),
+                               rad = rsrc_of(A.d + t0 * nb, int64_t(arows) * nb * 4),
+                               rbs = rsrc_of(A.bsums + t0 * nb * 16, int64_t(arows) * nb * 32);
+  const uint32_t srow = uint32_t(lane) * uint32_t(nb), brow = uint32_t(lane >> 1) * uint32_t(nb) * 32 + 16 * (lane & 1);
   struct Share {
-    u32x4_t q[2], h, sc, a[2], bs[2];
-    uint32_t d, m;
-    float da;
+    u32x4_t v;      // waves 0 and 2
+    uint16_t d, m;  // wave 1
+    uint32_t a;     // wave 3
   };
-  auto load_share = [&](int64_t sb, Share& sh) __attribute__((always_inline)) {
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const int e = tid + 256 * u, r = e >> 3, part = e & 7;
-      const int64_t rr = min(row0 + r, W.rows - 1);
-      sh.q[u] = reinterpret_cast<const u32x4_t*>(W.q + (rr * W.nb + sb) * 128)[part];
+  auto load_share = [&](int sb, Share& sh) __attribute__((always_inline)) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    if (wave == 0) {
+      sh.v = __builtin_amdgcn_raw_buffer_load_b128(rs, srow * 16, sb * 16, 0);
+    } else if (wave == 1) {
+      sh.d = __builtin_amdgcn_raw_buffer_load_b16(rd, srow * 2, sb * 2, 0);
+      if constexpr (T != kQ6_K) sh.m = __builtin_amdgcn_raw_buffer_load_b16(rm, srow * 2, sb * 2, 0);
+    } else if (wave == 2) {
+      if constexpr (T != kQ6_K) sh.v = __builtin_amdgcn_raw_buffer_load_b128(rbs, brow, sb * 32, 0);
+    } else {
+      sh.a = __builtin_amdgcn_raw_buffer_load_b32(rad, srow * 4, sb * 4, 0);
     }
-    if constexpr (T == kQ5_K) {
-      if (tid < WR * 2) {
-        const int64_t rr = min(row0 + (tid >> 1), W.rows - 1);
-        sh.h = reinterpret_cast<const u32x4_t*>(W.h + (rr * W.nb + sb) * 32)[tid & 1];
-      }
-    }
-    if constexpr (T == kQ6_K) {
-      const int64_t rr = min(row0 + (tid >> 2), W.rows - 1);
-      sh.h = reinterpret_cast<const u32x4_t*>(W.h + (rr * W.nb + sb) * 64)[tid & 3];
-    }
-    if (tid < WR) {
-      const int64_t wb = min(row0 + tid, W.rows - 1) * W.nb + sb;
-      sh.sc = *reinterpret_cast<const u32x4_t*>(W.s + wb * 16);
-      sh.d = W.d[wb];
-      sh.m = T == kQ6_K ? 0u : uint32_t(W.m[wb]);
-    }
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const int e = tid + 256 * u, r = e >> 4, part = e & 15;
-      const int64_t ab = min(t0 + r, n - 1) * A.nb + sb;
-      sh.a[u] = reinterpret_cast<const u32x4_t*>(A.qs + ab * 256)[part];
-    }
-    if (tid < AR) {
-      const int64_t ab = min(t0 + tid, n - 1) * A.nb + sb;
-      sh.da = A.d[ab];
-      if constexpr (T != kQ6_K) {
-        const u32x4_t* bp = reinterpret_cast<const u32x4_t*>(A.bsums + ab * 16);
-        sh.bs[0] = bp[0];
-        sh.bs[1] = bp[1];
-      }
+#endif
+  };
+  constexpr int kShareLoads = T == kQ6_K ? 0 : 1;  // at least, of any wave
+  auto store_share = [&](int p, Share& sh) __attribute__((always_inline)) {
+    // the loads are waited for here, on every path: one left pending on the paths around a branch would make the
+    // next reuse of its register wait for all loads in flight
+    asm volatile("" : "+v"(sh.v), "+v"(sh.d), "+v"(sh.m), "+v"(sh.a));
+    if (wave == 0) {
+      scales[p][lane] = sh.v;
+    } else if (wave == 1) {
+      wd[p][lane] = h2f(sh.d);
+      if constexpr (T != kQ6_K) wm[p][lane] = h2f(sh.m);
+    } else if (wave == 2) {
+      if constexpr (T != kQ6_K) reinterpret_cast<u32x4_t*>(&digits[p][0][0])[lane] = sh.v;
+    } else if (lane < AR) {
+      ad[p][lane] = __builtin_bit_cast(float, sh.a);
     }
   };
-  auto store_share = [&](const Share& sh) __attribute__((always_inline)) {
+  const int r0 = 16 * wave, ra_ = r0 + ml;  // this wave's weight rows, and the row of this lane's A operand
+  // sums[w][j][v]: weight row r0 + 4 kg + v, activation row 16 j + ml (the MFMA's result layout)
+  float sums[8][WN][4], acc[WN][4], dv[WN][4];
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const int e = tid + 256 * u, r = e >> 3, part = e & 7;
-#pragma unroll
-      for (int c = 0; c < 4; ++c) wq[r * QS + 4 * part + c] = sh.q[u][c];
-    }
-    if constexpr (T == kQ5_K) {
-      if (tid < WR * 2) {
-#pragma unroll
-        for (int c = 0; c < 4; ++c) wh[(tid >> 1) * HS + 4 * (tid & 1) + c] = sh.h[c];
-      }
-    }
-    if constexpr (T == kQ6_K) {
-#pragma unroll
-      for (int c = 0; c < 4; ++c) wh[(tid >> 2) * HS + 4 * (tid & 3) + c] = sh.h[c];
-    }
-    if (tid < WR) {
-      const uint32_t scw[4] = {sh.sc[0], sh.sc[1], sh.sc[2], sh.sc[3]};
-      auto sbyte = [&](int i) { return int((scw[i >> 2] >> (8 * (i & 3))) & 0xFFu); };
-      if constexpr (T == kQ6_K) {
-#pragma unroll
-        for (int c = 0; c < 4; ++c) wsq[tid][c] = scw[c];
-      } else {
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {  // ggml get_scale_min_k4 (quant.cpp:52-61), compile-time byte indices
-          int sk, mk;
-          if (k < 4) {
-            sk = sbyte(k) & 63;
-            mk = sbyte(k + 4) & 63;
-          } else {
-            sk = (sbyte(k + 4) & 0xF) | ((sbyte(k - 4) >> 6) << 4);
-            mk = (sbyte(k + 4) >> 4) | ((sbyte(k) >> 6) << 4);
-          }
-          wsc[tid][k] = sk;
-          wmn[tid][k] = mk;
-        }
-      }
-      wdm[tid][0] = h2f(uint16_t(sh.d));
-      wdm[tid][1] = h2f(uint16_t(sh.m));
-    }
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const int e = tid + 256 * u, r = e >> 4, part = e & 15;
-      *reinterpret_cast<u32x4_t*>(&aq[r * AS + 4 * part]) = sh.a[u];
-    }
-    if (tid < AR) {
-      ad[tid] = sh.da;
-      if constexpr (T != kQ6_K) {
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {  // 16-sums 2k and 2k + 1: the two int16 halves of word k
-          const uint32_t wk = sh.bs[k >> 2][k & 3];
-          abs_[tid][k] = int(int16_t(wk & 0xFFFFu)) + int(int16_t(wk >> 16));
-        }
-      }
-    }
-  };
-  // acc[j][v], sums[w][j][v]: weight row 16 wave + 4 kg + v, activation row 16 j + ml
-  float sums[8][2][4], acc[2][4];
-#pragma unroll
-  for (int j = 0; j < 2; ++j)
+  for (int j = 0; j < WN; ++j)
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
       acc[j][v] = 0.f;
 #pragma unroll
       for (int w = 0; w < 8; ++w) sums[w][j][v] = 0.f;
     }
-  const int ra = 16 * wave + ml;  // this lane's operand row
-  Share cur;
+  uint32_t boff[4];  // this lane's activation fragment of residue 4 half + wl, within the first 16 rows
+#pragma unroll
+  for (int wl = 0; wl < 4; ++wl) boff[wl] = uint32_t(ml * 256 + 16 * ((4 * wl + kg) ^ ml));
+  const int nt = 2 * nb;
+  Share cur{};
   load_share(0, cur);
-  for (int64_t sb = 0; sb < W.nb; ++sb) {
-    store_share(cur);
-    __syncthreads();
-    load_share(sb + 1 < W.nb ? sb + 1 : sb, cur);  // in flight while this super-block is computed
-    float dv[2][4];
+  store_share(0, cur);
+  fetch_quants(0, std::integral_constant<int, 0>{});
+  fetch(0, std::integral_constant<int, 0>{});
+  fetch(1, std::integral_constant<int, 1>{});
+  uint32_t sw[2];  // k_scale_words of this lane's row
+  auto step = [&](int t, auto m_c) __attribute__((always_inline)) {  // m: t % 12
+    constexpr int m = decltype(m_c)::value, half = m & 1, p = (m >> 1) & 1;
+    const int sb = t >> 1;
+    // Every wave's loads of stage t and its LDS stores; the barrier publishes both and certifies that every wave is
+    // done with stage t - 1. In flight stay, at half 0, stage t + 1's loads; at half 1 the small planes', the quants'
+    // and stage t + 1's, which half 0 issued after stage t's.
+    __builtin_amdgcn_s_waitcnt(vm_lds_wait(half == 0 ? kALoads : kShareLoads + kQLoads + kALoads));
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if constexpr (half == 0) {  // past the end: the last super-block and stage again
+      load_share(sb + 1 < nb ? sb + 1 : sb, cur);
+      fetch_quants(sb + 1 < nb ? sb + 1 : sb, std::integral_constant<int, p ^ 1>{});
+    }
+    fetch(t + 2 < nt ? t + 2 : nt - 1, std::integral_constant<int, m + 2>{});
+    const uint8_t* const base = ring(m_c);
+    const uint8_t* const qbase = quants(std::integral_constant<int, p>{});
+    if constexpr (half == 0) {
+      float da[WN];
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+      for (int j = 0; j < WN; ++j) da[j] = ad[p][16 * j + ml];
+      const u32x4_t sc = scales[p][ra_];
+      k_scale_words<T>(sc, kg, sw);
+      const floatx4_t dw = *reinterpret_cast<const floatx4_t*>(&wd[p][r0 + 4 * kg]);
 #pragma unroll
-      for (int v = 0; v < 4; ++v) dv[j][v] = __fmul_rn(wdm[16 * wave + 4 * kg + v][0], ad[16 * j + ml]);
-    // the lane's two sub-blocks' scales: 2 kg and 2 kg + 1 (Q4_K / Q5_K), or their int8 pairs (Q6_K)
-    int s_a = 0, s_b = 0;
-    uint32_t s6 = 0;
-    if constexpr (T == kQ6_K)
-      s6 = wsq[ra][kg];  // bytes 4 kg .. 4 kg + 3: scales 2k, 2k + 1 of sub-blocks k = 2 kg, 2 kg + 1
-    else
-      s_a = wsc[ra][2 * kg], s_b = wsc[ra][2 * kg + 1];
+      for (int j = 0; j < WN; ++j)
 #pragma unroll
-    for (int w = 0; w < 8; ++w) {
-      long aop[NS];
-      if constexpr (T == kQ6_K) {
-        // sub-block k = 2 kg + b: half h = kg >> 1, g = 2 (kg & 1) + b; ql group lg = b at word 16 h + 8 lg + w,
-        // nibble 4 (kg & 1); qh word 8 h + w at bits 2 g
-        const int h = kg >> 1, sel = kg & 1;
-        const uint32_t hq = wh[ra * HS + 8 * h + w];
-        uint32_t sl[4][2];
+        for (int v = 0; v < 4; ++v) dv[j][v] = __fmul_rn(dw[v], da[j]);
+      if constexpr (T != kQ6_K) {
+        const half4_t am = k_min_operand(sc, kg);
+        const floatx4_t dm = *reinterpret_cast<const floatx4_t*>(&wm[p][r0 + 4 * kg]);
 #pragma unroll
-        for (int b = 0; b < 2; ++b) {
-          const int g = 2 * sel + b;
-          const uint32_t lw = wq[ra * QS + 16 * h + 8 * b + w];
-          const uint32_t v = ((lw >> (4 * sel)) & 0x0F0F0F0Fu) | (((hq >> (2 * g)) & 0x03030303u) << 4);
-          const u16x2_t u0e = __builtin_bit_cast(u16x2_t, v & 0x00070007u);
-          const u16x2_t u0o = __builtin_bit_cast(u16x2_t, (v >> 8) & 0x00070007u);
-          const u16x2_t four = {4, 4};
-          const u16x2_t u1e = __builtin_bit_cast(u16x2_t, (v >> 3) & 0x00070007u) - four;
-          const u16x2_t u1o = __builtin_bit_cast(u16x2_t, (v >> 11) & 0x00070007u) - four;
-          const int slo = int(int8_t((s6 >> (16 * b)) & 0xFFu)), shi = int(int8_t((s6 >> (16 * b + 8)) & 0xFFu));
-          const u16x2_t s0 = {uint16_t(slo & 15), uint16_t(shi & 15)};
-          const u16x2_t s1 = {uint16_t(slo >> 4), uint16_t(shi >> 4)};
-          sl[0][b] = byte_products(u1e, u1o, s1);
-          sl[1][b] = byte_products(u0e, u0o, s1);
-          sl[2][b] = byte_products(u1e, u1o, s0);
-          sl[3][b] = byte_products(u0e, u0o, s0);
-        }
+        for (int j = 0; j < WN; ++j) {
+          const floatx4_t sumi =
+              __builtin_amdgcn_mfma_f32_16x16x16f16(am, digits[p][16 * j + ml][kg], floatx4_t{0, 0, 0, 0}, 0, 0, 0);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) aop[i] = long((uint64_t(sl[i][1]) << 32) | uint64_t(sl[i][0]));
-      } else {
-        const uint32_t qw = wq[ra * QS + 8 * kg + w];
-        uint32_t qa = qw & 0x0F0F0F0Fu, qb = (qw >> 4) & 0x0F0F0F0Fu;  // sub-blocks 2 kg and 2 kg + 1
-        if constexpr (T == kQ5_K) {
-          const uint32_t hb = wh[ra * HS + w];
-          qa |= ((hb >> (2 * kg)) & 0x01010101u) << 4;
-          qb |= ((hb >> (2 * kg + 1)) & 0x01010101u) << 4;
-        }
-        if constexpr (T == kQ4_K) {
-          aop[0] = long((uint64_t(qb * uint32_t(s_b & 7)) << 32) | uint64_t(qa * uint32_t(s_a & 7)));
-          aop[1] = long((uint64_t(qb * uint32_t(s_b >> 3)) << 32) | uint64_t(qa * uint32_t(s_a >> 3)));
-        } else {
-          aop[0] = long((uint64_t(qb * uint32_t(s_b & 3)) << 32) | uint64_t(qa * uint32_t(s_a & 3)));
-          aop[1] = long((uint64_t(qb * uint32_t((s_b >> 2) & 3)) << 32) | uint64_t(qa * uint32_t((s_a >> 2) & 3)));
-          aop[2] = long((uint64_t(qb * uint32_t(s_b >> 4)) << 32) | uint64_t(qa * uint32_t(s_a >> 4)));
-        }
-      }
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const uint2 bw = *reinterpret_cast<const uint2*>(&aq[(16 * j + ml) * AS + 8 * w + 2 * kg]);
-        const long bop = long((uint64_t(bw.y) << 32) | uint64_t(bw.x));
-        i32x4_t c[NS];
-#pragma unroll
-        for (int sl = 0; sl < NS; ++sl)
-          c[sl] = __builtin_amdgcn_mfma_i32_16x16x32_i8(aop[sl], bop, i32x4_t{0, 0, 0, 0}, 0, 0, 0);
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          int aux;
-          if constexpr (T == kQ6_K)
-            aux = 128 * c[0][v] + 16 * c[1][v] + 8 * c[2][v] + c[3][v];
-          else if constexpr (T == kQ5_K)
-            aux = c[0][v] + 4 * c[1][v] + 16 * c[2][v];
-          else
-            aux = c[0][v] + 8 * c[1][v];
-          sums[w][j][v] = __fadd_rn(sums[w][j][v], __fmul_rn(dv[j][v], float(aux)));
+          for (int v = 0; v < 4; ++v)
+            acc[j][v] = opaque(__fsub_rn(acc[j][v], __fmul_rn(__fmul_rn(dm[v], da[j]), sumi[v])));
         }
       }
     }
-    if constexpr (T != kQ6_K) {
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const int t = 16 * j + ml;
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int rv = 16 * wave + 4 * kg + v;
-          int sumi = 0;
-#pragma unroll
-          for (int k = 0; k < 8; ++k) sumi += abs_[t][k] * wmn[rv][k];
-          acc[j][v] = __fsub_rn(acc[j][v], __fmul_rn(__fmul_rn(wdm[rv][1], ad[t]), float(sumi)));
-        }
-      }
+    // the lane's raw words of the four residues, and its sub-blocks' constants
+    u32x4_t q0, q1, h;
+    KScales<T> ks;
+    ks.set(sw[0], sw[1]);
+    auto chunk = [&](int c) {
+      return *reinterpret_cast<const u32x4_t*>(qbase + ra_ * 128 + 16 * ((2 * c + half) ^ ((ra_ >> 1) & 7)));
+    };
+    const uint8_t* const hbase = qbase + 64 * 128 + ra_ * HB;
+    if constexpr (T == kQ6_K) {
+      q0 = chunk(2 * (kg >> 1));
+      q1 = chunk(2 * (kg >> 1) + 1);
+      h = *reinterpret_cast<const u32x4_t*>(hbase + 16 * ((2 * (kg >> 1) + half) ^ ((ra_ >> 2) & 3)));
+    } else {
+      q0 = chunk(kg);
+      if constexpr (T == kQ5_K) h = *reinterpret_cast<const u32x4_t*>(hbase + 16 * (half ^ ((ra_ >> 3) & 1)));
     }
-    __syncthreads();
+    // Residue wl's sums are added while the MFMAs of wl + 1 run and the fragments of wl + 2 are read.
+    half8_t b[2][WN];
+    floatx4_t c[2][WN];
+    auto load_b = [&](int wl) __attribute__((always_inline)) {
+#pragma unroll
+      for (int j = 0; j < WN; ++j) b[wl & 1][j] = *reinterpret_cast<const half8_t*>(base + boff[wl] + j * 4096);
+    };
+    auto multiply = [&](int wl) __attribute__((always_inline)) {
+      half8_t a[NS];
+      k_operand<T>(q0[wl], T == kQ6_K ? q1[wl] : 0u, HB ? h[wl] : 0u, kg, ks, a);
+#pragma unroll
+      for (int j = 0; j < WN; ++j) {
+        c[wl & 1][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[0], b[wl & 1][j], floatx4_t{0, 0, 0, 0}, 0, 0, 0);
+        if constexpr (NS == 2)
+          c[wl & 1][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[NS - 1], b[wl & 1][j], c[wl & 1][j], 0, 0, 0);
+      }
+    };
+    load_b(0);
+    load_b(1);
+    multiply(0);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int wl = 0; wl < 4; ++wl) {
+      if (wl < 3) multiply(wl + 1);
+      if (wl < 2) load_b(wl + 2);
+      constexpr int w0 = 4 * half;
+#pragma unroll
+      for (int j = 0; j < WN; ++j)
+#pragma unroll
+        for (int v = 0; v < 4; ++v)  // (opaque: added here, not later)
+          sums[w0 + wl][j][v] = opaque(__fadd_rn(sums[w0 + wl][j][v], __fmul_rn(dv[j][v], c[wl & 1][j][v])));
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    // the next super-block's small planes (this parity's last readers passed the barrier before this super-block)
+    if constexpr (half == 1) store_share(p ^ 1, cur);
+  };
+  auto pair = [&](int t, auto m_c) __attribute__((always_inline)) {  // a super-block; false: it was the last
+    constexpr int m = decltype(m_c)::value;
+    step(t, std::integral_constant<int, m>{});
+    step(t + 1, std::integral_constant<int, m + 1>{});
+    return t + 2 < nt;
+  };
+  for (int t = 0;; t += 12) {  // six super-blocks: every stage and parity a compile-time constant
+    if (!pair(t, std::integral_constant<int, 0>{}) || !pair(t + 2, std::integral_constant<int, 2>{}) ||
+        !pair(t + 4, std::integral_constant<int, 4>{}) || !pair(t + 6, std::integral_constant<int, 6>{}) ||
+        !pair(t + 8, std::integral_constant<int, 8>{}) || !pair(t + 10, std::integral_constant<int, 10>{}))
+      break;
   }
+  __builtin_amdgcn_s_waitcnt(vm_lds_wait(0));  // no load may land in LDS after the workgroup's end
+  const bool vec = W.rows % 4 == 0 && reinterpret_cast<uintptr_t>(y) % 16 == 0;
+  const int64_t r = row0 + r0 + 4 * kg;
 #pragma unroll
-  for (int j = 0; j < 2; ++j)
+  for (int j = 0; j < WN; ++j) {
+    const int64_t t = t0 + 16 * j + ml;
+    floatx4_t o;
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
-      float o = acc[j][v];
+      o[v] = acc[j][v];
 #pragma unroll
-      for (int w = 0; w < 8; ++w) o = __fadd_rn(o, sums[w][j][v]);
-      const int64_t r = row0 + 16 * wave + 4 * kg + v, t = t0 + 16 * j + ml;
-      if (r < W.rows && t < n) y[t * W.rows + r] = o;
+      for (int w = 0; w < 8; ++w) o[v] = __fadd_rn(o[v], sums[w][j][v]);
     }
+    if (t < n) {
+      if (vec && r < W.rows) {
+        *reinterpret_cast<floatx4_t*>(y + t * W.rows + r) = o;
+      } else {
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+          if (r + v < W.rows) y[t * W.rows + r + v] = o[v];
+      }
+    }
+  }
 }
 
 // qgemm_k_small_kernel: the K types for calls of few activation rows, where 64-row weight tiles leave most CUs
 // idle and each workgroup would walk every super-block alone. A workgroup takes 16 weight rows x 32 activation
 // rows and its 4 waves split the super-blocks (wave w: w, w + 4, ...): each computes its super-block's float terms
-// - d * aux[l] for the eight lanes and, for Q4_K / Q5_K, the minimum term, with the operands, slices and
-// expressions of qgemm_k_kernel, its operands read straight from global memory - and writes them to LDS; per round
+// - d * aux[l] for the eight lanes and, for Q4_K / Q5_K, the minimum term, with the operands and expressions of
+// qgemm_k_kernel, its operands read straight from global memory - and writes them to LDS; per round
 // of four super-blocks the 256 threads, two outputs each, add them to their running sums in super-block order:
 // the reference's order, so the same bits.
 template <int T>
@@ -1154,11 +1295,7 @@ __global__ __launch_bounds__(256) void qgemm_k_small_kernel(QGemmBatch B, QA A, 
   constexpr int NS = k_slices<T>();
   constexpr int NTM = T == kQ6_K ? 8 : 9;  // float terms per output and super-block
   __shared__ float terms[4][NTM][16][33];  // [wave][term][weight row][activation row], one column of padding
-  __shared__ float rowd[4][16][2];         // per wave: d, dmin of its super-block's 16 rows
-  __shared__ int rowm[4][16][8], rows6[4][16][8];  // minimums and 6-bit scales (Q4_K / Q5_K)
-  __shared__ uint32_t rowq6[4][16][4];     // Q6_K: the 16 int8 scales
-  __shared__ float actd[4][32];
-  __shared__ int actb[4][32][8];           // sums of the 16-sums per sub-block (Q4_K / Q5_K)
+  __shared__ __align__(16) float rowd[4][16], rowm[4][16];  // per wave: d, dmin of its super-block's 16 rows
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int ml = lane & 15, kg = lane >> 4;
   int wi = 0;
@@ -1180,49 +1317,10 @@ __global__ __launch_bounds__(256) void qgemm_k_small_kernel(QGemmBatch B, QA A, 
     const int64_t sb = s0 + wave;
     const bool has = sb < W.nb;
     const int64_t sbc = has ? sb : W.nb - 1;
-    // this wave's super-block: per-row and per-activation-row values into its LDS slices
-    if (lane < 16) {
-      const int64_t wb = min(row0 + lane, W.rows - 1) * W.nb + sbc;
-      const u32x4_t sc = *reinterpret_cast<const u32x4_t*>(W.s + wb * 16);
-      const uint32_t scw[4] = {sc[0], sc[1], sc[2], sc[3]};
-      auto sbyte = [&](int i) { return int((scw[i >> 2] >> (8 * (i & 3))) & 0xFFu); };
-      rowd[wave][lane][0] = h2f(W.d[wb]);
-      if constexpr (T == kQ6_K) {
-        rowd[wave][lane][1] = 0.f;
-#pragma unroll
-        for (int c = 0; c < 4; ++c) rowq6[wave][lane][c] = scw[c];
-      } else {
-        rowd[wave][lane][1] = h2f(W.m[wb]);
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {  // ggml get_scale_min_k4 (quant.cpp:52-61), compile-time byte indices
-          int sk, mk;
-          if (k < 4) {
-            sk = sbyte(k) & 63;
-            mk = sbyte(k + 4) & 63;
-          } else {
-            sk = (sbyte(k + 4) & 0xF) | ((sbyte(k - 4) >> 6) << 4);
-            mk = (sbyte(k + 4) >> 4) | ((sbyte(k) >> 6) << 4);
-          }
-          rows6[wave][lane][k] = sk;
-          rowm[wave][lane][k] = mk;
-        }
-      }
-    } else if (lane < 48) {
-      const int a = lane - 16;
-      const int64_t ab = min(t0 + a, n - 1) * A.nb + sbc;
-      actd[wave][a] = A.d[ab];
-      if constexpr (T != kQ6_K) {
-        const u32x4_t* bp = reinterpret_cast<const u32x4_t*>(A.bsums + ab * 16);
-        const u32x4_t b0 = bp[0], b1 = bp[1];
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {  // 16-sums 2k and 2k + 1: the two int16 halves of word k
-          const uint32_t wk = k < 4 ? b0[k] : b1[k - 4];
-          actb[wave][a][k] = int(int16_t(wk & 0xFFFFu)) + int(int16_t(wk >> 16));
-        }
-      }
-    }
-    // the lane's operand words: its row's quant words of its k group (and their high bits), every residue
     const int64_t wb = ra * W.nb + sbc;
+    const u32x4_t sc = *reinterpret_cast<const u32x4_t*>(W.s + wb * 16);
+    uint32_t sw[2];
+    // the lane's operand words: its row's quant words of its k group (and their high bits), every residue
     u32x4_t qv[T == kQ6_K ? 4 : 2], hv[2];
     if constexpr (T == kQ6_K) {
       const u32x4_t* q = reinterpret_cast<const u32x4_t*>(W.q + wb * 128 + 64 * (kg >> 1));
@@ -1238,103 +1336,55 @@ __global__ __launch_bounds__(256) void qgemm_k_small_kernel(QGemmBatch B, QA A, 
         hv[0] = h[0], hv[1] = h[1];
       }
     }
-    uint2 bw[2][8];
+    half8_t bw[2][8];
+    float da[2];
+    half4_t bs[2];
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       const int64_t ab = min(t0 + 16 * j + ml, n - 1) * A.nb + sbc;
-      const uint8_t* aq = reinterpret_cast<const uint8_t*>(A.qs) + ab * 256;
+      const half8_t* aq = reinterpret_cast<const half8_t*>(A.qs + ab * 512);
 #pragma unroll
-      for (int w = 0; w < 8; ++w) bw[j][w] = *reinterpret_cast<const uint2*>(aq + 32 * w + 8 * kg);
+      for (int w = 0; w < 8; ++w) bw[j][w] = aq[4 * w + kg];
+      da[j] = A.d[ab];
+      if constexpr (T != kQ6_K) bs[j] = reinterpret_cast<const half4_t*>(A.bsums)[ab * 4 + kg];
     }
-    __syncthreads();  // this round's row and activation values are in LDS
+    const float d1 = h2f(W.d[wb]), m1 = T == kQ6_K ? 0.f : h2f(W.m[wb]);
+    k_scale_words<T>(sc, kg, sw);
+    if (kg == 0) rowd[wave][ml] = d1, rowm[wave][ml] = m1;
+    __syncthreads();  // this round's row values are in LDS
     if (has) {
+      const floatx4_t dw = *reinterpret_cast<const floatx4_t*>(&rowd[wave][4 * kg]);
       float dv[2][4];
 #pragma unroll
       for (int j = 0; j < 2; ++j)
 #pragma unroll
-        for (int v = 0; v < 4; ++v) dv[j][v] = __fmul_rn(rowd[wave][4 * kg + v][0], actd[wave][16 * j + ml]);
-      int s_a = 0, s_b = 0;
-      uint32_t s6 = 0;
-      if constexpr (T == kQ6_K)
-        s6 = rowq6[wave][ml][kg];
-      else
-        s_a = rows6[wave][ml][2 * kg], s_b = rows6[wave][ml][2 * kg + 1];
+        for (int v = 0; v < 4; ++v) dv[j][v] = __fmul_rn(dw[v], da[j]);
+      KScales<T> ks;
+      ks.set(sw[0], sw[1]);
 #pragma unroll
       for (int w = 0; w < 8; ++w) {
-        long aop[NS];
-        if constexpr (T == kQ6_K) {
-          const int sel = kg & 1;
-          const uint32_t hq = hv[w >> 2][w & 3];
-          uint32_t sl[4][2];
-#pragma unroll
-          for (int b = 0; b < 2; ++b) {
-            const int g = 2 * sel + b;
-            const uint32_t lw = qv[(8 * b + w) >> 2][(8 * b + w) & 3];
-            const uint32_t v = ((lw >> (4 * sel)) & 0x0F0F0F0Fu) | (((hq >> (2 * g)) & 0x03030303u) << 4);
-            const u16x2_t u0e = __builtin_bit_cast(u16x2_t, v & 0x00070007u);
-            const u16x2_t u0o = __builtin_bit_cast(u16x2_t, (v >> 8) & 0x00070007u);
-            const u16x2_t four = {4, 4};
-            const u16x2_t u1e = __builtin_bit_cast(u16x2_t, (v >> 3) & 0x00070007u) - four;
-            const u16x2_t u1o = __builtin_bit_cast(u16x2_t, (v >> 11) & 0x00070007u) - four;
-            const int slo = int(int8_t((s6 >> (16 * b)) & 0xFFu)), shi = int(int8_t((s6 >> (16 * b + 8)) & 0xFFu));
-            const u16x2_t s0 = {uint16_t(slo & 15), uint16_t(shi & 15)};
-            const u16x2_t s1 = {uint16_t(slo >> 4), uint16_t(shi >> 4)};
-            sl[0][b] = byte_products(u1e, u1o, s1);
-            sl[1][b] = byte_products(u0e, u0o, s1);
-            sl[2][b] = byte_products(u1e, u1o, s0);
-            sl[3][b] = byte_products(u0e, u0o, s0);
-          }
-#pragma unroll
-          for (int i = 0; i < 4; ++i) aop[i] = long((uint64_t(sl[i][1]) << 32) | uint64_t(sl[i][0]));
-        } else {
-          const uint32_t qw = qv[w >> 2][w & 3];
-          uint32_t qa = qw & 0x0F0F0F0Fu, qb = (qw >> 4) & 0x0F0F0F0Fu;  // sub-blocks 2 kg and 2 kg + 1
-          if constexpr (T == kQ5_K) {
-            const uint32_t hb = hv[w >> 2][w & 3];
-            qa |= ((hb >> (2 * kg)) & 0x01010101u) << 4;
-            qb |= ((hb >> (2 * kg + 1)) & 0x01010101u) << 4;
-          }
-          if constexpr (T == kQ4_K) {
-            aop[0] = long((uint64_t(qb * uint32_t(s_b & 7)) << 32) | uint64_t(qa * uint32_t(s_a & 7)));
-            aop[1] = long((uint64_t(qb * uint32_t(s_b >> 3)) << 32) | uint64_t(qa * uint32_t(s_a >> 3)));
-          } else {
-            aop[0] = long((uint64_t(qb * uint32_t(s_b & 3)) << 32) | uint64_t(qa * uint32_t(s_a & 3)));
-            aop[1] = long((uint64_t(qb * uint32_t((s_b >> 2) & 3)) << 32) | uint64_t(qa * uint32_t((s_a >> 2) & 3)));
-            aop[2] = long((uint64_t(qb * uint32_t(s_b >> 4)) << 32) | uint64_t(qa * uint32_t(s_a >> 4)));
-          }
-        }
+        half8_t a[NS];
+        if constexpr (T == kQ6_K)
+          k_operand<T>(qv[w >> 2][w & 3], qv[2 + (w >> 2)][w & 3], hv[w >> 2][w & 3], kg, ks, a);
+        else
+          k_operand<T>(qv[w >> 2][w & 3], 0u, T == kQ5_K ? hv[w >> 2][w & 3] : 0u, kg, ks, a);
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
-          const long bop = long((uint64_t(bw[j][w].y) << 32) | uint64_t(bw[j][w].x));
-          i32x4_t c[NS];
+          floatx4_t c = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[0], bw[j][w], floatx4_t{0, 0, 0, 0}, 0, 0, 0);
+          if constexpr (NS == 2) c = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[NS - 1], bw[j][w], c, 0, 0, 0);
 #pragma unroll
-          for (int sl = 0; sl < NS; ++sl)
-            c[sl] = __builtin_amdgcn_mfma_i32_16x16x32_i8(aop[sl], bop, i32x4_t{0, 0, 0, 0}, 0, 0, 0);
-#pragma unroll
-          for (int v = 0; v < 4; ++v) {
-            int aux;
-            if constexpr (T == kQ6_K)
-              aux = 128 * c[0][v] + 16 * c[1][v] + 8 * c[2][v] + c[3][v];
-            else if constexpr (T == kQ5_K)
-              aux = c[0][v] + 4 * c[1][v] + 16 * c[2][v];
-            else
-              aux = c[0][v] + 8 * c[1][v];
-            terms[wave][w][4 * kg + v][16 * j + ml] = __fmul_rn(dv[j][v], float(aux));
-          }
+          for (int v = 0; v < 4; ++v) terms[wave][w][4 * kg + v][16 * j + ml] = __fmul_rn(dv[j][v], c[v]);
         }
       }
       if constexpr (T != kQ6_K) {
+        const half4_t am = k_min_operand(sc, kg);
+        const floatx4_t dm = *reinterpret_cast<const floatx4_t*>(&rowm[wave][4 * kg]);
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
-          const int t = 16 * j + ml;
+          const floatx4_t sumi = __builtin_amdgcn_mfma_f32_16x16x16f16(am, bs[j], floatx4_t{0, 0, 0, 0}, 0, 0, 0);
 #pragma unroll
-          for (int v = 0; v < 4; ++v) {
-            const int rv = 4 * kg + v;
-            int sumi = 0;
-#pragma unroll
-            for (int k = 0; k < 8; ++k) sumi += actb[wave][t][k] * rowm[wave][rv][k];
-            terms[wave][8][rv][t] = __fmul_rn(__fmul_rn(rowd[wave][rv][1], actd[wave][t]), float(sumi));
-          }
+          for (int v = 0; v < 4; ++v)
+            terms[wave][NTM - 1][4 * kg + v][16 * j + ml] = __fmul_rn(__fmul_rn(dm[v], da[j]), sumi[v]);
         }
       }
     }
@@ -1348,7 +1398,7 @@ __global__ __launch_bounds__(256) void qgemm_k_small_kernel(QGemmBatch B, QA A, 
           const int ot = (tid >> 4) + 16 * o;
 #pragma unroll
           for (int l = 0; l < 8; ++l) sums[o][l] = __fadd_rn(sums[o][l], terms[s][l][orow][ot]);
-          if constexpr (T != kQ6_K) acc[o] = __fsub_rn(acc[o], terms[s][8][orow][ot]);
+          if constexpr (T != kQ6_K) acc[o] = __fsub_rn(acc[o], terms[s][NTM - 1][orow][ot]);
         }
       }
     }
@@ -1364,14 +1414,15 @@ __global__ __launch_bounds__(256) void qgemm_k_small_kernel(QGemmBatch B, QA A, 
   }
 }
 
-// The small-call K kernel runs while 64 x 32 tiles would give fewer than this many workgroups (measured at the QKV
-// shape, 48 such row tiles: Q4_K faster up to 64 rows, Q5_K / Q6_K up to 128-160; beyond, the 64 x 32 kernel).
+// The small-call K kernel runs while 64 x 32 tiles would give fewer than kKSmallMaxWgs workgroups (QKV shape, 48 such
+// row tiles, K = 2048: Q4_K at 32 rows 10.8 us against 12.9, at 64 rows 13.9 against 12.3; 32 row tiles, K = 8192:
+// Q6_K at 64 rows 39.7 against 43.9, at 128 rows 62 against 44.7).
+constexpr int64_t kKSmallMaxWgs = 80;
 template <int T>
-constexpr int64_t k_small_max_wgs() { return T == kQ4_K ? 128 : 256; }
-template <int T>
-hipError_t launch_k(bool small, dim3 grid32, hipStream_t s, const QGemmBatch& B, const QA& A, int64_t n) {
-  if (small) return nbhs_timing::launch(NBHS_K_QGEMM, qgemm_k_small_kernel<T>, grid32, dim3(256), s, B, A, n);
-  return nbhs_timing::launch(NBHS_K_QGEMM, qgemm_k_kernel<T>, grid32, dim3(256), s, B, A, n);
+hipError_t launch_k(bool small, unsigned tiles, hipStream_t s, const QGemmBatch& B, const QA& A, int64_t n) {
+  const dim3 grid{tiles, unsigned((n + 31) / 32)};
+  if (small) return nbhs_timing::launch(NBHS_K_QGEMM, qgemm_k_small_kernel<T>, grid, dim3(256), s, B, A, n);
+  return nbhs_timing::launch(NBHS_K_QGEMM, qgemm_k_kernel<T>, grid, dim3(256), s, B, A, n);
 }
 
 // ---- dequantization (quant.cpp:157-242), one thread per block of one output row ----
@@ -1487,6 +1538,11 @@ int64_t nbhs_quant_act_bytes(int type, int64_t n, int64_t in) {
   return act_layout(act_of(type), n, in / block_elems(type)).bytes;
 }
 
+int64_t nbhs_quant_act_rm_bytes(int type, int64_t n, int64_t in) {
+  if (!is_k(type) || n <= 0 || in <= 0 || in % 256) return -1;
+  return act_layout(kActQ8_K16, n, in / 256).bytes;
+}
+
 int nbhs_quantize_acts(int type, const float* x, int64_t n, int64_t in, void* acts, nbhs_stream stream) {
   if (!is_quant(type) || !x || !acts || n <= 0 || in <= 0 || in % block_elems(type)) return NBHS_EINVAL;
   const int act = act_of(type);
@@ -1513,7 +1569,7 @@ int nbhs_quantize_acts_rm(int type, const float* x, int64_t n, int64_t in, void*
   if (!is_k(type) || !x || !acts || n <= 0 || in <= 0 || in % 256) return NBHS_EINVAL;
   const int64_t nb = in / 256, blocks = n * nb;
   if (blocks >= (int64_t(1) << 31)) return NBHS_EINVAL;
-  const ActLayout l = act_layout(kActQ8_K, n, nb);
+  const ActLayout l = act_layout(kActQ8_K16, n, nb);
   uint8_t* base = static_cast<uint8_t*>(acts);
   return nbhs_timing::launch(NBHS_K_QUANTIZE, quantize_q8k_kernel<true>, dim3(unsigned(blocks)), dim3(64),
                              reinterpret_cast<hipStream_t>(stream), x, in, reinterpret_cast<int8_t*>(base + l.qs_off),
@@ -1589,27 +1645,25 @@ int nbhs_qgemm_multi(int type, int n_w, const void* const* w, const int64_t* row
       tile = kTile32x32;
   }
   // K types: the small-call kernel (16-row weight tiles, super-blocks split over the waves) when 64-row tiles
-  // would give fewer than kKSmallMaxWgs workgroups
-  const bool small = is_k(type) && tiles64 * ((n + 31) / 32) < (type == kQ4_K ? k_small_max_wgs<kQ4_K>()
-                                                                                 : k_small_max_wgs<kQ6_K>());
+  // would give fewer than kKSmallMaxWgs workgroups, or a row is too long for the tiled kernel's 32-bit offsets
+  const bool small = is_k(type) && (tiles64 * ((n + 31) / 32) < kKSmallMaxWgs || in >= (int64_t(1) << 24));
   const int64_t tile_rows = small ? 16 : tile == kTile32x32 ? 32 : 64;
   int64_t tiles = 0;
   for (int i = 0; i < n_w; ++i) {
     B.tile0[i] = int(tiles);
     tiles += (rows[i] + tile_rows - 1) / tile_rows;
   }
-  const int act = act_of(type);
+  const int act = is_k(type) ? int(kActQ8_K16) : act_of(type);
   const ActLayout l = act_layout(act, n, B.w[0].nb);
   const uint8_t* base = static_cast<const uint8_t*>(acts);
   const QA A{reinterpret_cast<const int8_t*>(base + l.qs_off), reinterpret_cast<const float*>(base + l.d_off),
              act == kActQ8_1 ? reinterpret_cast<const float*>(base + l.s_off) : nullptr,
-             act == kActQ8_K ? reinterpret_cast<const int16_t*>(base + l.bsums_off) : nullptr, B.w[0].nb};
-  const dim3 grid32{unsigned(tiles), unsigned((n + 31) / 32), 1}, block{256, 1, 1};
+             act == kActQ8_K16 ? reinterpret_cast<const int16_t*>(base + l.bsums_off) : nullptr, B.w[0].nb};
   const hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   switch (type) {
-    case kQ4_K: return launch_k<kQ4_K>(small, grid32, s, B, A, n);
-    case kQ5_K: return launch_k<kQ5_K>(small, grid32, s, B, A, n);
-    case kQ6_K: return launch_k<kQ6_K>(small, grid32, s, B, A, n);
+    case kQ4_K: return launch_k<kQ4_K>(small, unsigned(tiles), s, B, A, n);
+    case kQ5_K: return launch_k<kQ5_K>(small, unsigned(tiles), s, B, A, n);
+    case kQ6_K: return launch_k<kQ6_K>(small, unsigned(tiles), s, B, A, n);
     case kQ4_0: return launch_legacy<kQ4_0>(tile, unsigned(tiles), n, s, B, A);
     case kQ5_0: return launch_legacy<kQ5_0>(tile, unsigned(tiles), n, s, B, A);
     case kQ5_1: return launch_legacy<kQ5_1>(tile, unsigned(tiles), n, s, B, A);

@@ -18,13 +18,16 @@
 //
 // Activations are quantized on the device into planes too: qs (int8, 32 or 256 per block), d (float: the
 // block's scale, for Q8_0 / Q8_1 the fp16-rounded value widened exactly), s (float, Q8_1's fp16-rounded sum term)
-// and bsums (int16 x 16 per Q8_K block).
+// and bsums (int16 x 16 per Q8_K block). The tiled K kernels take a form of Q8_K of their own, kActQ8_K16: qs holds
+// 16 a as fp16 (exact) for every quant a, residue w's 32 at halves 32 w, in the order of their A operand (chunk c:
+// sub-block 2c's elements 0, 2, sub-block 2c + 1's 0, 2, then both's 1, 3, element i being w + 8 i); bsums holds, as
+// fp16, b & 63 of each sub-block's quant sum b (sub-blocks 0, 2, 1, 3, 4, 6, 5, 7) and then b >> 6.
 #include <cstdint>
 
 namespace nbh_quant {
 
 enum Type : int { kQ4_0 = 2, kQ5_0 = 6, kQ5_1 = 7, kQ8_0 = 8, kQ4_K = 12, kQ5_K = 13, kQ6_K = 14 };
-enum Act : int { kActQ8_0 = 0, kActQ8_1 = 1, kActQ8_K = 2 };
+enum Act : int { kActQ8_0 = 0, kActQ8_1 = 1, kActQ8_K = 2, kActQ8_K16 = 3 };
 
 constexpr int64_t align256(int64_t v) { return (v + 255) & ~int64_t(255); }
 
@@ -77,12 +80,12 @@ struct ActLayout {
 };
 inline ActLayout act_layout(int act, int64_t n, int64_t nb) {
   ActLayout l{};
-  const int64_t blocks = n * nb, per = act == kActQ8_K ? 256 : 32;
+  const int64_t blocks = n * nb, per = act == kActQ8_K16 ? 512 : act == kActQ8_K ? 256 : 32;
   l.qs_off = 0;
   l.d_off = align256(blocks * per);
   l.s_off = align256(l.d_off + blocks * 4);
   l.bsums_off = align256(l.s_off + (act == kActQ8_1 ? blocks * 4 : 0));
-  l.bytes = align256(l.bsums_off + (act == kActQ8_K ? blocks * 32 : 0));
+  l.bytes = align256(l.bsums_off + (act == kActQ8_K || act == kActQ8_K16 ? blocks * 32 : 0));
   return l;
 }
 

@@ -272,3 +272,37 @@ def test_quant_single_row_over_many_rows(backend, t):
     ref = oracle.matmul_q(t, w.raw, in_, rows, x)
     assert np.array_equal(bits(got), bits(ref))
     backend.release_weights()
+
+
+@pytest.mark.parametrize("extreme", [False, True], ids=["random", "extreme"])
+@pytest.mark.parametrize("nb", [1, 2, 3, 4, 5, 6, 7, 13])
+@pytest.mark.parametrize("t", KTYPES, ids=[U.NAMES[t] for t in KTYPES])
+def test_quant_tiled_k_super_block_counts(backend, t, nb, extreme):
+    """The 64 x 32 K kernel over every length of its unrolled super-block loop (six per trip: one trip cut short at
+    each point, a whole one, two and a rest), rows and activation rows that end inside a tile, row counts that are and
+    are not a multiple of four (vector stores). `extreme`: the operands whose exact sums come closest to the fp32
+    accumulator's 2^24 - every quant and sub-block scale the largest (Q6_K: -32 times -128 and 31 times 127) against
+    activations quantized to +-127. Every output bit-exact."""
+    in_ = 256 * nb
+    for rows, n in ((2497, 33), (1300, 61)):
+        w = U.random_qmat(t, rows, in_, seed=40 + t + nb)
+        x = (np.random.default_rng(nb).standard_normal((n, in_)) * 2).astype(np.float32)
+        if extreme:
+            raw = w.raw.copy().reshape(rows * nb, -1)
+            if t == oracle.Q6_K:
+                raw[:, :192] = 0
+                raw[::2, :192] = 0xFF
+                raw[:, 192:208] = 0x80
+                raw[::2, 192:208] = 0x7F
+            else:
+                raw[:, 4:] = 0xFF  # every scale and minimum 63, every quant 15 (31)
+            w = U.QMat(t, raw.reshape(-1), rows, in_)
+            x = np.where(np.arange(in_) % 7 < 3 * (np.arange(n) % 3)[:, None] // 2, -3.0, 3.0).astype(np.float32)
+        with Buffers(backend) as B:
+            dx, dy = B.upload(x), B.alloc(n * rows)
+            backend.matmul(w, dx, dy, n)
+            got = backend.download(dy, (n, rows))
+        ref = oracle.matmul_q(t, w.raw, in_, rows, x)
+        diff = int(np.sum(bits(got) != bits(ref)))
+        assert diff == 0, (U.NAMES[t], rows, n, nb, diff)
+        backend.release_weights()
