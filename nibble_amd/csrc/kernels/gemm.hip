@@ -10,13 +10,13 @@
 // order of an fp32 GEMM's (the classical bound in * 2^-24 * sum_k |x_k w_k| holds with a wide margin) at two fp16
 // MFMAs per product instead of fp32 arithmetic - and without an fp32 copy of the weights.
 //
-//  * split_acts_kernel: one wave per activation row: the row's largest magnitude, then hi and lo written as fp16
+//  * split_acts_kernel: one workgroup per activation row: the row's largest magnitude, then hi and lo written as fp16
 //    rows padded with zeros to a multiple of the K slice (16-byte stores), and 1 / s_t.
-//  * gemm_f16w_kernel: output tiles of 64 x 64 (64-deep K slices) or, for grids with many tiles, 128 x 128 (32-deep
-//    slices), four waves each on a quarter, K slices through a 3-stage LDS ring filled by direct-to-LDS buffer loads
-//    (rows past the activation count or a weight's row count, and columns past `in`, read as zeros). Per 16-deep
-//    step a wave reads its hi, lo and weight fragments once and issues the lo then the hi MFMA into each
-//    accumulator. Up to kMaxWeights weights sharing x run in one launch over their stacked tiles.
+//  * gemm_f16w_kernel: output tiles of 64 x 64 or, for grids with many tiles, 64 x 128, four waves each on a quarter,
+//    64-deep K slices through an LDS ring filled by direct-to-LDS buffer loads (rows past the activation count or a
+//    weight's row count, and columns past `in`, read as zeros). Per 16-deep step a wave reads its hi, lo and weight
+//    fragments once and issues the lo then the hi MFMA into each accumulator. Up to kMaxWeights weights sharing x run
+//    in one launch over their stacked tiles.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -71,16 +71,19 @@ __device__ __forceinline__ void split_f16(float x, _Float16& hi, _Float16& lo) {
   lo = __builtin_isfinite(h) ? (_Float16)(x - h) : (_Float16)0.f;  // an infinite or NaN hi carries the value alone
 }
 
-// One wave per activation row, each lane on runs of 8 consecutive elements: the row's largest magnitude (a wave
-// reduction), then the hi and lo rows in 16-byte stores. Runs past `in` (up to in_pad) are written as zeros.
-// in % 8 == 0; `vec`: x is 16-byte aligned, so a run is two 16-byte loads. Up to kHeld runs per lane stay in
-// registers between the two passes (rows up to 4096 wide); longer rows read the rest again.
-constexpr int kHeld = 8;
-__global__ __launch_bounds__(64) void split_acts_kernel(const float* __restrict__ x, int64_t in, int64_t in_pad,
-                                                        _Float16* __restrict__ xh, _Float16* __restrict__ xl,
-                                                        float* __restrict__ inv_scale, int vec) {
+// One workgroup per activation row, each thread on runs of 8 consecutive elements: the row's largest magnitude (wave
+// reductions, then LDS), then the hi and lo rows in 16-byte stores. Runs past `in` (up to in_pad) are written as
+// zeros. in % 8 == 0; `vec`: x is 16-byte aligned, so a run is two 16-byte loads. A row is one round trip to memory
+// whatever its width, so it is spread over kSplitThreads threads rather than one wave (512 x 2048: 7.4 -> 6.5 us). Up to
+// kHeld runs per thread stay in registers between the two passes (rows up to 4096 wide); longer rows read the rest
+// again.
+constexpr int kHeld = 2, kSplitThreads = 256;
+__global__ __launch_bounds__(kSplitThreads) void split_acts_kernel(const float* __restrict__ x, int64_t in, int64_t in_pad,
+                                                                   _Float16* __restrict__ xh, _Float16* __restrict__ xl,
+                                                                   float* __restrict__ inv_scale, int vec) {
+  __shared__ float part[kSplitThreads / 64];
   const int64_t t = blockIdx.x;
-  const int lane = threadIdx.x;
+  const int tid = threadIdx.x;
   const float* xr = x + t * in;
   auto load_run = [&](int64_t k, float (&v)[8]) {
     if (k >= in) {
@@ -99,11 +102,11 @@ __global__ __launch_bounds__(64) void split_acts_kernel(const float* __restrict_
   float m = 0.f;
 #pragma unroll
   for (int c = 0; c < kHeld; ++c) {
-    load_run(8 * (lane + int64_t(c) * 64), held[c]);  // runs past in read as zeros
+    load_run(8 * (tid + int64_t(c) * kSplitThreads), held[c]);  // runs past in read as zeros
 #pragma unroll
     for (int e = 0; e < 8; ++e) m = fmaxf(m, fabsf(held[c][e]));  // NaN elements are skipped
   }
-  for (int64_t j = lane + kHeld * 64; j < runs; j += 64) {
+  for (int64_t j = tid + kHeld * kSplitThreads; j < runs; j += kSplitThreads) {
     float v[8];
     load_run(8 * j, v);
 #pragma unroll
@@ -111,6 +114,10 @@ __global__ __launch_bounds__(64) void split_acts_kernel(const float* __restrict_
   }
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
+  if ((tid & 63) == 0) part[tid >> 6] = m;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < kSplitThreads / 64; ++w) m = fmaxf(m, part[w]);
   // s = 2^e with m s in [2^13, 2^14): m in [2^(ex-1), 2^ex) gives e = 14 - ex. A zero or infinite row is not scaled;
   // e is capped so that s and 1 / s stay normal floats (x s is then exact unless it is an fp32 subnormal).
   int e = 0;
@@ -120,7 +127,7 @@ __global__ __launch_bounds__(64) void split_acts_kernel(const float* __restrict_
     e = min(14 - ex, 120);
   }
   const float sc = ldexpf(1.0f, e);
-  if (lane == 0) inv_scale[t] = ldexpf(1.0f, -e);
+  if (tid == 0) inv_scale[t] = ldexpf(1.0f, -e);
   auto store_run = [&](int64_t j, const float (&v)[8]) {
     half8_t h, l;
 #pragma unroll
@@ -135,10 +142,10 @@ __global__ __launch_bounds__(64) void split_acts_kernel(const float* __restrict_
   };
 #pragma unroll
   for (int c = 0; c < kHeld; ++c) {
-    const int64_t j = lane + int64_t(c) * 64;
+    const int64_t j = tid + int64_t(c) * kSplitThreads;
     if (j < runs) store_run(j, held[c]);
   }
-  for (int64_t j = lane + kHeld * 64; j < runs; j += 64) {
+  for (int64_t j = tid + kHeld * kSplitThreads; j < runs; j += kSplitThreads) {
     float v[8];
     load_run(8 * j, v);
     store_run(j, v);
@@ -146,28 +153,27 @@ __global__ __launch_bounds__(64) void split_acts_kernel(const float* __restrict_
 }
 
 // Tile configuration: BM activation rows x BN weight rows per tile (each of the four waves takes BM/2 x BN/2),
-// BK-deep K slices, a STAGES-deep LDS ring. Two instances, chosen per weight: 128 x 128 tiles with 32-deep slices for
-// a weight that alone makes at least kWideMinTiles of them (an FFN gate or up projection at 512 rows: each operand
-// byte fetched from L2 serves twice the products), 64 x 64 tiles with 64-deep slices otherwise (a 512-row QKV or
-// FFN-down projection: more workgroups to spread the operand traffic). Both keep 72 KB of LDS per workgroup.
-constexpr int kSmallBM = 64, kSmallBN = 64, kSmallBK = 64, kSmallStages = 3;
-constexpr int kWideBM = 128, kWideBN = 128, kWideBK = 32, kWideStages = 3;
-constexpr int kPadK = 64;  // K padding of the split activation rows (a multiple of both slice depths)
-constexpr int64_t kWideMinTiles = 256;
-// K ranges of a weight with few 128 x 128 tiles: up to kMaxSplit, each at least kSplitMinKTiles 32-deep slices
-// (1536 elements; measured at 512 rows: an FFN-down projection, K = 8192, 108 -> 80 us in 4 ranges; a QKV one, K =
-// 2048, 38 -> 40 us in 4 ranges of 512, whose partial sums cost more than the halved operand traffic saves, so it is
-// not cut); the partial sums live in a fixed area of the workspace (64 MB), which bounds a split weight's outputs.
-constexpr int kMaxSplit = 4, kSplitMinKTiles = 48;
-// K ranges of a weight's 64 x 64 tiles in calls of few rows, where the tiles are too few to fill the CUs and each
-// walks the whole K: up to kFewMaxSplit ranges of at least kFewMinKTiles 64-deep slices, while the weight's tiles
-// times its ranges stay within kFewMinWgs (measured at the QKV shape, K = 2048, 3072 output rows: 12-64 rows,
-// 27-29 -> 15-19 us per call; 65-128 rows, 29-30 -> 19-22 us; FFN gate + up and down shapes unchanged. A target of
-// 512 workgroups, up to 256 rows, gained 2-4 us at 192-256 QKV rows but cost gate + up 4-10 us at 32-128 rows).
-// Such calls take these ranges rather than the wide tiles' ones above, whose few 128 x 128 tiles would leave most CUs
-// idle (FFN down, K = 8192, 2048 output rows: 17-64 rows 61-64 -> 28-30 us, 96-128 rows 64-65 -> 40-41 us).
-constexpr int kFewMaxRows = 128, kFewMaxSplit = 8, kFewMinKTiles = 4;
-constexpr int64_t kFewMinWgs = 256;
+// BK-deep K slices, a STAGES-deep LDS ring. Two instances, chosen per launch: 64 x 128 tiles with a 2-stage ring when the
+// launch has at least kWideMinTiles of them (each activation byte fetched from L2 serves twice the products: 16384
+// weight rows x 512, K = 2048: 105 -> 81 us, x 200: 48 -> 39), 64 x 64 tiles with a 3-stage ring otherwise (more
+// workgroups: QKV, 3072 x 512, 22.5 us against 25.4 with 192 tiles of 64 x 128). Both accumulate an output's products
+// in the same order, so its bits do not depend on the choice. 64-72 KB of LDS: two workgroups per CU, one of which
+// multiplies while the other waits; 128 x 128 tiles with 32-deep slices measured 84 us at 16384 x 512. Tiles whose four
+// waves split K and not the outputs (half the LDS reads; one workgroup per CU with a ring of 4-6 slices, the waves'
+// sums added at the end) were no faster: QKV 22.7, 16384 x 512 96 us - what the deeper ring gains goes to each
+// workgroup's fixed part, which nothing overlaps.
+constexpr int kBM = 64, kBK = 64, kSmallBN = 64, kSmallStages = 3, kWideBN = 128, kWideStages = 2;
+constexpr int kPadK = 64;  // K padding of the split activation rows (a multiple of the slice depth)
+constexpr int64_t kWideMinTiles = 384;
+// K ranges of a weight whose 64 x 64 tiles are too few to fill the CUs and each walk the whole K: up to kMaxSplit
+// ranges, doubling while the weight's tiles times its ranges stay within kSplitWgs, of at least kFewMinSlices slices in
+// calls of up to kFewMaxRows activation rows (QKV shape, K = 2048, 3072 weight rows: 12-64 rows 27-29 -> 15-19 us per
+// call, 65-128 rows 29-30 -> 19-22) and kMinSlices in longer ones (K = 8192, 2048 weight rows x 140, after a
+// gate + up that is not split: 130 -> 92 us for the block, against 128 x 128 tiles in K ranges). A target of
+// 512 workgroups gained 2-4 us at 192-256 QKV rows but cost gate + up 4-10 us at 32-128 rows. The partial sums live
+// in a fixed area of the workspace (64 MB), which bounds a split weight's outputs.
+constexpr int kFewMaxRows = 128, kMaxSplit = 8, kFewMinSlices = 4, kMinSlices = 32;
+constexpr int64_t kSplitWgs = 256;
 constexpr int64_t kSplitPartFloats = int64_t(1) << 24;
 
 template <int BM, int BN, int BK, int STAGES>
@@ -184,7 +190,7 @@ __global__ __launch_bounds__(kThreads) void gemm_f16w_kernel(GemmBatch b, const 
   int wi = 0;
   for (int j = 1; j < b.n_w; ++j)
     if (int(blockIdx.x) >= b.w[j].tile0) wi = j;
-  const GemmWeight& d = b.w[wi];
+  const GemmWeight d = b.w[wi];
   // this workgroup's output tile and K range: workgroups of a split weight are tile-major within each range
   const int local = int(blockIdx.x) - d.tile0, tiles = int((d.rows + BN - 1) / BN);
   const int ks = local / tiles;
@@ -194,7 +200,9 @@ __global__ __launch_bounds__(kThreads) void gemm_f16w_kernel(GemmBatch b, const 
 
   // Buffer resources over the valid rows only: reads past the activation count or the weight's row count return
   // zeros (their results are never stored), so no row index is clamped.
-  const uint32_t xrows = uint32_t(min<int64_t>(n - m0, BM)), wrows = uint32_t(min<int64_t>(d.rows - n0, BN));
+  // (Compared by hand: HIP's min of int64_t goes through double on the VALU, which would put the resources in vector
+  // registers and every load below in a loop over their values.)
+  const uint32_t xrows = uint32_t(n - m0 < BM ? n - m0 : BM), wrows = uint32_t(d.rows - n0 < BN ? d.rows - n0 : BN);
   const __amdgpu_buffer_rsrc_t rh = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<_Float16*>(xh + m0 * in_pad), 0, int(xrows * uint32_t(in_pad) * 2), 0x00020000);
   const __amdgpu_buffer_rsrc_t rl = __builtin_amdgcn_make_buffer_rsrc(
@@ -330,17 +338,26 @@ __global__ __launch_bounds__(kThreads) void gemm_f16w_kernel(GemmBatch b, const 
 
   // acc[i][j][r] holds activation row 8 (r / 4) + 4 hf + r % 4 of the wave's block i and weight row lane % 32 of
   // its block j. A K range's partial sums go unscaled to its slice of part.
-  float* const dst = d.split > 1 ? d.part + int64_t(ks) * n * d.rows : d.y;
+  const int tr = wm * (BM / 2) + 4 * hf;  // of the tile: the lane's row at r = 0
+  float inv[MB][16];
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int t = tr + 32 * i + 8 * (r / 4) + (r % 4);
+      inv[i][r] = d.split > 1 ? 1.f : inv_scale[m0 + (t < int(xrows) ? t : 0)];
+    }
+  float* const dst = (d.split > 1 ? d.part + int64_t(ks) * n * d.rows : d.y) + m0 * d.rows + n0;
 #pragma unroll
   for (int j = 0; j < NB; ++j) {
-    const int64_t col = n0 + wn * (BN / 2) + 32 * j + (lane & 31);
-    if (col < d.rows) {
+    const int col = wn * (BN / 2) + 32 * j + (lane & 31);
+    if (col < int(wrows)) {
 #pragma unroll
       for (int i = 0; i < MB; ++i)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-          const int64_t t = m0 + wm * (BM / 2) + 32 * i + 8 * (r / 4) + 4 * hf + (r % 4);
-          if (t < n) dst[t * d.rows + col] = d.split > 1 ? acc[i][j][r] : acc[i][j][r] * inv_scale[t];
+          const int t = tr + 32 * i + 8 * (r / 4) + (r % 4);
+          if (t < int(xrows)) dst[int64_t(t) * d.rows + col] = acc[i][j][r] * inv[i][r];
         }
     }
   }
@@ -387,8 +404,7 @@ int nbhs_gemm_f16w_multi(int n_w, const void* const* w, float* const* y, const i
   if (need < 0 || ws_bytes < need || reinterpret_cast<uintptr_t>(ws) % 256 != 0) return NBHS_EINVAL;
   const int64_t in_pad = round_up(in, kPadK);
   // every operand a buffer resource addresses must fit 32-bit offsets
-  if (kWideBM * in_pad * 2 > INT32_MAX || kWideBN * in * 2 > INT32_MAX || n > 65535 * int64_t(kSmallBM))
-    return NBHS_EINVAL;
+  if (kWideBN * in_pad * 2 > INT32_MAX || n > 65535 * int64_t(kBM)) return NBHS_EINVAL;
   // every weight is checked before anything is launched, so a rejected call writes no output
   for (int i = 0; i < n_w; ++i)
     if (!w[i] || !y[i] || rows[i] <= 0 || rows[i] > INT32_MAX || reinterpret_cast<uintptr_t>(w[i]) % 16 != 0)
@@ -400,88 +416,58 @@ int nbhs_gemm_f16w_multi(int n_w, const void* const* w, float* const* y, const i
   float* part = reinterpret_cast<float*>(base + round_up(2 * n * in_pad * 2, 256) + round_up(n * 4, 256));
   const hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   const int vec = reinterpret_cast<uintptr_t>(x) % 16 == 0 ? 1 : 0;
-  const unsigned wide_rows = unsigned((n + kWideBM - 1) / kWideBM), small_rows = unsigned((n + kSmallBM - 1) / kSmallBM);
-  // Each weight's configuration follows from its own shape (so its results do not depend on the other weights of
-  // the call: matmul_multi equals separate calls): 128 x 128 tiles when they alone are many; otherwise, when K is
-  // long and the output fits the partial-sum area, 128 x 128 tiles over 2 or 4 K ranges (each range's workgroup
-  // fetches half the operand bytes per product of a 64 x 64 tile's, and the ranges restore the workgroup count;
-  // the partials are summed in range order); otherwise 64 x 64 tiles. The weights of each configuration share a
-  // launch; split weights share one while their partials fit the area, then the next group starts.
-  GemmBatch wide{}, small{}, split{}, fsplit{};
-  int64_t wide_tiles = 0, small_tiles = 0, split_wgs = 0, split_out = 0, fsplit_wgs = 0, fsplit_out = 0,
-          part_used = 0;
-  hipError_t e = nbhs_timing::launch(NBHS_K_SPLIT_ACTS, split_acts_kernel, dim3(unsigned(n)), dim3(64), s, x, in,
-                                     in_pad, xh, xl, inv, vec);
-  // the weights taking K ranges (128 x 128 tiles, or 64 x 64 ones in calls of few rows), whose partial sums share
-  // the partial-sum area: their launches and sums, then the area is free again
-  auto flush_split = [&]() {
-    if (e == hipSuccess && split.n_w > 0) {
-      e = nbhs_timing::launch(NBHS_K_GEMM, gemm_f16w_kernel<kWideBM, kWideBN, kWideBK, kWideStages>,
-                              dim3(unsigned(split_wgs), wide_rows), dim3(kThreads), s, split, xh, xl, inv, n, in,
-                              in_pad);
-      if (e == hipSuccess)
-        e = nbhs_timing::launch(NBHS_K_GEMM_REDUCE, gemm_split_reduce_kernel,
-                                dim3(unsigned((split_out + 255) / 256)), dim3(256), s, split, inv, n, split_out);
+  const int64_t mt = (n + kBM - 1) / kBM;
+  hipError_t e = nbhs_timing::launch(NBHS_K_SPLIT_ACTS, split_acts_kernel, dim3(unsigned(n)), dim3(kSplitThreads), s,
+                                     x, in, in_pad, xh, xl, inv, vec);
+  // Each weight's K ranges follow from its own shape, so its results do not depend on the other weights of the call
+  // (matmul_multi equals separate calls). The weights share a launch while the split ones' partial sums fit their area,
+  // then the next group starts.
+  GemmBatch g{}, split{};  // the group, and its split weights
+  int64_t part_used = 0, split_out = 0;
+  auto flush = [&]() {
+    if (e != hipSuccess || g.n_w == 0) return;
+    auto tiles = [&](int bn, bool set) {
+      int64_t x0 = 0;
+      for (int i = 0; i < g.n_w; ++i) {
+        if (set) g.w[i].tile0 = int(x0);
+        x0 += (g.w[i].rows + bn - 1) / bn * g.w[i].split;
+      }
+      return x0;
+    };
+    const bool wide = tiles(kWideBN, false) * mt >= kWideMinTiles;
+    const int64_t xt = tiles(wide ? kWideBN : kSmallBN, true);
+    if (xt > INT32_MAX) {
+      e = hipErrorInvalidValue;
+      return;
     }
-    if (e == hipSuccess && fsplit.n_w > 0) {
-      e = nbhs_timing::launch(NBHS_K_GEMM, gemm_f16w_kernel<kSmallBM, kSmallBN, kSmallBK, kSmallStages>,
-                              dim3(unsigned(fsplit_wgs), small_rows), dim3(kThreads), s, fsplit, xh, xl, inv, n, in,
-                              in_pad);
-      if (e == hipSuccess)
-        e = nbhs_timing::launch(NBHS_K_GEMM_REDUCE, gemm_split_reduce_kernel,
-                                dim3(unsigned((fsplit_out + 255) / 256)), dim3(256), s, fsplit, inv, n, fsplit_out);
-    }
-    split = fsplit = GemmBatch{};
-    split_wgs = split_out = fsplit_wgs = fsplit_out = part_used = 0;
+    const dim3 grid{unsigned(xt), unsigned(mt)};
+    e = wide ? nbhs_timing::launch(NBHS_K_GEMM, gemm_f16w_kernel<kBM, kWideBN, kBK, kWideStages>, grid, dim3(kThreads), s,
+                                   g, xh, xl, inv, n, in, in_pad)
+             : nbhs_timing::launch(NBHS_K_GEMM, gemm_f16w_kernel<kBM, kSmallBN, kBK, kSmallStages>, grid,
+                                   dim3(kThreads), s, g, xh, xl, inv, n, in, in_pad);
+    if (e == hipSuccess && split.n_w > 0)
+      e = nbhs_timing::launch(NBHS_K_GEMM_REDUCE, gemm_split_reduce_kernel, dim3(unsigned((split_out + 255) / 256)),
+                              dim3(256), s, split, inv, n, split_out);
+    g = split = GemmBatch{};
+    part_used = split_out = 0;
   };
-  for (int i = 0; i < n_w && e == hipSuccess; ++i) {
-    const int64_t wt = (rows[i] + kWideBN - 1) / kWideBN * wide_rows;
+  for (int i = 0; i < n_w; ++i) {
+    const int64_t st = (rows[i] + kSmallBN - 1) / kSmallBN * mt, slices = in_pad / kBK;
+    const int64_t min_slices = n <= kFewMaxRows ? kFewMinSlices : kMinSlices;
     int sp = 1;
-    if (wt < kWideMinTiles && n > kFewMaxRows && n * rows[i] * kMaxSplit <= kSplitPartFloats) {
-      const int64_t nkt = in_pad / kWideBK;
-      while (sp < kMaxSplit && wt * sp < kWideMinTiles && nkt / (2 * sp) >= kSplitMinKTiles) sp *= 2;
-    }
-    const _Float16* wd = static_cast<const _Float16*>(w[i]);
-    if (wt >= kWideMinTiles) {
-      wide.w[wide.n_w++] = GemmWeight{wd, y[i], rows[i], int(wide_tiles), 1, nullptr};
-      wide_tiles += (rows[i] + kWideBN - 1) / kWideBN;
-    } else if (sp > 1) {
-      const int64_t cnt = n * rows[i] * sp;
-      if (part_used + cnt > kSplitPartFloats) flush_split();
-      split.w[split.n_w++] = GemmWeight{wd, y[i], rows[i], int(split_wgs), sp, part + part_used};
-      split_wgs += (rows[i] + kWideBN - 1) / kWideBN * sp;
-      split_out += n * rows[i];
+    if (n * rows[i] * kMaxSplit <= kSplitPartFloats)
+      while (sp < kMaxSplit && st * sp * 2 <= kSplitWgs && slices / (2 * sp) >= min_slices) sp *= 2;
+    const int64_t cnt = sp > 1 ? n * rows[i] * sp : 0;
+    if (part_used + cnt > kSplitPartFloats) flush();
+    g.w[g.n_w++] =
+        GemmWeight{static_cast<const _Float16*>(w[i]), y[i], rows[i], 0, sp, sp > 1 ? part + part_used : nullptr};
+    if (sp > 1) {
+      split.w[split.n_w++] = g.w[g.n_w - 1];
       part_used += cnt;
-    } else {
-      const int64_t st = (rows[i] + kSmallBN - 1) / kSmallBN * small_rows;
-      int fsp = 1;
-      if (n <= kFewMaxRows && n * rows[i] * kFewMaxSplit <= kSplitPartFloats) {
-        const int64_t nkt = in_pad / kSmallBK;
-        while (fsp < kFewMaxSplit && st * fsp * 2 <= kFewMinWgs && nkt / (2 * fsp) >= kFewMinKTiles) fsp *= 2;
-      }
-      if (fsp > 1) {
-        const int64_t cnt = n * rows[i] * fsp;
-        if (part_used + cnt > kSplitPartFloats) flush_split();
-        fsplit.w[fsplit.n_w++] = GemmWeight{wd, y[i], rows[i], int(fsplit_wgs), fsp, part + part_used};
-        fsplit_wgs += (rows[i] + kSmallBN - 1) / kSmallBN * fsp;
-        fsplit_out += n * rows[i];
-        part_used += cnt;
-      } else {
-        small.w[small.n_w++] = GemmWeight{wd, y[i], rows[i], int(small_tiles), 1, nullptr};
-        small_tiles += (rows[i] + kSmallBN - 1) / kSmallBN;
-      }
+      split_out += n * rows[i];
     }
-    if (wide_tiles > INT32_MAX || small_tiles > INT32_MAX || split_wgs > INT32_MAX || fsplit_wgs > INT32_MAX)
-      return NBHS_EINVAL;
   }
-  flush_split();
-  if (e == hipSuccess && wide.n_w > 0)
-    e = nbhs_timing::launch(NBHS_K_GEMM, gemm_f16w_kernel<kWideBM, kWideBN, kWideBK, kWideStages>,
-                            dim3(unsigned(wide_tiles), wide_rows), dim3(kThreads), s, wide, xh, xl, inv, n, in, in_pad);
-  if (e == hipSuccess && small.n_w > 0)
-    e = nbhs_timing::launch(NBHS_K_GEMM, gemm_f16w_kernel<kSmallBM, kSmallBN, kSmallBK, kSmallStages>,
-                            dim3(unsigned(small_tiles), small_rows), dim3(kThreads), s, small, xh, xl, inv, n, in,
-                            in_pad);
+  flush();
   return e;
 }
 

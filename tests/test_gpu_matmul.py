@@ -350,3 +350,29 @@ def test_f16_gemm_few_rows_k_ranges(backend, n):
             assert_matmul_close(g, w, x, f"in {in_}, weight {i} ({w.shape[0]} rows), n {n}")
             assert np.array_equal(bits(g), bits(sep[i])), f"weight {i}: matmul_multi differs from a separate call"
     backend.release_weights()
+
+
+@pytest.mark.parametrize("in_", [64, 200, 1096], ids=["one-slice", "short", "many-slices"])
+def test_f16_gemm_wide_tiles(backend, in_):
+    """A launch with enough 64 x 128 tiles to take them (12300 + 130 weight rows, 250 activation rows: 98 x 4), both
+    row counts ending inside a tile and K inside a slice, and the same weights in calls of their own: the small one then
+    takes 64 x 64 tiles, with the same bits."""
+    rng = np.random.default_rng(in_)
+    n = 250
+    ws = [rand(rng, (12300, in_), np.float16, in_ ** -0.5), rand(rng, (130, in_), np.float16, in_ ** -0.5)]
+    x = rand(rng, (n, in_))
+    x[3] *= 1e20
+    x[7, 1:] = 0
+    with Buffers(backend) as B:
+        dx = B.upload(x)
+        ys = [B.alloc(n * w.shape[0]) for w in ws]
+        backend.matmul_multi(ws, dx, ys, n)
+        got = [backend.download(y, (n, w.shape[0])) for y, w in zip(ys, ws)]
+    pick = np.r_[0:130, 6000:6100, 12200:12300]  # the reference on a part of the large weight's rows
+    for g, w, rows in zip(got, ws, (pick, np.arange(130))):
+        exact = x.astype(np.float64) @ w[rows].astype(np.float64).T
+        bound = in_ * U * (np.abs(x.astype(np.float64)) @ np.abs(w[rows].astype(np.float64)).T) + 1e-37
+        assert np.all(np.abs(g[:, rows] - exact) <= bound)
+    for g, w in zip(got, ws):
+        assert np.array_equal(bits(gpu_matmul(backend, w, x, n)), bits(g))
+    backend.release_weights()
