@@ -267,9 +267,12 @@ int nbhs_gemm_f16w_multi(int n_w, const void* const* w, float* const* y, const i
 
 /* ---- the other per-token ops (Backend::embed / rmsnorm / add / silu_mul, backend.h:55-70) ---- */
 
-/* out[t, :] = row ids[t] of table [rows, d] (F32, or F16 widened exactly); ids in device memory, already checked
- * against the row count by the caller (ref_ops.cpp:80-99). */
-int nbhs_embed(int f16, const void* table, const int32_t* ids, int64_t n, int64_t d, float* out, nbhs_stream s);
+/* Host ids that an embedding launch carries as its argument. */
+#define NBHS_EMBED_ARG_IDS 512
+/* out[t, :] = row ids[t] of a float table (F32 copied, F16 widened exactly). The ids are n <= NBHS_EMBED_ARG_IDS host
+ * ones, read before the call returns, or (host_ids NULL) device ones. */
+int nbhs_embed(int f16, const void* table, const int32_t* host_ids, const int32_t* ids, int64_t n, int64_t d, float* out,
+               nbhs_stream s);
 /* ref_ops.cpp:137-148: y[t] = float(x[t] * scale * w) with scale = 1 / sqrt(sum(x^2) / d + eps) in double. */
 int nbhs_rmsnorm_f32(const float* x, const float* w, float* y, int64_t n, int64_t d, float eps, nbhs_stream s);
 /* x[i] += y[i] (ref_ops.cpp:151-153). */
@@ -301,9 +304,10 @@ int nbhs_quantize_acts_rm(int type, const float* x, int64_t n, int64_t in, void*
  * as nbhs_qgemv_multi. */
 int nbhs_qgemm_multi(int type, int n_w, const void* const* w, const int64_t* rows, float* const* y, int64_t in,
                      const void* acts, int64_t n, nbhs_stream s);
-/* out[t, :] = dequantized row ids[t] (device ids) of the weight, quant.cpp:157-242 bit for bit. */
-int nbhs_dequant_rows(int type, const void* w, int64_t rows, int64_t in, const int32_t* ids, int64_t n, float* out,
-                      nbhs_stream s);
+/* out[t, :] = dequantized row ids[t] of the weight, quant.cpp:157-242 bit for bit. The ids are n <= NBHS_EMBED_ARG_IDS
+ * host ones, read before the call returns, or (host_ids NULL) device ones. */
+int nbhs_dequant_rows(int type, const void* w, int64_t rows, int64_t in, const int32_t* host_ids, const int32_t* ids,
+                      int64_t n, float* out, nbhs_stream s);
 
 /* ---- per-kernel timing (measurement only) ----
  * While enabled for a kernel, its launcher launches it with a HIP event pair (hipExtLaunchKernel) stamped from the

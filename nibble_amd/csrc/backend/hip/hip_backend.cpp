@@ -650,16 +650,17 @@ void HipBackend::embed(const Tensor& table, std::span<const int32_t> ids, float*
   if (d <= 0 || overflow_mul(n, d, &count)) throw Error("embed: invalid table width " + str(d));
   check_range(out, count, "embed", "out");
   const DeviceWeight w = device_weight(table, "embed");
-  ensure(ids_buf_, ids_buf_bytes_, size_t(n) * sizeof(int32_t));
-  check(nbhs_memcpy_h2d(ids_buf_, ids.data(), size_t(n) * sizeof(int32_t), stream_), "embed ids upload");
-  if (nbh_quant::is_quant(int(w.type))) {
-    check(nbhs_dequant_rows(int(w.type), w.dev, w.rows, d, reinterpret_cast<const int32_t*>(ids_buf_), n, out,
-                            stream_),
-          "embed (dequantize)");
-    return;
+  // the ids of a call of this size travel in the launch; more go through a buffer (and a wait for the stream)
+  const int32_t* host_ids = n <= NBHS_EMBED_ARG_IDS ? ids.data() : nullptr;
+  if (!host_ids) {
+    ensure(ids_buf_, ids_buf_bytes_, size_t(n) * sizeof(int32_t));
+    check(nbhs_memcpy_h2d(ids_buf_, ids.data(), size_t(n) * sizeof(int32_t), stream_), "embed ids upload");
   }
-  check(nbhs_embed(w.type == DType::F16, w.dev, reinterpret_cast<const int32_t*>(ids_buf_), n, d, out, stream_),
-        "embed");
+  const auto* dev_ids = reinterpret_cast<const int32_t*>(ids_buf_);
+  if (nbh_quant::is_quant(int(w.type)))
+    check(nbhs_dequant_rows(int(w.type), w.dev, w.rows, d, host_ids, dev_ids, n, out, stream_), "embed (dequantize)");
+  else
+    check(nbhs_embed(w.type == DType::F16, w.dev, host_ids, dev_ids, n, d, out, stream_), "embed");
 }
 
 void HipBackend::rmsnorm(const float* x, const Tensor& weight, float* y, int64_t n, float eps) {

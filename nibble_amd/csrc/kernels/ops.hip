@@ -11,6 +11,8 @@
 // All four are HBM-bound streams.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "backend/hip/kernel_timing.h"
 #include "nibble_hip_shim.h"
 
@@ -23,12 +25,17 @@ unsigned grid_for(int64_t count) {
   return unsigned(blocks < 8192 ? (blocks > 0 ? blocks : 1) : 8192);
 }
 
+struct EmbedIds {
+  int32_t id[NBHS_EMBED_ARG_IDS];
+};
+
 // out[t, :] = row ids[t] of the table, widened to float. One workgroup per output row.
 template <bool F16>
-__global__ __launch_bounds__(kThreads) void embed_kernel(const void* __restrict__ table, const int32_t* __restrict__ ids,
-                                                         float* __restrict__ out, int64_t d) {
+__global__ __launch_bounds__(kThreads) void embed_kernel(const void* __restrict__ table, EmbedIds ids,
+                                                         const int32_t* __restrict__ far_ids, float* __restrict__ out,
+                                                         int64_t d) {
   const int64_t t = blockIdx.x;
-  const int64_t id = ids[t];
+  const int64_t id = far_ids ? far_ids[t] : ids.id[t];
   float* o = out + t * d;
   if constexpr (F16) {
     const _Float16* r = static_cast<const _Float16*>(table) + id * d;
@@ -89,14 +96,20 @@ __global__ __launch_bounds__(kThreads) void silu_mul_kernel(float* __restrict__ 
 
 extern "C" {
 
-int nbhs_embed(int f16, const void* table, const int32_t* ids, int64_t n, int64_t d, float* out, nbhs_stream s) {
-  if (!table || !ids || !out || n <= 0 || d <= 0 || n >= (int64_t(1) << 31)) return NBHS_EINVAL;
+int nbhs_embed(int f16, const void* table, const int32_t* host_ids, const int32_t* ids, int64_t n, int64_t d, float* out,
+               nbhs_stream s) {
+  if (!table || !(host_ids ? n <= NBHS_EMBED_ARG_IDS : ids != nullptr) || !out || n <= 0 || d <= 0 ||
+      n >= (int64_t(1) << 31))
+    return NBHS_EINVAL;
   const hipStream_t st = reinterpret_cast<hipStream_t>(s);
+  EmbedIds arg{};
+  if (host_ids) std::copy(host_ids, host_ids + n, arg.id);
+  const int32_t* const dev_ids = host_ids ? nullptr : ids;
   if (f16)
-    return nbhs_timing::launch(NBHS_K_ELEMENTWISE, embed_kernel<true>, dim3(unsigned(n)), dim3(kThreads), st, table,
-                               ids, out, d);
-  return nbhs_timing::launch(NBHS_K_ELEMENTWISE, embed_kernel<false>, dim3(unsigned(n)), dim3(kThreads), st, table,
-                             ids, out, d);
+    return nbhs_timing::launch(NBHS_K_ELEMENTWISE, embed_kernel<true>, dim3(unsigned(n)), dim3(kThreads), st, table, arg,
+                               dev_ids, out, d);
+  return nbhs_timing::launch(NBHS_K_ELEMENTWISE, embed_kernel<false>, dim3(unsigned(n)), dim3(kThreads), st, table, arg,
+                             dev_ids, out, d);
 }
 
 int nbhs_rmsnorm_f32(const float* x, const float* w, float* y, int64_t n, int64_t d, float eps, nbhs_stream s) {

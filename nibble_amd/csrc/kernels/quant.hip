@@ -23,6 +23,7 @@
 // launch (into LDS, once per wave and block), with the same bits as the standalone quantizer.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "backend/hip/kernel_timing.h"
@@ -64,6 +65,49 @@ typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
 typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 typedef float floatx4_t __attribute__((ext_vector_type(4)));
+// Quant words as native vectors (a uint4 copy is a memcpy that keeps the value in scratch).
+typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
+
+// Lane exchanges on the VALU (DPP), a few cycles each where a __shfl goes through LDS: within quads, and mirrored within
+// 8 and 16 lanes. In this order they are the steps of a reduction over 16 lanes.
+template <int CTRL>
+__device__ __forceinline__ int dpp(int v) {
+  return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xF, 0xF, true);
+}
+template <int CTRL>
+__device__ __forceinline__ float dpp(float v) {
+  return __builtin_bit_cast(float, dpp<CTRL>(__builtin_bit_cast(int, v)));
+}
+constexpr int kQuadXor1 = 0xB1, kQuadXor2 = 0x4E, kMirror8 = 0x141, kMirror16 = 0x140;
+__device__ __forceinline__ int lane_int(int v, int l) { return __builtin_amdgcn_readlane(v, l); }
+
+// The first element of largest magnitude of a quantization block sets the sign of its scale: every lane gives its own
+// largest magnitude (NaN never counts) and 2 * (its first element of that magnitude) + (that element's sign bit).
+// Returns the block's value; KEYS lanes (8 consecutive ones, or the wave's 64) share a block.
+template <int KEYS>
+__device__ __forceinline__ float block_max(float amax, int key, float& out_amax) {
+  float m = amax;
+  m = fmaxf(m, dpp<kQuadXor1>(m));
+  m = fmaxf(m, dpp<kQuadXor2>(m));
+  m = fmaxf(m, dpp<kMirror8>(m));
+  if constexpr (KEYS == 64) {
+    m = fmaxf(m, dpp<kMirror16>(m));
+    const int b = __builtin_bit_cast(int, m);
+    m = fmaxf(fmaxf(__builtin_bit_cast(float, lane_int(b, 0)), __builtin_bit_cast(float, lane_int(b, 16))),
+              fmaxf(__builtin_bit_cast(float, lane_int(b, 32)), __builtin_bit_cast(float, lane_int(b, 48))));
+  }
+  int k = amax == m ? key : 0x7FFFFFFF;
+  k = min(k, dpp<kQuadXor1>(k));
+  k = min(k, dpp<kQuadXor2>(k));
+  k = min(k, dpp<kMirror8>(k));
+  if constexpr (KEYS == 64) {
+    k = min(k, dpp<kMirror16>(k));
+    k = min(min(lane_int(k, 0), lane_int(k, 16)), min(lane_int(k, 32), lane_int(k, 48)));
+  }
+  out_amax = m;
+  return k & 1 ? -m : m;
+}
 
 __device__ __forceinline__ int sdot4(uint32_t a, uint32_t b, int c) {
   return __builtin_amdgcn_sdot4(int(a), int(b), c, false);
@@ -118,37 +162,24 @@ __device__ __forceinline__ int nearest_int(float f) {
   return (__float_as_int(val) & 0x007fffff) - 0x00400000;
 }
 
-// One wave per 256-element super-block; lane l = 8k + w holds elements 32k + w + 8i (i < 4) of sub-block k: the four
-// elements of residue word w, which it stores as word w of the sub-block (residue order, quant_layout.h).
-// RM: the tiled K kernels' operand form instead (quant_layout.h, kActQ8_K16): 16 times each quant as fp16, residue
-// by residue, and each sub-block's sum of its quants as two fp16 digits.
-template <bool RM>
-__global__ __launch_bounds__(64) void quantize_q8k_kernel(const float* __restrict__ x, int64_t in,
-                                                          int8_t* __restrict__ qs, float* __restrict__ dq,
-                                                          int16_t* __restrict__ bsums) {
-  const int64_t nb = in / 256, i = blockIdx.x;
-  const int lane = threadIdx.x, k = lane >> 3, w = lane & 7;
-  const float* xb = x + (i / nb) * in + (i % nb) * 256 + 32 * k + w;
+// quantize_row_q8_K (quant.cpp:273-303) of one super-block by a wave; lane l = 8k + w holds elements 32k + w + 8i
+// (i < 4) of sub-block k, at xb[8 i]: its four quants, its sub-block's two 16-sums and the block's scale.
+__device__ __forceinline__ void q8k_lane(const float* xb, int lane, int (&q)[4], int& b0, int& b1, float& d) {
+  const int k = lane >> 3, w = lane & 7;
   const float v[4] = {xb[0], xb[8], xb[16], xb[24]};
-  // the first element of largest magnitude (strictly greater replaces; NaN never does)
-  float amax = 0.f, mx = 0.f;
-  int idx = 1 << 30;
+  float own = 0.f, amax;
+  int key = 0;
   bool nan = false;
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
     const float ax = fabsf(v[e]);
-    if (ax > amax) amax = ax, mx = v[e], idx = 32 * k + w + 8 * e;
+    if (ax > own) own = ax, key = 2 * (32 * k + w + 8 * e) + (v[e] < 0.f ? 1 : 0);
     nan |= v[e] != v[e];
   }
-#pragma unroll
-  for (int m = 1; m < 64; m <<= 1) {
-    const float oa = __shfl_xor(amax, m, 64), om = __shfl_xor(mx, m, 64);
-    const int oi = __shfl_xor(idx, m, 64);
-    if (oa > amax || (oa == amax && oi < idx)) amax = oa, mx = om, idx = oi;
-  }
+  const float mx = block_max<64>(own, key, amax);
   nan = __builtin_amdgcn_ballot_w64(nan) != 0;
-  int q[4] = {0, 0, 0, 0};
-  float d = 0.f;
+  d = 0.f;
+  q[0] = q[1] = q[2] = q[3] = 0;
   if (amax != 0.f) {
     const float iscale = __fdiv_rn(-127.f, mx);
 #pragma unroll
@@ -158,10 +189,27 @@ __global__ __launch_bounds__(64) void quantize_q8k_kernel(const float* __restric
     }
     d = __fdiv_rn(1.f, iscale);
   }
+  if (nan) d = __builtin_nanf("");
   // the sub-block's two 16-sums (elements w, w + 8 | w + 16, w + 24 of each lane)
-  int b0 = q[0] + q[1], b1 = q[2] + q[3];
-#pragma unroll
-  for (int m = 1; m < 8; m <<= 1) b0 += __shfl_xor(b0, m, 64), b1 += __shfl_xor(b1, m, 64);
+  b0 = q[0] + q[1], b1 = q[2] + q[3];
+  b0 += dpp<kQuadXor1>(b0), b1 += dpp<kQuadXor1>(b1);
+  b0 += dpp<kQuadXor2>(b0), b1 += dpp<kQuadXor2>(b1);
+  b0 += dpp<kMirror8>(b0), b1 += dpp<kMirror8>(b1);
+}
+
+// One wave per super-block; a lane's four quants are residue word w of its sub-block, which it stores as word w of the
+// sub-block (residue order, quant_layout.h).
+// RM: the tiled K kernels' operand form instead (quant_layout.h, kActQ8_K16): 16 times each quant as fp16, residue
+// by residue, and each sub-block's sum of its quants as two fp16 digits.
+template <bool RM>
+__global__ __launch_bounds__(64) void quantize_q8k_kernel(const float* __restrict__ x, int64_t in,
+                                                          int8_t* __restrict__ qs, float* __restrict__ dq,
+                                                          int16_t* __restrict__ bsums) {
+  const int64_t nb = in / 256, i = blockIdx.x;
+  const int lane = threadIdx.x, k = lane >> 3, w = lane & 7;
+  int q[4], b0, b1;
+  float d;
+  q8k_lane(x + (i / nb) * in + (i % nb) * 256 + 32 * k + w, lane, q, b0, b1, d);
   if constexpr (RM) {
     // chunk k / 2 of residue w: sub-block k's elements (0, 2) at halves 2 (k % 2), (1, 3) at 4 + 2 (k % 2)
     _Float16* o = reinterpret_cast<_Float16*>(qs) + i * 256 + 32 * w + 8 * (k >> 1) + 2 * (k & 1);
@@ -181,7 +229,7 @@ __global__ __launch_bounds__(64) void quantize_q8k_kernel(const float* __restric
     reinterpret_cast<uint32_t*>(qs + i * 256)[lane] = word;
     if (w == 0) bsums[i * 16 + 2 * k] = int16_t(b0), bsums[i * 16 + 2 * k + 1] = int16_t(b1);
   }
-  if (lane == 0) dq[i] = nan ? __builtin_nanf("") : d;
+  if (lane == 0) dq[i] = d;
 }
 
 // ---- activation blocks ----
@@ -257,21 +305,18 @@ __device__ __forceinline__ void quant_act_k(const float* xs, int k, uint32_t (&a
     const float4 f = *reinterpret_cast<const float4*>(xs + j);
     v[j] = f.x, v[j + 1] = f.y, v[j + 2] = f.z, v[j + 3] = f.w;
   }
-  float amax = 0.f, mx = 0.f;
-  int idx = 1 << 30, nanf = 0;
+  float own = 0.f, amax;
+  int key = 0, nanf = 0;
 #pragma unroll
   for (int e = 0; e < 32; ++e) {
     const float ax = fabsf(v[e]);
-    if (ax > amax) amax = ax, mx = v[e], idx = 32 * k + e;
+    if (ax > own) own = ax, key = 2 * (32 * k + e) + (v[e] < 0.f ? 1 : 0);
     nanf |= v[e] != v[e];
   }
-#pragma unroll
-  for (int m = 1; m < 8; m <<= 1) {
-    const float oa = __shfl_xor(amax, m, 64), om = __shfl_xor(mx, m, 64);
-    const int oi = __shfl_xor(idx, m, 64);
-    if (oa > amax || (oa == amax && oi < idx)) amax = oa, mx = om, idx = oi;
-    nanf |= __shfl_xor(nanf, m, 64);
-  }
+  const float mx = block_max<8>(own, key, amax);
+  nanf |= dpp<kQuadXor1>(nanf);
+  nanf |= dpp<kQuadXor2>(nanf);
+  nanf |= dpp<kMirror8>(nanf);
   int q[32];
   d = 0.f;
   bs0 = bs1 = 0;
@@ -632,6 +677,226 @@ __global__ __launch_bounds__(64) void qgemv_kernel(QBatch B, QA A, const float* 
   }
 }
 
+// ---- the K types with up to 4 activation rows ----
+//
+// kgemv_kernel: a workgroup of four waves quantizes the activation rows into LDS once, together, and each wave then
+// takes weight rows of its own. Four lanes share a (row, super-block) pair: lane c takes the 32-byte chunk c of its quants
+// (sub-blocks 2 c and 2 c + 1; Q6_K: sub-blocks k and k + 2, k = 4 (c / 2) + c % 2), so a wave's 16 pairs are 16 whole
+// super-blocks read contiguously, and its two sub-blocks' activation words stay in registers for every row. The four
+// lanes' integer lane sums are added exactly by DPP, lane c keeping aux[2 c] and aux[2 c + 1]; their float terms go to
+// the wave's LDS slice and are then added in super-block order, a lane per (row, integer lane) chain: the reference's
+// operations in its order (quant.cpp:118-144, 394-416).
+// It is bound by memory latency at decode sizes: a pass of 16 pairs is 2.3-3.4 KB per wave, so P passes are requested
+// before any is computed. The kernel it replaces gave a lane a whole super-block (64 scattered 128-byte reads an
+// instruction) and had every wave quantize the activations by itself, super-block chunk after chunk. Measured (start
+// to here): 131072 weight rows, K = 2048, Q6_K 72 -> 52 us (4.2 TB/s), Q4_K 57 -> 36; 2048 rows, K = 8192, Q6_K 20 -> 12;
+// 3072 rows, K = 2048, Q4_K 6.4 -> 5.8, three activation rows 14.2 -> 9.5.
+constexpr int kGemvChunk = 16;  // super-blocks of a pass
+constexpr int kgemv_max_sb(int nt) { return nt == 1 ? 64 : 32; }  // super-blocks of a row, at most (LDS)
+
+// Sum over the four lanes of a quad, lane c keeping values 2 c and 2 c + 1 of 8.
+__device__ __forceinline__ void quad_reduce(const int (&v)[8], int c, int& r0, int& r1) {
+  int h[4];
+  const bool hi = (c & 2) != 0, odd = (c & 1) != 0;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) h[i] = (hi ? v[4 + i] : v[i]) + dpp<kQuadXor2>(hi ? v[i] : v[4 + i]);
+  r0 = (odd ? h[2] : h[0]) + dpp<kQuadXor1>(odd ? h[0] : h[2]);
+  r1 = (odd ? h[3] : h[1]) + dpp<kQuadXor1>(odd ? h[1] : h[3]);
+}
+
+template <int T>
+struct KChunk {  // a lane's share of a (row, super-block) pair, as loaded
+  u32x4_t q[2], h[2];
+  u32x4_t sc;   // Q4_K / Q5_K: the 12 packed bytes; Q6_K: words 0, 1 hold the 8 scales of half c / 2
+  uint16_t d, m;
+  __device__ __forceinline__ void load(const QW& W, int64_t wb, int c) {
+    const u32x4_t* qp = reinterpret_cast<const u32x4_t*>(W.q + wb * 128 + 32 * c);
+    q[0] = __builtin_nontemporal_load(qp), q[1] = __builtin_nontemporal_load(qp + 1);
+    if constexpr (T == kQ5_K) {
+      const u32x4_t* hp = reinterpret_cast<const u32x4_t*>(W.h + wb * 32);
+      h[0] = hp[0], h[1] = hp[1];
+    }
+    if constexpr (T == kQ6_K) {
+      const u32x4_t* hp = reinterpret_cast<const u32x4_t*>(W.h + wb * 64 + 32 * (c >> 1));
+      h[0] = hp[0], h[1] = hp[1];
+      const u32x2_t s = *reinterpret_cast<const u32x2_t*>(W.s + wb * 16 + 8 * (c >> 1));
+      sc[0] = s[0], sc[1] = s[1];
+    } else {
+      sc = *reinterpret_cast<const u32x4_t*>(W.s + wb * 16);
+      m = W.m[wb];
+    }
+    d = W.d[wb];
+  }
+};
+
+// NT activation rows at most, super-blocks per row at most MAXSB, P passes in flight.
+template <int T, int NT, int P>
+__global__ __launch_bounds__(256) void kgemv_kernel(QBatch B, const float* __restrict__ x, int64_t in, int n, int batches) {
+  constexpr int MAXSB = kgemv_max_sb(NT);
+  constexpr int TS = kGemvChunk + 1;  // floats per chain of terms (one of padding)
+  constexpr int CH = T == kQ6_K ? 8 : 9;
+  __shared__ __align__(16) uint32_t qs[NT][MAXSB][64];
+  __shared__ float ad[NT][MAXSB];
+  __shared__ int bsum[NT][T == kQ6_K ? 1 : MAXSB][8];
+  constexpr int RB = 8;  // rows of a wave's batch, at most: a lane per (row, integer lane)
+  __shared__ float terms[4][RB][CH][TS];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c = lane & 3;
+  int wi = 0;
+  for (int j = 1; j < B.n_w; ++j)
+    if (int64_t(blockIdx.x) >= B.wave0[j]) wi = j;
+  const QW W = B.w[wi];
+  float* __restrict__ y = B.y[wi];
+  const int nb = int(W.nb), nbc = nb < kGemvChunk ? nb : kGemvChunk, rp = kGemvChunk / nbc;  // rows of a pass
+  const int rb = P * rp < RB ? P * rp : RB, np = (rb + rp - 1) / rp;                          // rows, passes of a batch
+  const int u = lane >> 2, ur = u / nbc, us = u - ur * nbc;  // this lane's row and super-block within a pass
+  const int64_t r00 = ((int64_t(blockIdx.x) - B.wave0[wi]) * 4 + wave) * rb * batches;
+  // the first weight loads, ahead of the activation work
+  KChunk<T> k[P];
+  auto load_pass = [&](int64_t r0, int s0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+      const int64_t r = r0 + p * rp + ur;
+      k[p].load(W, (r < W.rows ? r : W.rows - 1) * nb + (s0 + us < nb ? s0 + us : nb - 1), c);
+    }
+  };
+  load_pass(r00, 0);
+  // quantize_row_q8_K (quant.cpp:273-303), the same bits either way: few super-blocks a wave each, four elements per
+  // lane; many eight lanes each, 32 elements per lane
+  if (n * nb <= 16) {
+    for (int i = wave; i < n * nb; i += 4) {
+      const int t = i / nb, sb = i - t * nb, kk = lane >> 3, w = lane & 7;
+      int q[4], b0, b1;
+      float d;
+      q8k_lane(x + int64_t(t) * in + sb * 256 + 32 * kk + w, lane, q, b0, b1, d);
+      qs[t][sb][lane] = uint32_t(q[0] & 0xFF) | uint32_t(q[1] & 0xFF) << 8 | uint32_t(q[2] & 0xFF) << 16 |
+                        uint32_t(q[3] & 0xFF) << 24;
+      if (T != kQ6_K && w == 0) bsum[t][T == kQ6_K ? 0 : sb][kk] = b0 + b1;
+      if (lane == 0) ad[t][sb] = d;
+    }
+  } else {
+    for (int i0 = 0; i0 < n * nb; i0 += 32) {
+      const int i = i0 + (tid >> 3), kk = lane & 7, ic = i < n * nb ? i : 0;
+      const int t = ic / nb, sb = ic - t * nb;
+      uint32_t aw[8];
+      int b0, b1;
+      float d;
+      quant_act_k(x + int64_t(t) * in + sb * 256 + 32 * kk, kk, aw, b0, b1, d);
+      if (i < n * nb) {
+#pragma unroll
+        for (int w = 0; w < 8; ++w) qs[t][sb][8 * kk + w] = aw[w];
+        if constexpr (T != kQ6_K) bsum[t][sb][kk] = b0 + b1;
+        if (kk == 0) ad[t][sb] = d;
+      }
+    }
+  }
+  __syncthreads();
+  const int k0 = T == kQ6_K ? 4 * (c >> 1) + (c & 1) : 2 * c, k1 = T == kQ6_K ? k0 + 2 : k0 + 1;  // its sub-blocks
+  const int cr = lane >> 3, cl = lane & 7;  // the chain this lane adds: row of the batch, integer lane
+  for (int b = 0; b < batches; ++b) {
+    const int64_t r0 = r00 + int64_t(b) * rb;
+    if (r0 >= W.rows) break;  // (a wave leaves alone: no workgroup barrier follows)
+    float sum[NT], acc[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) sum[t] = acc[t] = 0.f;
+    for (int s0 = 0; s0 < nb; s0 += kGemvChunk) {
+      if (b > 0 || s0 > 0) load_pass(r0, s0);
+      const int sb = s0 + us < nb ? s0 + us : nb - 1;
+      const int nc = nb - s0 < kGemvChunk ? nb - s0 : kGemvChunk;
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        if (t >= n) break;
+        uint32_t a0[8], a1[8];
+        load32(reinterpret_cast<const uint8_t*>(&qs[t][sb][8 * k0]), a0);
+        load32(reinterpret_cast<const uint8_t*>(&qs[t][sb][8 * k1]), a1);
+        const float da = ad[t][sb];
+#pragma unroll
+        for (int p = 0; p < P; ++p) {
+          if (p >= np) break;
+          const KChunk<T>& K = k[p];
+          int aux[8], sumi = 0;
+          if constexpr (T == kQ6_K) {
+            const int sh = 16 * (c & 1);  // scales of sub-block k0: bytes 2 (c % 2), + 1 of the half; of k1: + 4
+            const int s0l = int8_t(K.sc[0] >> sh), s0h = int8_t(K.sc[0] >> (sh + 8));
+            const int s1l = int8_t(K.sc[1] >> sh), s1h = int8_t(K.sc[1] >> (sh + 8));
+            const int hs = 2 * (c & 1);  // bits of sub-block k0 in a high-bit byte; of k1: + 4
+#pragma unroll
+            for (int w = 0; w < 8; ++w) {
+              const uint32_t qw = K.q[w >> 2][w & 3], hw = K.h[w >> 2][w & 3] >> hs;
+              // values less 32, bytewise: (v | 128) - 32 never borrows, and the top bit flips back
+              const uint32_t v0 = (((qw & 0x0F0F0F0Fu) | ((hw & 0x03030303u) << 4) | 0x80808080u) - 0x20202020u) ^ 0x80808080u;
+              const uint32_t v1 =
+                  ((((qw >> 4) & 0x0F0F0F0Fu) | (hw & 0x30303030u) | 0x80808080u) - 0x20202020u) ^ 0x80808080u;
+              aux[w] = s0l * sdot4(v0 & 0xFFFFu, a0[w], 0) + s0h * sdot4(v0 & 0xFFFF0000u, a0[w], 0) +
+                       s1l * sdot4(v1 & 0xFFFFu, a1[w], 0) + s1h * sdot4(v1 & 0xFFFF0000u, a1[w], 0);
+            }
+          } else {
+            const uint32_t hi = c >= 2 ? ~0u : 0u;  // get_scale_min_k4 (quant.cpp:52-61), four sub-blocks to a word
+            const uint32_t d4 =
+                (((K.sc[2] & 0x0F0F0F0Fu) | ((K.sc[0] >> 2) & 0x30303030u)) & hi) | (K.sc[0] & 0x3F3F3F3Fu & ~hi);
+            const uint32_t m4 =
+                ((((K.sc[2] >> 4) & 0x0F0F0F0Fu) | ((K.sc[1] >> 2) & 0x30303030u)) & hi) | (K.sc[1] & 0x3F3F3F3Fu & ~hi);
+            const int sh = 16 * (c & 1);
+            const int s0_ = int((d4 >> sh) & 0xFFu), s1_ = int((d4 >> (sh + 8)) & 0xFFu);
+#pragma unroll
+            for (int w = 0; w < 8; ++w) {
+              const uint32_t qw = K.q[w >> 2][w & 3];
+              uint32_t v0 = qw & 0x0F0F0F0Fu, v1 = (qw >> 4) & 0x0F0F0F0Fu;
+              if constexpr (T == kQ5_K) {
+                const uint32_t hw = K.h[w >> 2][w & 3] >> (2 * c);
+                v0 |= (hw & 0x01010101u) << 4;
+                v1 |= (hw & 0x02020202u) << 3;
+              }
+              aux[w] = s0_ * sdot4(v0, a0[w], 0) + s1_ * sdot4(v1, a1[w], 0);
+            }
+            sumi = bsum[t][T == kQ6_K ? 0 : sb][2 * c] * int((m4 >> sh) & 0xFFu) +
+                   bsum[t][T == kQ6_K ? 0 : sb][2 * c + 1] * int((m4 >> (sh + 8)) & 0xFFu);
+          }
+          int x0, x1;
+          quad_reduce(aux, c, x0, x1);
+          const float d = __fmul_rn(h2f(K.d), da);
+          const int br = p * rp + ur;  // row of the batch
+          if (ur < rp && br < rb) {
+            float* o = &terms[wave][br][0][us];
+            o[(2 * c) * TS] = __fmul_rn(d, float(x0));
+            o[(2 * c + 1) * TS] = __fmul_rn(d, float(x1));
+          }
+          if constexpr (T != kQ6_K) {
+            sumi += dpp<kQuadXor1>(sumi);
+            sumi += dpp<kQuadXor2>(sumi);
+            if (c == 0 && ur < rp && br < rb) terms[wave][br][CH - 1][us] = __fmul_rn(__fmul_rn(h2f(K.m), da), float(sumi));
+          }
+        }
+        // the wave's terms of this chunk, in super-block order (LDS operations of one wave complete in order)
+        __builtin_amdgcn_wave_barrier();
+        const float* tp = &terms[wave][cr][cl][0];
+        const float* mp = &terms[wave][cr][CH - 1][0];
+        float tv[kGemvChunk], mv[kGemvChunk];
+#pragma unroll
+        for (int i = 0; i < kGemvChunk; ++i) {  // (past nc: read, not added)
+          tv[i] = tp[i];
+          if constexpr (T != kQ6_K) mv[i] = mp[i];
+        }
+#pragma unroll
+        for (int i = 0; i < kGemvChunk; ++i) {
+          if (i < nc) {
+            sum[t] = __fadd_rn(sum[t], tv[i]);
+            if constexpr (T != kQ6_K) acc[t] = __fsub_rn(acc[t], mv[i]);
+          }
+        }
+        __builtin_amdgcn_wave_barrier();
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      if (t >= n) break;
+      float o = acc[t];
+#pragma unroll
+      for (int l = 0; l < 8; ++l) o = __fadd_rn(o, __shfl(sum[t], (lane & 56) + l, 64));
+      if (cl == 0 && cr < rb && r0 + cr < W.rows) y[int64_t(t) * W.rows + r0 + cr] = o;
+    }
+  }
+}
+
 // ---- the tiled matmul for longer calls (prefill chunks) ----
 //
 // qgemm_legacy_kernel: a 256-thread workgroup computes 64 weight rows x 16 TJ activation rows on the int8 matrix
@@ -656,9 +921,6 @@ struct QGemmBatch {  // weights of one type sharing one input; tile0[i]: first r
   int n_w;
 };
 
-// Staged quant words as a native vector type (a uint4 copy is a memcpy that keeps the staging share in scratch).
-typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 typedef int i32x4_t __attribute__((ext_vector_type(4)));  // an integer MFMA result
 
 template <int T, int TJ, int WRT = 64>
@@ -1425,64 +1687,49 @@ hipError_t launch_k(bool small, unsigned tiles, hipStream_t s, const QGemmBatch&
   return nbhs_timing::launch(NBHS_K_QGEMM, qgemm_k_kernel<T>, grid, dim3(256), s, B, A, n);
 }
 
-// ---- dequantization (quant.cpp:157-242), one thread per block of one output row ----
+// ---- dequantization (quant.cpp:157-242), one thread per output element ----
 
+// The ids of a call that fit a kernel argument travel in it: no copy to the device, no wait for the stream.
+struct EmbedIds {
+  int32_t id[NBHS_EMBED_ARG_IDS];
+};
+
+// Element e of block wb of the weight: the reference's expression for it.
 template <int T>
-__global__ __launch_bounds__(256) void dequant_rows_kernel(QW W, const int32_t* __restrict__ ids, int64_t n,
-                                                           float* __restrict__ out) {
-  const int64_t be = block_elems(T), d_ = W.nb * be;
-  const int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x;
-  if (i >= n * W.nb) return;
-  const int64_t t = i / W.nb, b = i % W.nb, wb = int64_t(ids[t]) * W.nb + b;
-  float* o = out + t * d_ + b * be;
+__device__ __forceinline__ float dequant_one(const QW& W, int64_t wb, int e) {
   const float d = h2f(W.d[wb]);
   if constexpr (T == kQ8_0) {
-    const int8_t* q = reinterpret_cast<const int8_t*>(W.q + wb * 32);
-    for (int j = 0; j < 32; ++j) o[j] = __fmul_rn(float(q[j]), d);
+    return __fmul_rn(float(reinterpret_cast<const int8_t*>(W.q)[wb * 32 + e]), d);
   } else if constexpr (T == kQ4_0 || T == kQ5_0 || T == kQ5_1) {
-    const uint8_t* q = W.q + wb * 16;
-    const uint32_t qh = T == kQ4_0 ? 0u : *reinterpret_cast<const uint32_t*>(W.h + wb * 4);
-    const float m = T == kQ5_1 ? h2f(W.m[wb]) : 0.f;
-    for (int j = 0; j < 16; ++j) {
-      int x0 = q[j] & 0x0F, x1 = q[j] >> 4;
-      if constexpr (T != kQ4_0) x0 |= ((qh >> j) & 1) << 4, x1 |= ((qh >> (j + 16)) & 1) << 4;
-      if constexpr (T == kQ5_1) {
-        o[j] = __fadd_rn(__fmul_rn(float(x0), d), m);
-        o[j + 16] = __fadd_rn(__fmul_rn(float(x1), d), m);
-      } else {
-        constexpr int bias = T == kQ4_0 ? 8 : 16;
-        o[j] = __fmul_rn(float(x0 - bias), d);
-        o[j + 16] = __fmul_rn(float(x1 - bias), d);
-      }
-    }
+    int q = (W.q[wb * 16 + (e & 15)] >> (e < 16 ? 0 : 4)) & 0x0F;
+    if constexpr (T != kQ4_0) q |= ((reinterpret_cast<const uint32_t*>(W.h)[wb] >> e) & 1u) << 4;
+    if constexpr (T == kQ5_1) return __fadd_rn(__fmul_rn(float(q), d), h2f(W.m[wb]));
+    return __fmul_rn(float(q - (T == kQ4_0 ? 8 : 16)), d);
   } else if constexpr (T == kQ4_K || T == kQ5_K) {
-    const uint8_t* qs = W.q + wb * 128;
-    const float mn = h2f(W.m[wb]);
-    for (int k = 0; k < 8; ++k) {
-      int sc, m;
-      scale_min_k4(k, W.s + wb * 16, sc, m);
-      const float d1 = __fmul_rn(d, float(sc)), m1 = __fmul_rn(mn, float(m));
-      for (int e = 0; e < 32; ++e) {
-        const int p = residue_pos(e);
-        int q = (qs[32 * (k >> 1) + p] >> (4 * (k & 1))) & 0xF;
-        if constexpr (T == kQ5_K) q += ((W.h[wb * 32 + p] >> k) & 1) ? 16 : 0;
-        o[32 * k + e] = __fsub_rn(__fmul_rn(d1, float(q)), m1);
-      }
-    }
+    const int k = e >> 5, p = residue_pos(e & 31);
+    int sc, m;
+    scale_min_k4(k, W.s + wb * 16, sc, m);
+    int q = (W.q[wb * 128 + 32 * (k >> 1) + p] >> (4 * (k & 1))) & 0xF;
+    if constexpr (T == kQ5_K) q += ((W.h[wb * 32 + p] >> k) & 1) ? 16 : 0;
+    return __fsub_rn(__fmul_rn(__fmul_rn(d, float(sc)), float(q)), __fmul_rn(h2f(W.m[wb]), float(m)));
   } else {  // Q6_K
-    const int8_t* scl = reinterpret_cast<const int8_t*>(W.s + wb * 16);
-    for (int k = 0; k < 8; ++k) {
-      const int h = k >> 2, g = k & 3;
-      const uint8_t* ql = W.q + wb * 128 + 64 * h + 32 * (g & 1);
-      const uint8_t* qh = W.h + wb * 64 + 32 * h;
-      for (int e = 0; e < 32; ++e) {
-        const int p = residue_pos(e);
-        const int q = (((ql[p] >> ((g >> 1) * 4)) & 0xF) | (((qh[p] >> (2 * g)) & 3) << 4)) - 32;
-        const float dk = __fmul_rn(d, float(scl[2 * k + (e >> 4)]));
-        o[32 * k + e] = __fmul_rn(dk, float(q));
-      }
-    }
+    const int k = e >> 5, h = k >> 2, g = k & 3, p = residue_pos(e & 31);
+    const int q = (((W.q[wb * 128 + 64 * h + 32 * (g & 1) + p] >> ((g >> 1) * 4)) & 0xF) |
+                   (((W.h[wb * 64 + 32 * h + p] >> (2 * g)) & 3) << 4)) - 32;
+    return __fmul_rn(__fmul_rn(d, float(reinterpret_cast<const int8_t*>(W.s)[wb * 16 + (e >> 4)])), float(q));
   }
+}
+
+// Row blockIdx.y's elements. (A thread per block, which this replaces, took 40 us for one row of Q6_K, K = 2048: eight
+// threads, 256 dependent loads and stores each; now 5.)
+template <int T>
+__global__ __launch_bounds__(256) void dequant_rows_kernel(QW W, EmbedIds ids, const int32_t* __restrict__ far_ids,
+                                                           int64_t row0, float* __restrict__ out) {
+  constexpr int be = int(block_elems(T));
+  const int64_t in = W.nb * be, i = int64_t(blockIdx.x) * 256 + threadIdx.x, t = row0 + blockIdx.y;
+  if (i >= in) return;
+  const int64_t id = far_ids ? far_ids[t] : ids.id[blockIdx.y];
+  out[t * in + i] = dequant_one<T>(W, id * W.nb + i / be, int(i % be));
 }
 
 QW weight_of(int type, const void* w, int64_t rows, int64_t in) {
@@ -1493,11 +1740,42 @@ QW weight_of(int type, const void* w, int64_t rows, int64_t in) {
             reinterpret_cast<const uint16_t*>(base + l.m_off), rows, nb};
 }
 
+// Passes in flight per wave while that leaves the launch half of kKGemvWaves waves, and batches while it leaves all of
+// them (measured with 1024 .. 16384 waves: 131072 rows of Q4_K 48 / 38 / 35 / 40 / 42 us at 1 / 2 / 4 / 8 / 16 x 1024;
+// 16384 rows 9.6 us with four passes in flight and 2048 waves, 10.2 with two and 4096).
+constexpr int64_t kKGemvWaves = 4096;
+template <int T>
+int launch_kgemv(const QBatch& B, const int64_t* rows, int n_w, const float* x, int64_t in, int64_t n, hipStream_t s) {
+  const int64_t nb = in / 256, rp = kGemvChunk / (nb < kGemvChunk ? nb : kGemvChunk);
+  int64_t total = 0;
+  for (int i = 0; i < n_w; ++i) total += rows[i];
+  const int64_t passes = (total + rp - 1) / rp / kKGemvWaves;  // of each wave, at that size
+  const int p = passes >= 2 && 4 * rp <= 8 ? 4 : passes >= 1 && 2 * rp <= 8 ? 2 : 1;
+  const int64_t rb = std::min<int64_t>(p * rp, 8), batches = std::max<int64_t>(1, total / rb / kKGemvWaves);
+  QBatch b = B;
+  int64_t wgs = 0;
+  for (int i = 0; i < n_w; ++i) b.wave0[i] = wgs, wgs += (rows[i] + 4 * rb * batches - 1) / (4 * rb * batches);
+  if (wgs >= (int64_t(1) << 31) || batches > INT32_MAX) return NBHS_EINVAL;
+  const dim3 grid{unsigned(wgs), 1, 1}, block{256, 1, 1};
+  auto go = [&](auto nt, auto pc) {
+    return nbhs_timing::launch(NBHS_K_QGEMV, kgemv_kernel<T, decltype(nt)::value, decltype(pc)::value>, grid, block, s, b,
+                               x, in, int(n), int(batches));
+  };
+  using I1 = std::integral_constant<int, 1>;
+  using I2 = std::integral_constant<int, 2>;
+  using I4 = std::integral_constant<int, 4>;
+  if (n == 1) return p == 4 ? go(I1{}, I4{}) : p == 2 ? go(I1{}, I2{}) : go(I1{}, I1{});
+  return p == 4 ? go(I4{}, I4{}) : p == 2 ? go(I4{}, I2{}) : go(I4{}, I1{});
+}
+
 template <int T>
 int launch_gemv(const QBatch& B, const int64_t* rows, int n_w, const QA& A, const float* x, int64_t in, int64_t n,
                 bool fused, hipStream_t s) {
   int64_t total = 0;
   for (int i = 0; i < n_w; ++i) total += rows[i];
+  if constexpr (is_k(T)) {
+    if (fused && in / 256 <= kgemv_max_sb(n == 1 ? 1 : 4)) return launch_kgemv<T>(B, rows, n_w, x, in, n, s);
+  }
   const bool wide = fused && n == 1 && total >= kWideRows;
   const int rw = rows_per_wave(is_k(T), fused ? (n == 1 ? 1 : 4) : (n <= 4 ? 4 : 16), wide);
   QBatch b = B;
@@ -1517,11 +1795,19 @@ int launch_gemv(const QBatch& B, const int64_t* rows, int n_w, const QA& A, cons
   return nbhs_timing::launch(NBHS_K_QGEMV, qgemv_kernel<T, 16, false, false>, grid, block, s, b, A, x, in, int(n));
 }
 
+// ids: host_ids, at most NBHS_EMBED_ARG_IDS, or device memory.
 template <int T>
-int launch_dequant(const QW& W, const int32_t* ids, int64_t n, float* out, hipStream_t s) {
-  const int64_t blocks = (n * W.nb + 255) / 256;
-  return nbhs_timing::launch(NBHS_K_ELEMENTWISE, dequant_rows_kernel<T>, dim3(unsigned(blocks)), dim3(256), s, W, ids,
-                             n, out);
+int launch_dequant(const QW& W, const int32_t* host_ids, const int32_t* ids, int64_t n, float* out, hipStream_t s) {
+  const int64_t in = W.nb * block_elems(T);
+  EmbedIds arg{};
+  if (host_ids) std::copy(host_ids, host_ids + n, arg.id);
+  for (int64_t t0 = 0; t0 < n; t0 += 65535) {
+    const dim3 grid{unsigned((in + 255) / 256), unsigned(std::min<int64_t>(n - t0, 65535))};
+    const hipError_t e = nbhs_timing::launch(NBHS_K_ELEMENTWISE, dequant_rows_kernel<T>, grid, dim3(256), s, W, arg,
+                                             host_ids ? nullptr : ids, t0, out);
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
 }
 
 }  // namespace
@@ -1672,21 +1958,21 @@ int nbhs_qgemm_multi(int type, int n_w, const void* const* w, const int64_t* row
   }
 }
 
-int nbhs_dequant_rows(int type, const void* w, int64_t rows, int64_t in, const int32_t* ids, int64_t n, float* out,
-                      nbhs_stream stream) {
-  if (!is_quant(type) || !w || !ids || !out || rows <= 0 || in <= 0 || in % block_elems(type) || n <= 0)
+int nbhs_dequant_rows(int type, const void* w, int64_t rows, int64_t in, const int32_t* host_ids, const int32_t* ids,
+                      int64_t n, float* out, nbhs_stream stream) {
+  if (!is_quant(type) || !w || !(host_ids ? n <= NBHS_EMBED_ARG_IDS : ids != nullptr) || !out || rows <= 0 || in <= 0 ||
+      in % block_elems(type) || n <= 0 || (in + 255) / 256 >= (int64_t(1) << 31))
     return NBHS_EINVAL;
   const QW W = weight_of(type, w, rows, in);
-  if ((n * W.nb + 255) / 256 >= (int64_t(1) << 31)) return NBHS_EINVAL;
   const hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   switch (type) {
-    case kQ4_0: return launch_dequant<kQ4_0>(W, ids, n, out, s);
-    case kQ5_0: return launch_dequant<kQ5_0>(W, ids, n, out, s);
-    case kQ5_1: return launch_dequant<kQ5_1>(W, ids, n, out, s);
-    case kQ8_0: return launch_dequant<kQ8_0>(W, ids, n, out, s);
-    case kQ4_K: return launch_dequant<kQ4_K>(W, ids, n, out, s);
-    case kQ5_K: return launch_dequant<kQ5_K>(W, ids, n, out, s);
-    case kQ6_K: return launch_dequant<kQ6_K>(W, ids, n, out, s);
+    case kQ4_0: return launch_dequant<kQ4_0>(W, host_ids, ids, n, out, s);
+    case kQ5_0: return launch_dequant<kQ5_0>(W, host_ids, ids, n, out, s);
+    case kQ5_1: return launch_dequant<kQ5_1>(W, host_ids, ids, n, out, s);
+    case kQ8_0: return launch_dequant<kQ8_0>(W, host_ids, ids, n, out, s);
+    case kQ4_K: return launch_dequant<kQ4_K>(W, host_ids, ids, n, out, s);
+    case kQ5_K: return launch_dequant<kQ5_K>(W, host_ids, ids, n, out, s);
+    case kQ6_K: return launch_dequant<kQ6_K>(W, host_ids, ids, n, out, s);
     default: return NBHS_EINVAL;
   }
 }

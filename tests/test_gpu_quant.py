@@ -306,3 +306,29 @@ def test_quant_tiled_k_super_block_counts(backend, t, nb, extreme):
         diff = int(np.sum(bits(got) != bits(ref)))
         assert diff == 0, (U.NAMES[t], rows, n, nb, diff)
         backend.release_weights()
+
+
+@pytest.mark.parametrize("n", [1, 2, 4])
+@pytest.mark.parametrize("t", KTYPES, ids=[U.NAMES[t] for t in KTYPES])
+def test_quant_k_few_rows_every_width(backend, t, n):
+    """The K types' kernel for up to 4 activation rows (16 super-blocks a pass): rows of 1-16 super-blocks (16, 8, 5 ..
+    1 weight rows a pass, the last lanes idle where 16 is no multiple), two and three passes a row with a partial last
+    one, the widest row of its LDS and the next, which takes the general kernel; row counts that end inside a wave's
+    batch, and enough rows for several passes in flight and several batches a wave. Every output bit-exact."""
+    wide = 64 if n == 1 else 32
+    cases = [(nb, 41) for nb in (1, 2, 3, 5, 7, 8, 9, 15, 16, 17, 33, wide, wide + 1)]
+    cases += [(1, 70001), (2, 17003), (3, 40003)]
+    for nb, rows in cases:
+        in_ = 256 * nb
+        w = U.random_qmat(t, rows, in_, seed=nb + t) if rows < 1000 else U.QMat(
+            t, np.tile(U.random_qmat(t, 512, in_, seed=nb).raw, -(-rows // 512))[:rows * nb * oracle.block_bytes(t)],
+            rows, in_)
+        x = (np.random.default_rng(nb).standard_normal((n, in_)) * 2).astype(np.float32)
+        with Buffers(backend) as B:
+            dx, dy = B.upload(x), B.alloc(n * rows)
+            backend.matmul(w, dx, dy, n)
+            got = backend.download(dy, (n, rows))
+        ref = oracle.matmul_q(t, w.raw, in_, rows, x)
+        diff = int(np.sum(bits(got) != bits(ref)))
+        assert diff == 0, (U.NAMES[t], nb, rows, n, diff)
+        backend.release_weights()
