@@ -46,36 +46,66 @@ __global__ __launch_bounds__(kThreads) void embed_kernel(const void* __restrict_
   }
 }
 
-__device__ __forceinline__ double wave_sum_f64(double v) {
-#pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) v += __shfl_xor(v, m, 64);
-  return v;
+// A value from another lane of the 16-lane row, by DPP (a few cycles; a double __shfl is two trips through LDS).
+template <int CTRL>
+__device__ __forceinline__ double dpp_f64(double v) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = __builtin_amdgcn_update_dpp(0, int(uint32_t(b)), CTRL, 0xF, 0xF, true);
+  const uint32_t hi = __builtin_amdgcn_update_dpp(0, int(uint32_t(b >> 32)), CTRL, 0xF, 0xF, true);
+  return __builtin_bit_cast(double, uint64_t(hi) << 32 | lo);
+}
+__device__ __forceinline__ double lane_f64(double v, int l) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = __builtin_amdgcn_readlane(int(uint32_t(b)), l), hi = __builtin_amdgcn_readlane(int(uint32_t(b >> 32)), l);
+  return __builtin_bit_cast(double, uint64_t(hi) << 32 | lo);
 }
 
-// One workgroup per row of d elements.
+__device__ __forceinline__ double wave_sum_f64(double v) {
+  v += dpp_f64<0xB1>(v);   // quad_perm [1,0,3,2]
+  v += dpp_f64<0x4E>(v);   // quad_perm [2,3,0,1]
+  v += dpp_f64<0x141>(v);  // row_half_mirror
+  v += dpp_f64<0x140>(v);  // row_mirror
+  return (lane_f64(v, 0) + lane_f64(v, 16)) + (lane_f64(v, 32) + lane_f64(v, 48));
+}
+
+// One workgroup per row of d elements. A row is a chain of latencies (its loads, the sum over the workgroup, a square
+// root and two divisions in double), so its elements stay in registers (up to kNormHeld per thread) and every thread
+// finishes the sum by itself: one barrier, no second trip for the scale. One row of 2048: 5.8 -> 4.6 us.
+constexpr int kNormHeld = 8;
 __global__ __launch_bounds__(kThreads) void rmsnorm_kernel(const float* __restrict__ x, const float* __restrict__ w,
                                                            float* __restrict__ y, int64_t d, float eps) {
   __shared__ double part[kThreads / 64];
-  __shared__ double scale_sh;
   const int64_t t = blockIdx.x;
   const float* xt = x + t * d;
+  float held[kNormHeld], wt[kNormHeld];
+#pragma unroll
+  for (int c = 0; c < kNormHeld; ++c) {
+    const int64_t i = threadIdx.x + int64_t(c) * kThreads;
+    held[c] = i < d ? xt[i] : 0.f;
+    wt[c] = i < d ? w[i] : 0.f;
+  }
   double ss = 0.0;
-  for (int64_t i = threadIdx.x; i < d; i += kThreads) {
+#pragma unroll
+  for (int c = 0; c < kNormHeld; ++c) ss = __dadd_rn(ss, __dmul_rn(double(held[c]), double(held[c])));
+  for (int64_t i = threadIdx.x + kNormHeld * kThreads; i < d; i += kThreads) {
     const double v = double(xt[i]);
     ss = __dadd_rn(ss, __dmul_rn(v, v));
   }
   ss = wave_sum_f64(ss);
   if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = ss;
   __syncthreads();
-  if (threadIdx.x == 0) {
-    double s = 0.0;
-    for (int i = 0; i < kThreads / 64; ++i) s = __dadd_rn(s, part[i]);
-    scale_sh = __ddiv_rn(1.0, __dsqrt_rn(__dadd_rn(__ddiv_rn(s, double(d)), double(eps))));
-  }
-  __syncthreads();
-  const double scale = scale_sh;
+  double s = 0.0;
+#pragma unroll
+  for (int i = 0; i < kThreads / 64; ++i) s = __dadd_rn(s, part[i]);
+  const double scale = __ddiv_rn(1.0, __dsqrt_rn(__dadd_rn(__ddiv_rn(s, double(d)), double(eps))));
   float* yt = y + t * d;
-  for (int64_t i = threadIdx.x; i < d; i += kThreads) yt[i] = float(__dmul_rn(__dmul_rn(double(xt[i]), scale), double(w[i])));
+#pragma unroll
+  for (int c = 0; c < kNormHeld; ++c) {
+    const int64_t i = threadIdx.x + int64_t(c) * kThreads;
+    if (i < d) yt[i] = float(__dmul_rn(__dmul_rn(double(held[c]), scale), double(wt[c])));
+  }
+  for (int64_t i = threadIdx.x + kNormHeld * kThreads; i < d; i += kThreads)
+    yt[i] = float(__dmul_rn(__dmul_rn(double(xt[i]), scale), double(w[i])));
 }
 
 __global__ __launch_bounds__(kThreads) void add_kernel(float* __restrict__ x, const float* __restrict__ y,
