@@ -29,24 +29,6 @@ __global__ __launch_bounds__(kDecodeThreads) void attn_decode_partial(
                         blockIdx.z);
 }
 
-// Short windows in one launch: a 16-wave workgroup per (query row, query head) takes the whole window, so there is
-// nothing to combine. A decode step of a short context is bound by its launches (2-3 us each on the host, and the
-// combine waits for the partials), not by bytes: the query heads of a KV head reading its rows each from L2 costs less
-// than the second launch. Four row slots per lane and tensor in flight (two for head_dim 128), 512 rows of head_dim 64 a
-// round trip. 14 query heads of 64 over 400 fp32 rows, with the append: 12.0 -> 7.1 us a call (the kernel about as long
-// as the partials it replaces, the combine's 4 us gone); 32 of 128 over 200 rows 11.9 -> 8.3.
-constexpr int kShortWaves = 16;
-constexpr int short_slots(int hd) { return hd == 64 ? 4 : 2; }
-template <int HD, typename KV>
-__global__ __launch_bounds__(64 * kShortWaves) void attn_decode_short(
-    const float* __restrict__ q, const KV* __restrict__ k, const KV* __restrict__ v, float* __restrict__ out, int64_t pos0,
-    int n_heads, int n_kv, int group, int64_t groups, float qscale, const float2* __restrict__ q_rope, int q_rope_neox,
-    const float* __restrict__ k_new, const float* __restrict__ v_new, KV* __restrict__ k_dst, KV* __restrict__ v_dst) {
-  partial_block<HD, 1, KV, kShortWaves, short_slots(HD)>(q, k, v, out, nullptr, nullptr, pos0, n_heads, n_kv, group,
-                                                         group, 1, groups, 0, qscale, q_rope, q_rope_neox, k_new, v_new,
-                                                         k_dst, v_dst, 0, blockIdx.x, blockIdx.y);
-}
-
 // One workgroup per (row, head): rh = t * n_heads + head.
 template <int HD>
 __global__ __launch_bounds__(kDecodeThreads) void attn_decode_combine(const float* __restrict__ ws_o,
@@ -331,27 +313,6 @@ int launch_rows(const float* q, const KVT* k, const KVT* v, float* out, int64_t 
                              s, ws_o, ws_ml, out, int(G));
 }
 
-// Calls the single-launch kernel takes: at most one workgroup per CU, windows of at most 512 rows of head_dim 64 or 256
-// of 128. A workgroup reads about 45 bytes a ns, so its time grows with the window where the split kernels' hardly
-// does: 512 fp32 rows of 64 take 10.0 us with 32 query heads against 11.5, 513 (a second round trip) 13.3 against 11.1;
-// 256 rows of 128 9.2 against 11.4, 321 11.4 against 11.3, 513 15.9 against 11.1 (fp16 rows 8.3 against 11.7, 8.7
-// against 11.7, 12.5 against 11.8). Two workgroups per CU - 16 rows of 32 heads - take 14.8 us against 14.3, one - 8
-// rows - 11.3 against 14.4.
-constexpr int64_t kShortElems = 32768;  // of a head's K rows
-inline bool short_route(int64_t n, int64_t pos0, int64_t n_heads, int64_t hd, int cu_count) {
-  return pos0 <= kShortElems && (pos0 + n) * hd <= kShortElems && n * n_heads <= cu_count;
-}
-
-template <int HD, typename KVT>
-int launch_short(const float* q, const KVT* k, const KVT* v, float* out, int64_t n, int64_t pos0, int64_t H, int64_t KV,
-                 float qscale, const float2* q_rope, int q_rope_neox, const Append<KVT>& app, hipStream_t s) {
-  constexpr int64_t step = 64 / (HD / 8) * short_slots(HD) * kShortWaves;  // rows of an iteration
-  return nbhs_timing::launch(NBHS_K_DECODE_PARTIAL, attn_decode_short<HD, KVT>, dim3(unsigned(H), unsigned(n)),
-                             dim3(64 * kShortWaves), s, q, k, v, out, pos0, int(H), int(KV), int(H / KV),
-                             (pos0 + n + step - 1) / step, qscale, q_rope, q_rope_neox, app.k_new, app.v_new, app.k_dst,
-                             app.v_dst);
-}
-
 // allow_rows: single-row calls of the whole-row shapes take attn_decode_rows (off: the per-head split kernel, for
 // callers whose workspace is sized for it alone).
 template <typename KVT>
@@ -374,19 +335,10 @@ int decode(const float* q, const KVT* k, const KVT* v, float* out, int64_t n, in
                                  k, v, out, pos0, int(n_heads), int(n_kv_heads), int(head_dim), qscale);
     }
   }
-  const bool short_call = !single_chunk && short_route(n, pos0, n_heads, head_dim, cu_count);
-  auto run_short = [&] {
-    if (head_dim == 64)
-      return launch_short<64>(q, k, v, out, n, pos0, n_heads, n_kv_heads, qscale, q_rope, q_rope_neox, app, s);
-    return launch_short<128>(q, k, v, out, n, pos0, n_heads, n_kv_heads, qscale, q_rope, q_rope_neox, app, s);
-  };
-  // (a short call's workspace is still checked against the split kernels' need, so whether a call is refused does not
-  // depend on which kernel its window takes)
   if (allow_rows && !single_chunk && rows_route(n, n_heads, n_kv_heads, head_dim) && pos0 < kRowsMaxPos) {
     const int64_t G = rows_grid<KVT>(pos0, n_kv_heads, head_dim, cu_count);
     const int64_t need = G == 1 ? 0 : n_heads * G * (head_dim + 2);
     if (need > 0 && (!workspace || workspace_floats < need)) return NBHS_EINVAL;
-    if (short_call) return run_short();
     if (head_dim == 64)
       return launch_rows<64>(q, k, v, out, pos0, n_heads, n_kv_heads, workspace, G, qscale, q_rope, q_rope_neox, app,
                              s);
@@ -398,7 +350,6 @@ int decode(const float* q, const KVT* k, const KVT* v, float* out, int64_t n, in
   const int64_t need = p.n_chunks == 1 ? 0 : n * n_heads * p.n_chunks * (head_dim + 2);
   if (need > 0 && (!workspace || workspace_floats < need)) return NBHS_EINVAL;
   if (n_kv_heads * p.n_sub > 65535) return NBHS_EINVAL;
-  if (short_call) return run_short();
   if (head_dim == 64)
     return launch_decode<64>(q, k, v, out, n, pos0, n_heads, n_kv_heads, workspace, p, qscale, q_rope, q_rope_neox,
                              app, s);

@@ -159,9 +159,8 @@ __device__ __forceinline__ void merge(State<VPL>& a, float bm, float bl, const f
 
 // One workgroup of the split-context kernel: chunk `chunk` of query row t for KV head x head subgroup `by`
 // (by / n_sub, by % n_sub). HD: head_dim (64 or 128). GB: query heads per workgroup (the GQA group, or a slice of
-// it). KV: the cache element type (float, or _Float16 for an fp16 cache). Needs 64 NW threads; KU row slots per lane and
-// tensor in flight.
-template <int HD, int GB, typename KV = float, int NW = kDecodeThreads / 64, int KU = unroll_for(int(sizeof(KV)))>
+// it). KV: the cache element type (float, or _Float16 for an fp16 cache). Needs kDecodeThreads threads.
+template <int HD, int GB, typename KV = float>
 __device__ __forceinline__ void partial_block(
     const float* __restrict__ q, const KV* __restrict__ k, const KV* __restrict__ v, float* __restrict__ out,
     float* __restrict__ ws_o, float* __restrict__ ws_ml, int64_t pos0, int n_heads, int n_kv, int group, int n_sub,
@@ -171,7 +170,9 @@ __device__ __forceinline__ void partial_block(
   constexpr int VPL = 2;                            // float4 per lane per row
   constexpr int LPR = HD / (4 * VPL);               // lanes per K/V row: 8 (hd 64) or 16 (hd 128)
   constexpr int RPS = 64 / LPR;                     // rows per wave load
+  constexpr int KU = unroll_for(int(sizeof(KV)));   // row slots per lane per iteration
   constexpr int WAVE_ROWS = RPS * KU;               // rows per wave iteration
+  constexpr int NW = kDecodeThreads / 64;           // waves per workgroup
   constexpr int64_t kStep = NW * WAVE_ROWS;         // rows the workgroup covers per iteration
   __shared__ float sm_m[NW][GB], sm_l[NW][GB];
   __shared__ f32x4 sm_o[NW][GB][LPR * VPL];
@@ -405,30 +406,15 @@ __device__ __forceinline__ void partial_block(
   }
   __syncthreads();
   constexpr int V4 = HD / 4;  // float4 columns of a head row
-  for (int idx = threadIdx.x; idx < GB * V4; idx += 64 * NW) {
+  for (int idx = threadIdx.x; idx < GB * V4; idx += kDecodeThreads) {
     const int h = idx / V4, c4 = idx % V4;
     if (h >= gcount) continue;
     State<1> acc;
-    if constexpr (NW <= 4) {
-      acc.m = sm_m[0][h];
-      acc.l = sm_l[0][h];
-      acc.o[0] = sm_o[0][h][c4];
+    acc.m = sm_m[0][h];
+    acc.l = sm_l[0][h];
+    acc.o[0] = sm_o[0][h][c4];
 #pragma unroll
-      for (int w = 1; w < NW; ++w) merge<1>(acc, sm_m[w][h], sm_l[w][h], &sm_o[w][h][c4]);
-    } else {  // many waves: their common max first, then independent weights, not a chain of merges
-      acc.m = -INFINITY;
-#pragma unroll
-      for (int w = 0; w < NW; ++w) acc.m = fmaxf(acc.m, sm_m[w][h]);
-      const float ms = acc.m == -INFINITY ? 0.0f : acc.m;
-      acc.l = 0.f;
-      acc.o[0] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int w = 0; w < NW; ++w) {
-        const float e = exp2_raw(sm_m[w][h] - ms);
-        acc.l += sm_l[w][h] * e;
-        acc.o[0] += sm_o[w][h][c4] * e;
-      }
-    }
+    for (int w = 1; w < NW; ++w) merge<1>(acc, sm_m[w][h], sm_l[w][h], &sm_o[w][h][c4]);
     const int64_t head = h0 + h;
     if (n_chunks == 1) {
       reinterpret_cast<f32x4*>(out + (t * n_heads + head) * HD)[c4] = acc.o[0] * (1.0f / acc.l);
