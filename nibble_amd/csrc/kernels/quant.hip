@@ -923,7 +923,8 @@ struct QGemmBatch {  // weights of one type sharing one input; tile0[i]: first r
 
 typedef int i32x4_t __attribute__((ext_vector_type(4)));  // an integer MFMA result
 
-template <int T, int TJ, int WRT = 64>
+// UB: blocks whose LDS reads and MFMAs a wave has in flight.
+template <int T, int TJ, int WRT = 64, int UB = 1>
 __global__ __launch_bounds__(256) void qgemm_legacy_kernel(QGemmBatch B, QA A, int64_t n) {
   int wi = 0;
   for (int i = 1; i < B.n_w; ++i)
@@ -1069,7 +1070,7 @@ __global__ __launch_bounds__(256) void qgemm_legacy_kernel(QGemmBatch B, QA A, i
     __syncthreads();
     // the next chunk's share, in flight while this one is computed (the last chunk loads itself again, unused)
     load_share(c0 + kGemmCB < W.nb ? c0 + kGemmCB : c0, cur);
-    for (int b = 0; b < nc; ++b) {
+    auto block = [&](int b) __attribute__((always_inline)) {
       long bop[WN];
 #pragma unroll
       for (int j = 0; j < WN; ++j) {
@@ -1106,7 +1107,14 @@ __global__ __launch_bounds__(256) void qgemm_legacy_kernel(QGemmBatch B, QA A, i
           }
         }
       }
-    }
+    };
+    int b = 0;
+    if constexpr (UB > 1)
+      for (; b + UB <= nc; b += UB) {
+#pragma unroll
+        for (int u = 0; u < UB; ++u) block(b + u);
+      }
+    for (; b < nc; ++b) block(b);
     __syncthreads();
   }
 #pragma unroll
@@ -1122,7 +1130,12 @@ __global__ __launch_bounds__(256) void qgemm_legacy_kernel(QGemmBatch B, QA A, i
 
 // The legacy kernel's tile for a launch: 64 x 64 while 64 x 64 tiles give at least kLegacyMinWgs workgroups
 // (two per CU); else 64 x 32 while those do; else 32 x 32 (more, smaller workgroups: at the QKV shape 16-80 rows
-// run 10-20 % faster than with 64 x 32, and 512 rows 3-5 % slower).
+// run 10-20 % faster than with 64 x 32, and 512 rows 3-5 % slower). A wave of
+// a 32 x 32 tile has one MFMA per block, a chain of LDS read, MFMA and float term; up to kLegacyUnrollWgs workgroups
+// leave a SIMD about two such waves, so four blocks go in flight (Q8_0: the QKV shape at 40 rows, 192 workgroups, 15.0 ->
+// 13.0 us, at 150, 480, 17.1 -> 16.5; feed-forward blocks of 77 rows 896 -> 3584 -> 896 wide 42.6 -> 38.7, 2048 -> 8192
+// -> 2048 86.7 -> 77.4). With more workgroups the registers cost waves: at 300 rows, 960, 23.8 -> 24.6.
+constexpr int64_t kLegacyUnrollWgs = 512;
 constexpr int64_t kLegacyMinWgs = 512;
 enum LegacyTile { kTile64x64, kTile64x32, kTile32x32 };
 template <int T>
@@ -1134,6 +1147,8 @@ hipError_t launch_legacy(LegacyTile tile, unsigned tiles, int64_t n, hipStream_t
   const dim3 grid{tiles, unsigned((n + 31) / 32)};
   if (tile == kTile64x32)
     return nbhs_timing::launch(NBHS_K_QGEMM, qgemm_legacy_kernel<T, 2>, grid, dim3(256), s, B, A, n);
+  if (int64_t(grid.x) * grid.y <= kLegacyUnrollWgs)
+    return nbhs_timing::launch(NBHS_K_QGEMM, qgemm_legacy_kernel<T, 2, 32, 4>, grid, dim3(256), s, B, A, n);
   return nbhs_timing::launch(NBHS_K_QGEMM, qgemm_legacy_kernel<T, 2, 32>, grid, dim3(256), s, B, A, n);
 }
 

@@ -332,3 +332,21 @@ def test_quant_k_few_rows_every_width(backend, t, n):
         diff = int(np.sum(bits(got) != bits(ref)))
         assert diff == 0, (U.NAMES[t], nb, rows, n, diff)
         backend.release_weights()
+
+
+@pytest.mark.parametrize("nb", [1, 3, 4, 5, 7, 8, 9, 12, 15, 21])
+@pytest.mark.parametrize("t", [oracle.Q4_0, oracle.Q5_0, oracle.Q5_1, oracle.Q8_0], ids=lambda t: U.NAMES[t])
+def test_quant_tiled_legacy_block_counts(backend, t, nb):
+    """The 32 x 32 tile of the 32-element types over every remainder of its chunk of eight blocks and of the four its
+    small launches run at once, rows and activation rows that end inside a tile: every output bit-exact."""
+    in_ = 32 * nb
+    for rows, n in ((130, 17), (33, 70), (5473, 90)):  # the last with more workgroups than run four blocks at once
+        w = U.random_qmat(t, rows, in_, seed=70 + t + nb)
+        x = (np.random.default_rng(nb).standard_normal((n, in_)) * 2).astype(np.float32)
+        with Buffers(backend) as B:
+            dx, dy = B.upload(x), B.alloc(n * rows)
+            backend.matmul(w, dx, dy, n)
+            got = backend.download(dy, (n, rows))
+        ref = oracle.matmul_q(t, w.raw, in_, rows, x)
+        assert np.array_equal(bits(got), bits(ref)), (U.NAMES[t], rows, n, nb)
+        backend.release_weights()
