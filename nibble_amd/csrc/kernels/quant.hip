@@ -20,7 +20,8 @@
 // a legacy block or a whole K super-block each - and write each pair's float term(s) to LDS; then one lane per
 // (row, activation row) adds its terms in block order. K quants are stored in residue order (quant_layout.h), so a
 // sub-block's eight integer lanes are eight v_dot4. With up to 4 activation rows the rows are quantized inside the
-// launch (into LDS, once per wave and block), with the same bits as the standalone quantizer.
+// launch (into LDS, once per wave and block), with the same bits as the standalone quantizer. K types at up to 4 rows
+// take kgemv_kernel instead (a workgroup quantizes the rows once), longer calls of either kind the tiled kernels.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
