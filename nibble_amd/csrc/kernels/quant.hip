@@ -70,6 +70,15 @@ typedef float floatx4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 
+// Orders a wave's LDS operations across its lanes: the writes of every lane before it are seen by the reads of every lane
+// after it, and none of them moves across it. The LDS unit completes one wave's operations in order, so wavefront-scope
+// fences keep the compiler to that order and cost no wait; the barrier alone orders no memory access.
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Lane exchanges on the VALU (DPP), a few cycles each where a __shfl goes through LDS: within quads, and mirrored within
 // 8 and 16 lanes. In this order they are the steps of a reduction over 16 lanes.
 template <int CTRL>
@@ -867,8 +876,8 @@ __global__ __launch_bounds__(256) void kgemv_kernel(QBatch B, const float* __res
             if (c == 0 && ur < rp && br < rb) terms[wave][br][CH - 1][us] = __fmul_rn(__fmul_rn(h2f(K.m), da), float(sumi));
           }
         }
-        // the wave's terms of this chunk, in super-block order (LDS operations of one wave complete in order)
-        __builtin_amdgcn_wave_barrier();
+        // the wave's terms of this chunk, in super-block order
+        wave_lds_sync();
         const float* tp = &terms[wave][cr][cl][0];
         const float* mp = &terms[wave][cr][CH - 1][0];
         float tv[kGemvChunk], mv[kGemvChunk];
@@ -884,7 +893,7 @@ __global__ __launch_bounds__(256) void kgemv_kernel(QBatch B, const float* __res
             if constexpr (T != kQ6_K) acc[t] = __fsub_rn(acc[t], mv[i]);
           }
         }
-        __builtin_amdgcn_wave_barrier();
+        wave_lds_sync();
       }
     }
 #pragma unroll
