@@ -249,11 +249,10 @@ def test_f16_gemm_nonfinite_activations(backend):
 
 
 def test_f16_gemm_wide_tiles(backend):
-    """A weight with many output tiles takes the 128 x 128 tile configuration (32-deep K slices): 300 rows (a partial
-    last row tile), weights of 11000 rows (partial last weight tiles), in = 200 (a partial last slice), within the
-    summation bound. The configuration follows from each weight's own shape, so a call mixing two such weights and a
-    500-row one (64 x 64 tiles; the two configurations in two launches) equals separate calls bit for bit
-    (backend.h:57)."""
+    """A launch with many output tiles takes 64 x 128 ones: three weights at 300 rows (a partial last row tile), two of
+    11000 rows (partial last weight tiles) and one of 500, in = 200 (a partial last slice), every output within the
+    summation bound. The tiles follow from the launch and an output's sum does not depend on them, so the call equals
+    separate calls bit for bit (backend.h:57), that of the 500-row weight in 64 x 64 tiles."""
     rng = np.random.default_rng(23)
     n, in_ = 300, 200
     ws = [rand(rng, (r, in_), np.float16, 0.3) for r in (11000, 500, 11000)]
@@ -353,8 +352,8 @@ def test_f16_gemm_few_rows_k_ranges(backend, n):
 
 
 @pytest.mark.parametrize("in_", [64, 200, 1096], ids=["one-slice", "short", "many-slices"])
-def test_f16_gemm_wide_tiles(backend, in_):
-    """A launch with enough 64 x 128 tiles to take them (12300 + 130 weight rows, 250 activation rows: 98 x 4), both
+def test_f16_gemm_tile_choice_keeps_bits(backend, in_):
+    """A launch with enough 64 x 128 tiles to take them (12300 + 130 weight rows, 250 activation rows: 99 x 4), both
     row counts ending inside a tile and K inside a slice, and the same weights in calls of their own: the small one then
     takes 64 x 64 tiles, with the same bits."""
     rng = np.random.default_rng(in_)

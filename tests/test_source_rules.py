@@ -1,4 +1,5 @@
 """Rules that the sources keep, checked on their text (CPU)."""
+import ast
 import glob
 import os
 import re
@@ -21,3 +22,15 @@ def test_wave_barriers_carry_fences():
         found += len(fenced)
         assert text.count("__builtin_amdgcn_wave_barrier") == len(fenced), os.path.relpath(path, ROOT)
     assert found
+
+
+def test_every_test_is_collected():
+    """A module's second definition of a name replaces the first, which pytest then never sees."""
+    for path in glob.glob(os.path.join(ROOT, "tests", "*.py")):
+        with open(path) as f:
+            tree = ast.parse(f.read())
+        scopes = [tree] + [n for n in tree.body if isinstance(n, ast.ClassDef)]
+        for scope in scopes:
+            names = [n.name for n in scope.body if isinstance(n, (ast.FunctionDef, ast.ClassDef))]
+            twice = sorted({n for n in names if names.count(n) > 1})
+            assert not twice, (os.path.basename(path), twice)
