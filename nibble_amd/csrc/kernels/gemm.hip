@@ -153,18 +153,20 @@ __global__ __launch_bounds__(kSplitThreads) void split_acts_kernel(const float* 
 }
 
 // Tile configuration: BM activation rows x BN weight rows per tile (each of the four waves takes BM/2 x BN/2),
-// BK-deep K slices, a STAGES-deep LDS ring. Two instances, chosen per launch: 64 x 128 tiles with a 2-stage ring when the
-// launch has at least kWideMinTiles of them (each activation byte fetched from L2 serves twice the products: 16384
-// weight rows x 512, K = 2048: 105 -> 81 us, x 200: 48 -> 39), 64 x 64 tiles with a 3-stage ring otherwise (more
-// workgroups: QKV, 3072 x 512, 22.5 us against 25.4 with 192 tiles of 64 x 128). Both accumulate an output's products
-// in the same order, so its bits do not depend on the choice. 64-72 KB of LDS: two workgroups per CU, one of which
-// multiplies while the other waits; 128 x 128 tiles with 32-deep slices measured 84 us at 16384 x 512. Tiles whose four
-// waves split K and not the outputs (half the LDS reads; one workgroup per CU with a ring of 4-6 slices, the waves'
-// sums added at the end) were no faster: QKV 22.7, 16384 x 512 96 us - what the deeper ring gains goes to each
-// workgroup's fixed part, which nothing overlaps.
+// BK-deep K slices, a STAGES-deep LDS ring. The instance is chosen per launch; each accumulates an output's products in the
+// same order, so its bits do not depend on the choice. 64-72 KB of LDS: two workgroups per CU, one of which multiplies
+// while the other waits.
+//  * 64 x 64 tiles with a 3-stage ring while all of them run at once, two to a CU.
+//  * 64 x 128 tiles with a 2-stage ring from kWideMinTiles tiles of 64 x 64 on: each activation byte fetched from L2 serves
+//    twice the products, and no few workgroups are left for a second round. About the line, 64 x 64 against 64 x 128: 4096
+//    weight rows x 448, K = 4096, 448 tiles, 51.5 us a call against 54.2; 5120 x 448, K = 2048, 560 tiles, 41.6 against
+//    36.3; 3072 x 704, K = 8192, 528 tiles, 141 against 116; 2048 x 1152, K = 8192, 576 tiles, 148 against 125.
+// Tiles whose four waves split K and not the outputs (half the LDS reads; one workgroup per CU with a ring of 4-6 slices,
+// the waves' sums added at the end) were no faster: QKV 22.7 us, 16384 x 512 96 us - what the deeper ring gains goes to
+// each workgroup's fixed part, which nothing overlaps.
 constexpr int kBM = 64, kBK = 64, kSmallBN = 64, kSmallStages = 3, kWideBN = 128, kWideStages = 2;
 constexpr int kPadK = 64;  // K padding of the split activation rows (a multiple of the slice depth)
-constexpr int64_t kWideMinTiles = 384;
+constexpr int64_t kWideMinTiles = 513;
 // K ranges of a weight whose 64 x 64 tiles are too few to fill the CUs and each walk the whole K: up to kMaxSplit
 // ranges, doubling while the weight's tiles times its ranges stay within kSplitWgs, of at least kFewMinSlices slices in
 // calls of up to kFewMaxRows activation rows (QKV shape, K = 2048, 3072 weight rows: 12-64 rows 27-29 -> 15-19 us per
@@ -339,7 +341,7 @@ __global__ __launch_bounds__(kThreads) void gemm_f16w_kernel(GemmBatch b, const 
   // acc[i][j][r] holds activation row 8 (r / 4) + 4 hf + r % 4 of the wave's block i and weight row lane % 32 of
   // its block j. A K range's partial sums go unscaled to its slice of part. The two cases are stored by code of their
   // own: with the scales loaded on one path to a common store, every store waits for all memory operations before it,
-  // the previous store among them (QKV x 64 in 4 and 8 K ranges: the kernel 12.2 us so, 10.0 apart).
+  // the previous store among them (QKV x 64, K = 2048: 18.1 us a call so, 16.6 apart).
   const int tr = wm * (BM / 2) + 4 * hf;  // of the tile: the lane's row at r = 0
   auto row_of = [&](int i, int r) { return tr + 32 * i + 8 * (r / 4) + (r % 4); };
   auto store = [&](float* dst, auto value) __attribute__((always_inline)) {
@@ -443,7 +445,7 @@ int nbhs_gemm_f16w_multi(int n_w, const void* const* w, float* const* y, const i
       }
       return x0;
     };
-    const bool wide = tiles(kWideBN, false) * mt >= kWideMinTiles;
+    const bool wide = tiles(kSmallBN, false) * mt >= kWideMinTiles;
     const int64_t xt = tiles(wide ? kWideBN : kSmallBN, true);
     if (xt > INT32_MAX) {
       e = hipErrorInvalidValue;
