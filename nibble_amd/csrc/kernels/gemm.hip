@@ -12,8 +12,8 @@
 //
 //  * split_acts_kernel: one workgroup per activation row: the row's largest magnitude, then hi and lo written as fp16
 //    rows padded with zeros to a multiple of the K slice (16-byte stores), and 1 / s_t.
-//  * gemm_f16w_kernel: output tiles of 64 x 64 or, for grids with many tiles, 64 x 128, four waves each on a quarter,
-//    64-deep K slices through an LDS ring filled by direct-to-LDS buffer loads (rows past the activation count or a
+//  * gemm_f16w_kernel: output tiles of 64 x 64 or, for grids with many tiles, 64 x 128 or 128 x 128, four waves each on a
+//    quarter, K slices through an LDS ring filled by direct-to-LDS buffer loads (rows past the activation count or a
 //    weight's row count, and columns past `in`, read as zeros). Per 16-deep step a wave reads its hi, lo and weight
 //    fragments once and issues the lo then the hi MFMA into each accumulator. Up to kMaxWeights weights sharing x run
 //    in one launch over their stacked tiles.
@@ -161,12 +161,20 @@ __global__ __launch_bounds__(kSplitThreads) void split_acts_kernel(const float* 
 //    twice the products, and no few workgroups are left for a second round. About the line, 64 x 64 against 64 x 128: 4096
 //    weight rows x 448, K = 4096, 448 tiles, 51.5 us a call against 54.2; 5120 x 448, K = 2048, 560 tiles, 41.6 against
 //    36.3; 3072 x 704, K = 8192, 528 tiles, 141 against 116; 2048 x 1152, K = 8192, 576 tiles, 148 against 125.
+//  * 128 x 128 tiles of 32-deep slices with a 3-stage ring where a row of tiles is so long that its workgroups share few
+//    weight tiles among themselves and every row of tiles reads the weights again: half as many rows of tiles then, from
+//    kHugeMinCols tiles of 128 weight rows and kHugeMinTiles tiles on, if they do not add an empty half row of tiles
+//    (an odd number of 64-row ones), and from kHugeAllCols on always. 64 x 128 against 128 x 128: 110000 weight rows x 128,
+//    K = 2048, 228 us a call against 174; 57344 x 512, K = 8192, 1395 against 1203; 32768 x 512, K = 2048, 169 against 165;
+//    x 448, an odd number, 149 against 157; 20480 x 640, K = 1024, 800 tiles, 73.9 against 75.8, x 768, 960 tiles, 83.2
+//    against 82.2; 16384 x 2048, K = 2048, 312 against 316.
 // Tiles whose four waves split K and not the outputs (half the LDS reads; one workgroup per CU with a ring of 4-6 slices,
 // the waves' sums added at the end) were no faster: QKV 22.7 us, 16384 x 512 96 us - what the deeper ring gains goes to
 // each workgroup's fixed part, which nothing overlaps.
 constexpr int kBM = 64, kBK = 64, kSmallBN = 64, kSmallStages = 3, kWideBN = 128, kWideStages = 2;
 constexpr int kPadK = 64;  // K padding of the split activation rows (a multiple of the slice depth)
-constexpr int64_t kWideMinTiles = 513;
+constexpr int kHugeBM = 128, kHugeBK = 32, kHugeStages = 3;
+constexpr int64_t kWideMinTiles = 513, kHugeMinCols = 160, kHugeMinTiles = 960, kHugeAllCols = 512;
 // K ranges of a weight whose 64 x 64 tiles are too few to fill the CUs and each walk the whole K: up to kMaxSplit
 // ranges, doubling while the weight's tiles times its ranges stay within kSplitWgs, of at least kFewMinSlices slices in
 // calls of up to kFewMaxRows activation rows (QKV shape, K = 2048, 3072 weight rows: 12-64 rows 27-29 -> 15-19 us per
@@ -235,7 +243,8 @@ __global__ __launch_bounds__(kThreads) void gemm_f16w_kernel(GemmBatch b, const 
     woff[i] = uint32_t((r * int(in) + 8 * x) * 2);
   }
   const int wave_u = __builtin_amdgcn_readfirstlane(wave);
-  const int nk_all = int(in_pad / BK), per = (nk_all + d.split - 1) / d.split;
+  // (K ranges in whole kPadK-deep slices, the same ones in every instance)
+  const int nk_all = int(in_pad / BK), per = (int(in_pad / kPadK) + d.split - 1) / d.split * (kPadK / BK);
   const int kb = ks * per;  // this range's first K tile
   auto fetch = [&](int kt, int st) {
     const uint32_t k0 = uint32_t(kb + kt) * BK;
@@ -445,17 +454,22 @@ int nbhs_gemm_f16w_multi(int n_w, const void* const* w, float* const* y, const i
       }
       return x0;
     };
-    const bool wide = tiles(kSmallBN, false) * mt >= kWideMinTiles;
+    const int64_t xt128 = tiles(kWideBN, false), mt128 = (n + kHugeBM - 1) / kHugeBM;
+    const bool huge = n > kBM && (xt128 >= kHugeAllCols ||
+                                  (xt128 >= kHugeMinCols && mt % 2 == 0 && xt128 * mt128 >= kHugeMinTiles));
+    const bool wide = huge || tiles(kSmallBN, false) * mt >= kWideMinTiles;
     const int64_t xt = tiles(wide ? kWideBN : kSmallBN, true);
     if (xt > INT32_MAX) {
       e = hipErrorInvalidValue;
       return;
     }
-    const dim3 grid{unsigned(xt), unsigned(mt)};
-    e = wide ? nbhs_timing::launch(NBHS_K_GEMM, gemm_f16w_kernel<kBM, kWideBN, kBK, kWideStages>, grid, dim3(kThreads), s,
-                                   g, xh, xl, inv, n, in, in_pad)
-             : nbhs_timing::launch(NBHS_K_GEMM, gemm_f16w_kernel<kBM, kSmallBN, kBK, kSmallStages>, grid,
-                                   dim3(kThreads), s, g, xh, xl, inv, n, in, in_pad);
+    auto launch = [&](auto kernel, int64_t row_tiles) {
+      return nbhs_timing::launch(NBHS_K_GEMM, kernel, dim3(unsigned(xt), unsigned(row_tiles)), dim3(kThreads), s, g, xh, xl,
+                                 inv, n, in, in_pad);
+    };
+    e = huge   ? launch(gemm_f16w_kernel<kHugeBM, kWideBN, kHugeBK, kHugeStages>, mt128)
+        : wide ? launch(gemm_f16w_kernel<kBM, kWideBN, kBK, kWideStages>, mt)
+               : launch(gemm_f16w_kernel<kBM, kSmallBN, kBK, kSmallStages>, mt);
     if (e == hipSuccess && split.n_w > 0)
       e = nbhs_timing::launch(NBHS_K_GEMM_REDUCE, gemm_split_reduce_kernel, dim3(unsigned((split_out + 255) / 256)),
                               dim3(256), s, split, inv, n, split_out);

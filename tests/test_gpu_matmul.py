@@ -375,3 +375,30 @@ def test_f16_gemm_tile_choice_keeps_bits(backend, in_):
     for g, w in zip(got, ws):
         assert np.array_equal(bits(gpu_matmul(backend, w, x, n)), bits(g))
     backend.release_weights()
+
+
+@pytest.mark.parametrize("in_,big,n", [(64, 20500, 740), (200, 20500, 740), (4160, 20500, 740), (72, 65500, 130)],
+                         ids=["one-slice", "short", "k-ranges", "odd-rows-of-tiles"])
+def test_f16_gemm_128_row_tiles(backend, in_, big, n):
+    """Launches large enough for 128 x 128 tiles (20500 + 130 weight rows, 740 activation rows: 163 x 6; 65500 + 130, 130
+    rows: 514 x 2), every row count ending inside a tile and K inside a slice: the bits of calls of fewer rows and of the
+    small weight alone, which take other tiles. At in = 4160 the small weight takes 2 K ranges, of 33 and 32 slices in
+    every tile shape."""
+    rng = np.random.default_rng(in_ + 1)
+    ws = [rand(rng, (r, in_), np.float16, in_ ** -0.5) for r in (big, 130)]
+    x = rand(rng, (n, in_))
+    x[3] *= 1e20
+    x[n - 1, 1:] = 0
+    with Buffers(backend) as B:
+        dx = B.upload(x)
+        ys = [B.alloc(n * w.shape[0]) for w in ws]
+        backend.matmul_multi(ws, dx, ys, n)
+        got = [backend.download(y, (n, w.shape[0])) for y, w in zip(ys, ws)]
+    pick = np.r_[0:130, 8000:8100, big - 100:big]  # the reference on a part of the large weight's rows
+    for g, w, rows in zip(got, ws, (pick, np.arange(130))):
+        assert_within_bound(g[:, rows], w[rows], x)
+    assert np.array_equal(bits(gpu_matmul(backend, ws[1], x, n)), bits(got[1]))
+    m = 60 if n == 130 else 300  # (few enough for other tiles; both sides of 128 rows take no K ranges here)
+    for part in (slice(0, m), slice(n - m, n)):
+        assert np.array_equal(bits(gpu_matmul(backend, ws[0], np.ascontiguousarray(x[part]), m)), bits(got[0][part]))
+    backend.release_weights()
