@@ -50,8 +50,8 @@ struct GemmBatch {
 // lanes a ds_read_b128 serves per cycle (16 consecutive rows, one chunk) cover all 64 banks.
 template <int CPR>
 __device__ __forceinline__ int swz(int r) {
-  if constexpr (CPR == 8) return (r ^ (r >> 3)) & 7;
-  return (r >> 2) & 3;
+  static_assert(CPR == 8 || CPR == 4);
+  return CPR == 8 ? (r ^ (r >> 3)) & 7 : (r >> 2) & 3;
 }
 
 constexpr int vmcnt_wait(int n) { return (n & 15) | (7 << 4) | (15 << 8) | ((n >> 4) << 14); }
@@ -180,11 +180,11 @@ constexpr int64_t kWideMinTiles = 513, kHugeMinCols = 160, kHugeMinTiles = 960, 
 // calls of up to kFewMaxRows activation rows (QKV shape, K = 2048, 3072 weight rows: 12-64 rows 27-29 -> 15-19 us per
 // call, 65-128 rows 29-30 -> 19-22) and kMinSlices in longer ones (K = 8192, 2048 weight rows x 140, after a
 // gate + up that is not split: 130 -> 92 us for the block, against 128 x 128 tiles in K ranges). A target of
-// 512 workgroups gained 2-4 us at 192-256 QKV rows but cost gate + up 4-10 us at 32-128 rows. The partial sums live
-// in a fixed area of the workspace (64 MB), which bounds a split weight's outputs.
+// 512 workgroups gained 2-4 us at 192-256 QKV rows but cost gate + up 4-10 us at 32-128 rows. A split weight's partial
+// sums are thus at most kSplitWgs tiles of kBM x kSmallBN; the workspace holds those of kMaxWeights weights (32 MB).
 constexpr int kFewMaxRows = 128, kMaxSplit = 8, kFewMinSlices = 4, kMinSlices = 32;
 constexpr int64_t kSplitWgs = 256;
-constexpr int64_t kSplitPartFloats = int64_t(1) << 24;
+constexpr int64_t kSplitPartFloats = kMaxWeights * kSplitWgs * kBM * kSmallBN;
 
 template <int BM, int BN, int BK, int STAGES>
 __global__ __launch_bounds__(kThreads) void gemm_f16w_kernel(GemmBatch b, const _Float16* __restrict__ xh,
@@ -195,6 +195,7 @@ __global__ __launch_bounds__(kThreads) void gemm_f16w_kernel(GemmBatch b, const 
   constexpr int XT = BM * BK, WT = BN * BK;  // halves per activation-part tile and per weight tile
   constexpr int XLD = BM * CPR / 256;     // loads per wave per activation part (1 KB pieces over 4 waves)
   constexpr int WLD = BN * CPR / 256;     // loads per wave for the weight tile
+  static_assert(STAGES == 2 || STAGES == 3);
   constexpr int MB = BM / 64, NB = BN / 64;  // 32-wide activation-row and weight-row blocks per wave
   __shared__ __attribute__((aligned(16))) _Float16 lds[STAGES][2 * XT + WT];
   int wi = 0;
@@ -298,21 +299,10 @@ __global__ __launch_bounds__(kThreads) void gemm_f16w_kernel(GemmBatch b, const 
   auto step = [&](int kt, auto cur_c) {
     constexpr int cur = decltype(cur_c)::value;
     const int ahead = min(nk - 1 - kt, STAGES - 2);  // tiles after kt already fetched
-    if constexpr (STAGES >= 4) {
-      if (ahead >= 2)
-        __builtin_amdgcn_s_waitcnt(vmcnt_wait(2 * kLoads));
-      else if (ahead == 1)
-        __builtin_amdgcn_s_waitcnt(vmcnt_wait(kLoads));
-      else
-        __builtin_amdgcn_s_waitcnt(vmcnt_wait(0));
-    } else if constexpr (STAGES == 3) {
-      if (ahead >= 1)
-        __builtin_amdgcn_s_waitcnt(vmcnt_wait(kLoads));
-      else
-        __builtin_amdgcn_s_waitcnt(vmcnt_wait(0));
-    } else {
+    if (STAGES == 3 && ahead >= 1)
+      __builtin_amdgcn_s_waitcnt(vmcnt_wait(kLoads));
+    else
       __builtin_amdgcn_s_waitcnt(vmcnt_wait(0));
-    }
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
@@ -339,12 +329,9 @@ __global__ __launch_bounds__(kThreads) void gemm_f16w_kernel(GemmBatch b, const 
   };
   for (int kt = 0; kt < nk; kt += STAGES) {
     step(kt, std::integral_constant<int, 0>{});
-    if constexpr (STAGES > 1)
-      if (kt + 1 < nk) step(kt + 1, std::integral_constant<int, 1>{});
-    if constexpr (STAGES > 2)
+    if (kt + 1 < nk) step(kt + 1, std::integral_constant<int, 1>{});
+    if constexpr (STAGES == 3)
       if (kt + 2 < nk) step(kt + 2, std::integral_constant<int, 2>{});
-    if constexpr (STAGES > 3)
-      if (kt + 3 < nk) step(kt + 3, std::integral_constant<int, 3 % STAGES>{});
   }
 
   // acc[i][j][r] holds activation row 8 (r / 4) + 4 hf + r % 4 of the wave's block i and weight row lane % 32 of
@@ -437,62 +424,50 @@ int nbhs_gemm_f16w_multi(int n_w, const void* const* w, float* const* y, const i
   const hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   const int vec = reinterpret_cast<uintptr_t>(x) % 16 == 0 ? 1 : 0;
   const int64_t mt = (n + kBM - 1) / kBM;
-  hipError_t e = nbhs_timing::launch(NBHS_K_SPLIT_ACTS, split_acts_kernel, dim3(unsigned(n)), dim3(kSplitThreads), s,
-                                     x, in, in_pad, xh, xl, inv, vec);
   // Each weight's K ranges follow from its own shape, so its results do not depend on the other weights of the call
-  // (matmul_multi equals separate calls). The weights share a launch while the split ones' partial sums fit their area,
-  // then the next group starts.
-  GemmBatch g{}, split{};  // the group, and its split weights
+  // (matmul_multi equals separate calls).
+  GemmBatch g{}, split{};  // the weights, and the split ones
   int64_t part_used = 0, split_out = 0;
-  auto flush = [&]() {
-    if (e != hipSuccess || g.n_w == 0) return;
-    auto tiles = [&](int bn, bool set) {
-      int64_t x0 = 0;
-      for (int i = 0; i < g.n_w; ++i) {
-        if (set) g.w[i].tile0 = int(x0);
-        x0 += (g.w[i].rows + bn - 1) / bn * g.w[i].split;
-      }
-      return x0;
-    };
-    const int64_t xt128 = tiles(kWideBN, false), mt128 = (n + kHugeBM - 1) / kHugeBM;
-    const bool huge = n > kBM && (xt128 >= kHugeAllCols ||
-                                  (xt128 >= kHugeMinCols && mt % 2 == 0 && xt128 * mt128 >= kHugeMinTiles));
-    const bool wide = huge || tiles(kSmallBN, false) * mt >= kWideMinTiles;
-    const int64_t xt = tiles(wide ? kWideBN : kSmallBN, true);
-    if (xt > INT32_MAX) {
-      e = hipErrorInvalidValue;
-      return;
-    }
-    auto launch = [&](auto kernel, int64_t row_tiles) {
-      return nbhs_timing::launch(NBHS_K_GEMM, kernel, dim3(unsigned(xt), unsigned(row_tiles)), dim3(kThreads), s, g, xh, xl,
-                                 inv, n, in, in_pad);
-    };
-    e = huge   ? launch(gemm_f16w_kernel<kHugeBM, kWideBN, kHugeBK, kHugeStages>, mt128)
-        : wide ? launch(gemm_f16w_kernel<kBM, kWideBN, kBK, kWideStages>, mt)
-               : launch(gemm_f16w_kernel<kBM, kSmallBN, kBK, kSmallStages>, mt);
-    if (e == hipSuccess && split.n_w > 0)
-      e = nbhs_timing::launch(NBHS_K_GEMM_REDUCE, gemm_split_reduce_kernel, dim3(unsigned((split_out + 255) / 256)),
-                              dim3(256), s, split, inv, n, split_out);
-    g = split = GemmBatch{};
-    part_used = split_out = 0;
-  };
   for (int i = 0; i < n_w; ++i) {
     const int64_t st = (rows[i] + kSmallBN - 1) / kSmallBN * mt, slices = in_pad / kBK;
     const int64_t min_slices = n <= kFewMaxRows ? kFewMinSlices : kMinSlices;
     int sp = 1;
-    if (n * rows[i] * kMaxSplit <= kSplitPartFloats)
-      while (sp < kMaxSplit && st * sp * 2 <= kSplitWgs && slices / (2 * sp) >= min_slices) sp *= 2;
-    const int64_t cnt = sp > 1 ? n * rows[i] * sp : 0;
-    if (part_used + cnt > kSplitPartFloats) flush();
+    while (sp < kMaxSplit && st * sp * 2 <= kSplitWgs && slices / (2 * sp) >= min_slices) sp *= 2;
     g.w[g.n_w++] =
         GemmWeight{static_cast<const _Float16*>(w[i]), y[i], rows[i], 0, sp, sp > 1 ? part + part_used : nullptr};
     if (sp > 1) {
       split.w[split.n_w++] = g.w[g.n_w - 1];
-      part_used += cnt;
+      part_used += n * rows[i] * sp;
       split_out += n * rows[i];
     }
   }
-  flush();
+  // weight-row tiles of the launch (at most kMaxWeights weights of 2^25 64-row tiles, or of kSplitWgs with their ranges)
+  auto tiles = [&](int bn) {
+    int64_t x0 = 0;
+    for (int i = 0; i < n_w; ++i) {
+      g.w[i].tile0 = int(x0);
+      x0 += (rows[i] + bn - 1) / bn * g.w[i].split;
+    }
+    return x0;
+  };
+  const int64_t xt64 = tiles(kSmallBN), xt128 = tiles(kWideBN), mt128 = (n + kHugeBM - 1) / kHugeBM;
+  const bool huge = n > kBM && (xt128 >= kHugeAllCols ||
+                                (xt128 >= kHugeMinCols && mt % 2 == 0 && xt128 * mt128 >= kHugeMinTiles));
+  const bool wide = huge || xt64 * mt >= kWideMinTiles;
+  if (!wide) tiles(kSmallBN);
+  auto launch = [&](auto kernel, int64_t row_tiles) {
+    return nbhs_timing::launch(NBHS_K_GEMM, kernel, dim3(unsigned(wide ? xt128 : xt64), unsigned(row_tiles)), dim3(kThreads),
+                               s, g, xh, xl, inv, n, in, in_pad);
+  };
+  hipError_t e = nbhs_timing::launch(NBHS_K_SPLIT_ACTS, split_acts_kernel, dim3(unsigned(n)), dim3(kSplitThreads), s,
+                                     x, in, in_pad, xh, xl, inv, vec);
+  if (e == hipSuccess)
+    e = huge   ? launch(gemm_f16w_kernel<kHugeBM, kWideBN, kHugeBK, kHugeStages>, mt128)
+        : wide ? launch(gemm_f16w_kernel<kBM, kWideBN, kBK, kWideStages>, mt)
+               : launch(gemm_f16w_kernel<kBM, kSmallBN, kBK, kSmallStages>, mt);
+  if (e == hipSuccess && split.n_w > 0)
+    e = nbhs_timing::launch(NBHS_K_GEMM_REDUCE, gemm_split_reduce_kernel, dim3(unsigned((split_out + 255) / 256)),
+                            dim3(256), s, split, inv, n, split_out);
   return e;
 }
 

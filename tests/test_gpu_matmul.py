@@ -300,11 +300,11 @@ def assert_within_bound(got, w, x, what=""):
 
 
 def test_f16_gemm_split_k(backend):
-    """Weights with few 128 x 128 tiles and a long K take K ranges (partials summed in range order): 700 and 90 rows at
-    n = 300, in = 8200 (4 ranges of 65, 65, 65 and 63 slices; partial activation, weight and K tiles), in one call
-    with a 12000-row weight (128 x 128 tiles, no ranges). Within the summation bound (the split weights also against
-    the restated reference), and matmul_multi equals separate calls bit for bit (each weight's configuration follows
-    from its own shape, backend.h:57)."""
+    """Weights with few 64 x 64 tiles and a long K take K ranges (partials summed in range order): 700 and 90 rows at
+    n = 300, in = 8200 (4 ranges of 33, 33, 33 and 30 slices; partial activation, weight and K tiles), in one call
+    with a 12000-row weight (no ranges). Within the summation bound (the split weights also against the restated
+    reference), and matmul_multi equals separate calls bit for bit (each weight's ranges follow from its own shape,
+    backend.h:57)."""
     rng = np.random.default_rng(29)
     n, in_ = 300, 8200
     ws = [rand(rng, (r, in_), np.float16, 0.3) for r in (700, 90, 12000)]
@@ -319,13 +319,14 @@ def test_f16_gemm_split_k(backend):
     backend.release_weights()
 
 
-def test_f16_gemm_split_k_groups(backend):
-    """Three 9000-row weights at n = 300, in = 4160, each in 2 K ranges: their partial sums (5.4M floats each) exceed
-    the 16M-float partial area together, so the call runs them as two groups (two weights, then one). Within the
-    summation bound, and equal to separate calls bit for bit."""
+@pytest.mark.parametrize("n,in_,rows", [(300, 4160, (1600, 1, 64, 65, 900, 1600, 300, 1600)), (64, 2056, (2048,) * 8)],
+                         ids=["two-ranges", "eight-ranges"])
+def test_f16_gemm_split_k_groups(backend, n, in_, rows):
+    """Eight weights in K ranges in one call: 2 ranges each of 33 and 32 slices, up to the 250 workgroups a weight of 1600
+    rows takes; and 8 ranges each of 5 slices (the seventh of 3, the last empty), 256 workgroups a weight and so the whole
+    partial-sum area. Within the summation bound, and equal to separate calls bit for bit."""
     rng = np.random.default_rng(31)
-    n, in_ = 300, 4160
-    ws = [rand(rng, (9000, in_), np.float16, 0.3) for _ in range(3)]
+    ws = [rand(rng, (r, in_), np.float16, 0.3) for r in rows]
     x = rand(rng, (n, in_))
     got, sep = multi_vs_separate(backend, ws, x, n)
     for i, (g, w) in enumerate(zip(got, ws)):
