@@ -267,12 +267,13 @@ int nbhs_gemm_f16w_multi(int n_w, const void* const* w, float* const* y, const i
 
 /* ---- the other per-token ops (Backend::embed / rmsnorm / add / silu_mul, backend.h:55-70) ---- */
 
+/* out[t, :] = row ids[t] of table [rows, d] (F32, or F16 widened exactly); ids in device memory, already checked
+ * against the row count by the caller (ref_ops.cpp:80-99). */
+int nbhs_embed(int f16, const void* table, const int32_t* ids, int64_t n, int64_t d, float* out, nbhs_stream s);
 /* Host ids that an embedding launch carries as its argument. */
 #define NBHS_EMBED_ARG_IDS 512
-/* out[t, :] = row ids[t] of a float table (F32 copied, F16 widened exactly). The ids are n <= NBHS_EMBED_ARG_IDS host
- * ones, read before the call returns, or (host_ids NULL) device ones. */
-int nbhs_embed(int f16, const void* table, const int32_t* host_ids, const int32_t* ids, int64_t n, int64_t d, float* out,
-               nbhs_stream s);
+/* nbhs_embed with n <= NBHS_EMBED_ARG_IDS ids in host memory, read before the call returns. */
+int nbhs_embed_host_ids(int f16, const void* table, const int32_t* ids, int64_t n, int64_t d, float* out, nbhs_stream s);
 /* ref_ops.cpp:137-148: y[t] = float(x[t] * scale * w) with scale = 1 / sqrt(sum(x^2) / d + eps) in double. */
 int nbhs_rmsnorm_f32(const float* x, const float* w, float* y, int64_t n, int64_t d, float eps, nbhs_stream s);
 /* x[i] += y[i] (ref_ops.cpp:151-153). */
@@ -293,21 +294,28 @@ int nbhs_quantize_acts(int type, const float* x, int64_t n, int64_t in, void* ac
  * rows of x quantized inside the launch (the same bits). */
 int nbhs_qgemv_multi(int type, int n_w, const void* const* w, const int64_t* rows, float* const* y, int64_t in,
                      const float* x, const void* acts, int64_t n_acts, int64_t t0, int64_t n, nbhs_stream s);
-/* Bytes of the n x in activations in the form nbhs_quantize_acts_rm writes, or -1. */
-int64_t nbhs_quant_act_rm_bytes(int type, int64_t n, int64_t in);
-/* nbhs_quantize_acts for the K types in the form nbhs_qgemm_multi reads for them: 16 times each quant as fp16, residue
- * by residue, and the sub-blocks' sums as fp16 digits (kActQ8_K16 of kernels/quant_layout.h). */
-int nbhs_quantize_acts_rm(int type, const float* x, int64_t n, int64_t in, void* acts, nbhs_stream s);
 /* The same products for any n (prefill chunks), tiled, in one launch for up to NBHS_GEMV_MAX_WEIGHTS weights of
- * one type: y[i][t * rows[i] + r] for t < n over all n quantized activation rows in acts; Q4_0, Q5_0, Q5_1, Q8_0
- * (acts from nbhs_quantize_acts) and Q4_K, Q5_K, Q6_K (acts from nbhs_quantize_acts_rm). Same bits
- * as nbhs_qgemv_multi. */
+ * one type: y[i][t * rows[i] + r] for t < n over all n quantized activation rows in acts (from nbhs_quantize_acts); Q4_0,
+ * Q5_0, Q5_1, Q8_0. Same bits as nbhs_qgemv_multi. The K types have entry points of their own: */
 int nbhs_qgemm_multi(int type, int n_w, const void* const* w, const int64_t* rows, float* const* y, int64_t in,
                      const void* acts, int64_t n, nbhs_stream s);
-/* out[t, :] = dequantized row ids[t] of the weight, quant.cpp:157-242 bit for bit. The ids are n <= NBHS_EMBED_ARG_IDS
- * host ones, read before the call returns, or (host_ids NULL) device ones. */
-int nbhs_dequant_rows(int type, const void* w, int64_t rows, int64_t in, const int32_t* host_ids, const int32_t* ids,
-                      int64_t n, float* out, nbhs_stream s);
+/* Bytes of n x in activations in the form that the tiled kernels of Q4_K, Q5_K and Q6_K read, or -1: nearly twice
+ * nbhs_quant_act_bytes, so the two functions below are given the buffer's size and reject a smaller one. */
+int64_t nbhs_quant_act_k16_bytes(int type, int64_t n, int64_t in);
+/* nbhs_quantize_acts in that form: 16 times each quant as fp16, residue by residue, and the sub-blocks' sums as fp16
+ * digits (kActQ8_K16 of kernels/quant_layout.h). */
+int nbhs_quantize_acts_k16(int type, const float* x, int64_t n, int64_t in, void* acts, int64_t acts_bytes, nbhs_stream s);
+/* nbhs_qgemm_multi for Q4_K, Q5_K and Q6_K over acts from nbhs_quantize_acts_k16. */
+int nbhs_qgemm_k16_multi(int type, int n_w, const void* const* w, const int64_t* rows, float* const* y, int64_t in,
+                         const void* acts, int64_t acts_bytes, int64_t n, nbhs_stream s);
+/* Always NBHS_EINVAL: the K types' 8-bit form of nbhs_quant_act_bytes bytes that it wrote is read by no kernel. */
+int nbhs_quantize_acts_rm(int type, const float* x, int64_t n, int64_t in, void* acts, nbhs_stream s);
+/* out[t, :] = dequantized row ids[t] (device ids) of the weight, quant.cpp:157-242 bit for bit. */
+int nbhs_dequant_rows(int type, const void* w, int64_t rows, int64_t in, const int32_t* ids, int64_t n, float* out,
+                      nbhs_stream s);
+/* nbhs_dequant_rows with n <= NBHS_EMBED_ARG_IDS ids in host memory, read before the call returns. */
+int nbhs_dequant_rows_host_ids(int type, const void* w, int64_t rows, int64_t in, const int32_t* ids, int64_t n, float* out,
+                               nbhs_stream s);
 
 /* ---- per-kernel timing (measurement only) ----
  * While enabled for a kernel, its launcher launches it with a HIP event pair (hipExtLaunchKernel) stamped from the

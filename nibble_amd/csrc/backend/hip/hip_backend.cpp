@@ -169,7 +169,7 @@ void HipBackend::reserve(const ReserveParams& rp) {
     for (const int t : {2, 6, 7, 8, 12, 13, 14}) {
       const int64_t be = nbh_quant::block_elems(t), w = rp.max_width / be * be;
       if (w > 0) {
-        const int64_t b = nbh_quant::is_k(t) ? nbhs_quant_act_rm_bytes(t, rp.max_rows, w)  // the larger form
+        const int64_t b = nbh_quant::is_k(t) ? nbhs_quant_act_k16_bytes(t, rp.max_rows, w)  // the larger form
                                              : nbhs_quant_act_bytes(t, rp.max_rows, w);
         if (b < 0) throw Error("reserve: activation scratch for max_rows=" + str(rp.max_rows) + " max_width=" +
                                str(rp.max_width) + " is too large");
@@ -488,14 +488,14 @@ void HipBackend::matmul_multi(std::span<const Tensor* const> ws, const float* x,
     const int64_t min_rows =
         t == nbh_quant::kQ6_K ? kQ6KTiledMinRows : nbh_quant::is_k(t) ? kKTiledMinRows : kGemvMaxRows;
     const bool tiled = n > min_rows;
-    const bool rm = tiled && nbh_quant::is_k(t);
-    const int act_key = 2 * nbh_quant::act_of(t) + (rm ? 1 : 0);
+    const bool k16 = tiled && nbh_quant::is_k(t);
+    const int act_key = 2 * nbh_quant::act_of(t) + (k16 ? 1 : 0);
     if (!fuse && act_key != done_act) {
-      const int64_t ab = rm ? nbhs_quant_act_rm_bytes(t, n, in) : nbhs_quant_act_bytes(t, n, in);
+      const int64_t ab = k16 ? nbhs_quant_act_k16_bytes(t, n, in) : nbhs_quant_act_bytes(t, n, in);
       if (ab < 0) throw Error("matmul: invalid quantized shape");
       ensure(acts_buf_, acts_buf_bytes_, size_t(ab));
-      check(rm ? nbhs_quantize_acts_rm(t, x, n, in, acts_buf_, stream_)
-               : nbhs_quantize_acts(t, x, n, in, acts_buf_, stream_),
+      check(k16 ? nbhs_quantize_acts_k16(t, x, n, in, acts_buf_, int64_t(acts_buf_bytes_), stream_)
+                : nbhs_quantize_acts(t, x, n, in, acts_buf_, stream_),
             "matmul (activation quantization)");
       done_act = act_key;
     }
@@ -515,7 +515,9 @@ void HipBackend::matmul_multi(std::span<const Tensor* const> ws, const float* x,
           rows[j] = dw[i].rows;
           yp[j] = ys[i];
         }
-        check(nbhs_qgemm_multi(t, int(cnt), wp, rows, yp, in, acts_buf_, n, stream_), "matmul (quantized, tiled)");
+        check(k16 ? nbhs_qgemm_k16_multi(t, int(cnt), wp, rows, yp, in, acts_buf_, int64_t(acts_buf_bytes_), n, stream_)
+                  : nbhs_qgemm_multi(t, int(cnt), wp, rows, yp, in, acts_buf_, n, stream_),
+              "matmul (quantized, tiled)");
       }
       continue;
     }
@@ -651,16 +653,19 @@ void HipBackend::embed(const Tensor& table, std::span<const int32_t> ids, float*
   check_range(out, count, "embed", "out");
   const DeviceWeight w = device_weight(table, "embed");
   // the ids of a call of this size travel in the launch; more go through a buffer (and a wait for the stream)
-  const int32_t* host_ids = n <= NBHS_EMBED_ARG_IDS ? ids.data() : nullptr;
-  if (!host_ids) {
-    ensure(ids_buf_, ids_buf_bytes_, size_t(n) * sizeof(int32_t));
-    check(nbhs_memcpy_h2d(ids_buf_, ids.data(), size_t(n) * sizeof(int32_t), stream_), "embed ids upload");
+  const bool quant = nbh_quant::is_quant(int(w.type)), f16 = w.type == DType::F16;
+  if (n <= NBHS_EMBED_ARG_IDS) {
+    check(quant ? nbhs_dequant_rows_host_ids(int(w.type), w.dev, w.rows, d, ids.data(), n, out, stream_)
+                : nbhs_embed_host_ids(f16, w.dev, ids.data(), n, d, out, stream_),
+          "embed");
+    return;
   }
+  ensure(ids_buf_, ids_buf_bytes_, size_t(n) * sizeof(int32_t));
+  check(nbhs_memcpy_h2d(ids_buf_, ids.data(), size_t(n) * sizeof(int32_t), stream_), "embed ids upload");
   const auto* dev_ids = reinterpret_cast<const int32_t*>(ids_buf_);
-  if (nbh_quant::is_quant(int(w.type)))
-    check(nbhs_dequant_rows(int(w.type), w.dev, w.rows, d, host_ids, dev_ids, n, out, stream_), "embed (dequantize)");
-  else
-    check(nbhs_embed(w.type == DType::F16, w.dev, host_ids, dev_ids, n, d, out, stream_), "embed");
+  check(quant ? nbhs_dequant_rows(int(w.type), w.dev, w.rows, d, dev_ids, n, out, stream_)
+              : nbhs_embed(f16, w.dev, dev_ids, n, d, out, stream_),
+        "embed");
 }
 
 void HipBackend::rmsnorm(const float* x, const Tensor& weight, float* y, int64_t n, float eps) {

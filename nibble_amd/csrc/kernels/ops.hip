@@ -122,24 +122,31 @@ __global__ __launch_bounds__(kThreads) void silu_mul_kernel(float* __restrict__ 
   }
 }
 
+// far_ids: device ids, or null with the ids in arg.
+int launch_embed(int f16, const void* table, const EmbedIds& arg, const int32_t* far_ids, int64_t n, int64_t d, float* out,
+                 nbhs_stream s) {
+  const hipStream_t st = reinterpret_cast<hipStream_t>(s);
+  if (f16)
+    return nbhs_timing::launch(NBHS_K_ELEMENTWISE, embed_kernel<true>, dim3(unsigned(n)), dim3(kThreads), st, table, arg,
+                               far_ids, out, d);
+  return nbhs_timing::launch(NBHS_K_ELEMENTWISE, embed_kernel<false>, dim3(unsigned(n)), dim3(kThreads), st, table, arg,
+                             far_ids, out, d);
+}
+
 }  // namespace
 
 extern "C" {
 
-int nbhs_embed(int f16, const void* table, const int32_t* host_ids, const int32_t* ids, int64_t n, int64_t d, float* out,
-               nbhs_stream s) {
-  if (!table || !(host_ids ? n <= NBHS_EMBED_ARG_IDS : ids != nullptr) || !out || n <= 0 || d <= 0 ||
-      n >= (int64_t(1) << 31))
-    return NBHS_EINVAL;
-  const hipStream_t st = reinterpret_cast<hipStream_t>(s);
+int nbhs_embed(int f16, const void* table, const int32_t* ids, int64_t n, int64_t d, float* out, nbhs_stream s) {
+  if (!table || !ids || !out || n <= 0 || d <= 0 || n >= (int64_t(1) << 31)) return NBHS_EINVAL;
+  return launch_embed(f16, table, EmbedIds{}, ids, n, d, out, s);
+}
+
+int nbhs_embed_host_ids(int f16, const void* table, const int32_t* ids, int64_t n, int64_t d, float* out, nbhs_stream s) {
+  if (!table || !ids || !out || n <= 0 || d <= 0 || n > NBHS_EMBED_ARG_IDS) return NBHS_EINVAL;
   EmbedIds arg{};
-  if (host_ids) std::copy(host_ids, host_ids + n, arg.id);
-  const int32_t* const dev_ids = host_ids ? nullptr : ids;
-  if (f16)
-    return nbhs_timing::launch(NBHS_K_ELEMENTWISE, embed_kernel<true>, dim3(unsigned(n)), dim3(kThreads), st, table, arg,
-                               dev_ids, out, d);
-  return nbhs_timing::launch(NBHS_K_ELEMENTWISE, embed_kernel<false>, dim3(unsigned(n)), dim3(kThreads), st, table, arg,
-                             dev_ids, out, d);
+  std::copy(ids, ids + n, arg.id);
+  return launch_embed(f16, table, arg, nullptr, n, d, out, s);
 }
 
 int nbhs_rmsnorm_f32(const float* x, const float* w, float* y, int64_t n, int64_t d, float eps, nbhs_stream s) {

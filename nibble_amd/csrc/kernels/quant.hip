@@ -1835,101 +1835,27 @@ int launch_dequant(const QW& W, const int32_t* host_ids, const int32_t* ids, int
   return hipSuccess;
 }
 
-}  // namespace
-
-extern "C" {
-
-int64_t nbhs_quant_weight_bytes(int type, int64_t rows, int64_t in) {
-  if (!is_quant(type) || rows <= 0 || in <= 0 || in % block_elems(type)) return -1;
-  return weight_layout(type, rows, in / block_elems(type)).bytes;
-}
-
-int64_t nbhs_quant_act_bytes(int type, int64_t n, int64_t in) {
-  if (!is_quant(type) || n <= 0 || in <= 0 || in % block_elems(type)) return -1;
-  return act_layout(act_of(type), n, in / block_elems(type)).bytes;
-}
-
-int64_t nbhs_quant_act_rm_bytes(int type, int64_t n, int64_t in) {
-  if (!is_k(type) || n <= 0 || in <= 0 || in % 256) return -1;
-  return act_layout(kActQ8_K16, n, in / 256).bytes;
-}
-
-int nbhs_quantize_acts(int type, const float* x, int64_t n, int64_t in, void* acts, nbhs_stream stream) {
-  if (!is_quant(type) || !x || !acts || n <= 0 || in <= 0 || in % block_elems(type)) return NBHS_EINVAL;
-  const int act = act_of(type);
-  const int64_t nb = in / block_elems(type), blocks = n * nb;
-  const ActLayout l = act_layout(act, n, nb);
-  uint8_t* base = static_cast<uint8_t*>(acts);
-  int8_t* qs = reinterpret_cast<int8_t*>(base + l.qs_off);
-  float* d = reinterpret_cast<float*>(base + l.d_off);
-  const hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  if (act == kActQ8_K) {
-    if (blocks >= (int64_t(1) << 31)) return NBHS_EINVAL;
-    return nbhs_timing::launch(NBHS_K_QUANTIZE, quantize_q8k_kernel<false>, dim3(unsigned(blocks)), dim3(64), s, x, in,
-                               qs, d, reinterpret_cast<int16_t*>(base + l.bsums_off));
-  }
-  const dim3 grid{unsigned((blocks + 255) / 256), 1, 1};
-  if (act == kActQ8_1)
-    return nbhs_timing::launch(NBHS_K_QUANTIZE, quantize_q8_kernel<true>, grid, dim3(256), s, x, in, n, qs, d,
-                               reinterpret_cast<float*>(base + l.s_off));
-  return nbhs_timing::launch(NBHS_K_QUANTIZE, quantize_q8_kernel<false>, grid, dim3(256), s, x, in, n, qs, d,
-                             static_cast<float*>(nullptr));
-}
-
-int nbhs_quantize_acts_rm(int type, const float* x, int64_t n, int64_t in, void* acts, nbhs_stream stream) {
-  if (!is_k(type) || !x || !acts || n <= 0 || in <= 0 || in % 256) return NBHS_EINVAL;
-  const int64_t nb = in / 256, blocks = n * nb;
-  if (blocks >= (int64_t(1) << 31)) return NBHS_EINVAL;
-  const ActLayout l = act_layout(kActQ8_K16, n, nb);
-  uint8_t* base = static_cast<uint8_t*>(acts);
-  return nbhs_timing::launch(NBHS_K_QUANTIZE, quantize_q8k_kernel<true>, dim3(unsigned(blocks)), dim3(64),
-                             reinterpret_cast<hipStream_t>(stream), x, in, reinterpret_cast<int8_t*>(base + l.qs_off),
-                             reinterpret_cast<float*>(base + l.d_off), reinterpret_cast<int16_t*>(base + l.bsums_off));
-}
-
-int nbhs_qgemv_multi(int type, int n_w, const void* const* w, const int64_t* rows, float* const* y, int64_t in,
-                     const float* x, const void* acts, int64_t n_acts, int64_t t0, int64_t n, nbhs_stream stream) {
-  if (!is_quant(type) || n_w <= 0 || n_w > kMaxQWeights || !w || !rows || !y || in <= 0 ||
-      in % block_elems(type) || n <= 0 || n > NBHS_GEMV_MAX_ROWS)
+int dequant_rows(int type, const void* w, int64_t rows, int64_t in, const int32_t* host_ids, const int32_t* ids, int64_t n,
+                 float* out, nbhs_stream stream) {
+  if (!is_quant(type) || !w || !out || rows <= 0 || in <= 0 || in % block_elems(type) || n <= 0 ||
+      (in + 255) / 256 >= (int64_t(1) << 31))
     return NBHS_EINVAL;
-  const bool fused = acts == nullptr;
-  if (fused ? (!x || n > 4 || t0 != 0 || reinterpret_cast<uintptr_t>(x) % 16 || in % 4) : (t0 < 0 || t0 + n > n_acts))
-    return NBHS_EINVAL;
-  QBatch B{};
-  for (int i = 0; i < n_w; ++i) {
-    if (!w[i] || !y[i] || rows[i] <= 0) return NBHS_EINVAL;
-    B.w[i] = weight_of(type, w[i], rows[i], in);
-    B.y[i] = y[i];
-  }
-  B.n_w = n_w;
-  const int64_t nb = in / block_elems(type);
-  QA A{};
-  A.nb = nb;
-  if (!fused) {
-    const int act = act_of(type);
-    const ActLayout l = act_layout(act, n_acts, nb);
-    const uint8_t* base = static_cast<const uint8_t*>(acts);
-    const int64_t b0 = t0 * nb;  // first block of activation row t0
-    A.qs = reinterpret_cast<const int8_t*>(base + l.qs_off) + b0 * (act == kActQ8_K ? 256 : 32);
-    A.d = reinterpret_cast<const float*>(base + l.d_off) + b0;
-    A.s = act == kActQ8_1 ? reinterpret_cast<const float*>(base + l.s_off) + b0 : nullptr;
-    A.bsums = reinterpret_cast<const int16_t*>(base + l.bsums_off) + b0 * 16;
-  }
+  const QW W = weight_of(type, w, rows, in);
   const hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   switch (type) {
-    case kQ4_0: return launch_gemv<kQ4_0>(B, rows, n_w, A, x, in, n, fused, s);
-    case kQ5_0: return launch_gemv<kQ5_0>(B, rows, n_w, A, x, in, n, fused, s);
-    case kQ5_1: return launch_gemv<kQ5_1>(B, rows, n_w, A, x, in, n, fused, s);
-    case kQ8_0: return launch_gemv<kQ8_0>(B, rows, n_w, A, x, in, n, fused, s);
-    case kQ4_K: return launch_gemv<kQ4_K>(B, rows, n_w, A, x, in, n, fused, s);
-    case kQ5_K: return launch_gemv<kQ5_K>(B, rows, n_w, A, x, in, n, fused, s);
-    case kQ6_K: return launch_gemv<kQ6_K>(B, rows, n_w, A, x, in, n, fused, s);
+    case kQ4_0: return launch_dequant<kQ4_0>(W, host_ids, ids, n, out, s);
+    case kQ5_0: return launch_dequant<kQ5_0>(W, host_ids, ids, n, out, s);
+    case kQ5_1: return launch_dequant<kQ5_1>(W, host_ids, ids, n, out, s);
+    case kQ8_0: return launch_dequant<kQ8_0>(W, host_ids, ids, n, out, s);
+    case kQ4_K: return launch_dequant<kQ4_K>(W, host_ids, ids, n, out, s);
+    case kQ5_K: return launch_dequant<kQ5_K>(W, host_ids, ids, n, out, s);
+    case kQ6_K: return launch_dequant<kQ6_K>(W, host_ids, ids, n, out, s);
     default: return NBHS_EINVAL;
   }
 }
 
-int nbhs_qgemm_multi(int type, int n_w, const void* const* w, const int64_t* rows, float* const* y, int64_t in,
-                     const void* acts, int64_t n, nbhs_stream stream) {
+int qgemm_multi(int type, int n_w, const void* const* w, const int64_t* rows, float* const* y, int64_t in, const void* acts,
+                int64_t n, nbhs_stream stream) {
   if (!is_quant(type) || n_w <= 0 || n_w > kMaxQWeights || !w || !rows || !y || !acts ||
       in <= 0 || in % block_elems(type) || n <= 0 || (n + 31) / 32 > 65535)
     return NBHS_EINVAL;
@@ -1983,23 +1909,122 @@ int nbhs_qgemm_multi(int type, int n_w, const void* const* w, const int64_t* row
   }
 }
 
-int nbhs_dequant_rows(int type, const void* w, int64_t rows, int64_t in, const int32_t* host_ids, const int32_t* ids,
-                      int64_t n, float* out, nbhs_stream stream) {
-  if (!is_quant(type) || !w || !(host_ids ? n <= NBHS_EMBED_ARG_IDS : ids != nullptr) || !out || rows <= 0 || in <= 0 ||
-      in % block_elems(type) || n <= 0 || (in + 255) / 256 >= (int64_t(1) << 31))
+}  // namespace
+
+extern "C" {
+
+int64_t nbhs_quant_weight_bytes(int type, int64_t rows, int64_t in) {
+  if (!is_quant(type) || rows <= 0 || in <= 0 || in % block_elems(type)) return -1;
+  return weight_layout(type, rows, in / block_elems(type)).bytes;
+}
+
+int64_t nbhs_quant_act_bytes(int type, int64_t n, int64_t in) {
+  if (!is_quant(type) || n <= 0 || in <= 0 || in % block_elems(type)) return -1;
+  return act_layout(act_of(type), n, in / block_elems(type)).bytes;
+}
+
+int64_t nbhs_quant_act_k16_bytes(int type, int64_t n, int64_t in) {
+  if (!is_k(type) || n <= 0 || in <= 0 || in % 256) return -1;
+  return act_layout(kActQ8_K16, n, in / 256).bytes;
+}
+
+int nbhs_quantize_acts(int type, const float* x, int64_t n, int64_t in, void* acts, nbhs_stream stream) {
+  if (!is_quant(type) || !x || !acts || n <= 0 || in <= 0 || in % block_elems(type)) return NBHS_EINVAL;
+  const int act = act_of(type);
+  const int64_t nb = in / block_elems(type), blocks = n * nb;
+  const ActLayout l = act_layout(act, n, nb);
+  uint8_t* base = static_cast<uint8_t*>(acts);
+  int8_t* qs = reinterpret_cast<int8_t*>(base + l.qs_off);
+  float* d = reinterpret_cast<float*>(base + l.d_off);
+  const hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  if (act == kActQ8_K) {
+    if (blocks >= (int64_t(1) << 31)) return NBHS_EINVAL;
+    return nbhs_timing::launch(NBHS_K_QUANTIZE, quantize_q8k_kernel<false>, dim3(unsigned(blocks)), dim3(64), s, x, in,
+                               qs, d, reinterpret_cast<int16_t*>(base + l.bsums_off));
+  }
+  const dim3 grid{unsigned((blocks + 255) / 256), 1, 1};
+  if (act == kActQ8_1)
+    return nbhs_timing::launch(NBHS_K_QUANTIZE, quantize_q8_kernel<true>, grid, dim3(256), s, x, in, n, qs, d,
+                               reinterpret_cast<float*>(base + l.s_off));
+  return nbhs_timing::launch(NBHS_K_QUANTIZE, quantize_q8_kernel<false>, grid, dim3(256), s, x, in, n, qs, d,
+                             static_cast<float*>(nullptr));
+}
+
+int nbhs_quantize_acts_rm(int, const float*, int64_t, int64_t, void*, nbhs_stream) { return NBHS_EINVAL; }
+
+int nbhs_quantize_acts_k16(int type, const float* x, int64_t n, int64_t in, void* acts, int64_t acts_bytes,
+                           nbhs_stream stream) {
+  const int64_t need = nbhs_quant_act_k16_bytes(type, n, in);
+  if (need < 0 || acts_bytes < need || !x || !acts) return NBHS_EINVAL;
+  const int64_t nb = in / 256, blocks = n * nb;
+  if (blocks >= (int64_t(1) << 31)) return NBHS_EINVAL;
+  const ActLayout l = act_layout(kActQ8_K16, n, nb);
+  uint8_t* base = static_cast<uint8_t*>(acts);
+  return nbhs_timing::launch(NBHS_K_QUANTIZE, quantize_q8k_kernel<true>, dim3(unsigned(blocks)), dim3(64),
+                             reinterpret_cast<hipStream_t>(stream), x, in, reinterpret_cast<int8_t*>(base + l.qs_off),
+                             reinterpret_cast<float*>(base + l.d_off), reinterpret_cast<int16_t*>(base + l.bsums_off));
+}
+
+int nbhs_qgemv_multi(int type, int n_w, const void* const* w, const int64_t* rows, float* const* y, int64_t in,
+                     const float* x, const void* acts, int64_t n_acts, int64_t t0, int64_t n, nbhs_stream stream) {
+  if (!is_quant(type) || n_w <= 0 || n_w > kMaxQWeights || !w || !rows || !y || in <= 0 ||
+      in % block_elems(type) || n <= 0 || n > NBHS_GEMV_MAX_ROWS)
     return NBHS_EINVAL;
-  const QW W = weight_of(type, w, rows, in);
+  const bool fused = acts == nullptr;
+  if (fused ? (!x || n > 4 || t0 != 0 || reinterpret_cast<uintptr_t>(x) % 16 || in % 4) : (t0 < 0 || t0 + n > n_acts))
+    return NBHS_EINVAL;
+  QBatch B{};
+  for (int i = 0; i < n_w; ++i) {
+    if (!w[i] || !y[i] || rows[i] <= 0) return NBHS_EINVAL;
+    B.w[i] = weight_of(type, w[i], rows[i], in);
+    B.y[i] = y[i];
+  }
+  B.n_w = n_w;
+  const int64_t nb = in / block_elems(type);
+  QA A{};
+  A.nb = nb;
+  if (!fused) {
+    const int act = act_of(type);
+    const ActLayout l = act_layout(act, n_acts, nb);
+    const uint8_t* base = static_cast<const uint8_t*>(acts);
+    const int64_t b0 = t0 * nb;  // first block of activation row t0
+    A.qs = reinterpret_cast<const int8_t*>(base + l.qs_off) + b0 * (act == kActQ8_K ? 256 : 32);
+    A.d = reinterpret_cast<const float*>(base + l.d_off) + b0;
+    A.s = act == kActQ8_1 ? reinterpret_cast<const float*>(base + l.s_off) + b0 : nullptr;
+    A.bsums = reinterpret_cast<const int16_t*>(base + l.bsums_off) + b0 * 16;
+  }
   const hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   switch (type) {
-    case kQ4_0: return launch_dequant<kQ4_0>(W, host_ids, ids, n, out, s);
-    case kQ5_0: return launch_dequant<kQ5_0>(W, host_ids, ids, n, out, s);
-    case kQ5_1: return launch_dequant<kQ5_1>(W, host_ids, ids, n, out, s);
-    case kQ8_0: return launch_dequant<kQ8_0>(W, host_ids, ids, n, out, s);
-    case kQ4_K: return launch_dequant<kQ4_K>(W, host_ids, ids, n, out, s);
-    case kQ5_K: return launch_dequant<kQ5_K>(W, host_ids, ids, n, out, s);
-    case kQ6_K: return launch_dequant<kQ6_K>(W, host_ids, ids, n, out, s);
+    case kQ4_0: return launch_gemv<kQ4_0>(B, rows, n_w, A, x, in, n, fused, s);
+    case kQ5_0: return launch_gemv<kQ5_0>(B, rows, n_w, A, x, in, n, fused, s);
+    case kQ5_1: return launch_gemv<kQ5_1>(B, rows, n_w, A, x, in, n, fused, s);
+    case kQ8_0: return launch_gemv<kQ8_0>(B, rows, n_w, A, x, in, n, fused, s);
+    case kQ4_K: return launch_gemv<kQ4_K>(B, rows, n_w, A, x, in, n, fused, s);
+    case kQ5_K: return launch_gemv<kQ5_K>(B, rows, n_w, A, x, in, n, fused, s);
+    case kQ6_K: return launch_gemv<kQ6_K>(B, rows, n_w, A, x, in, n, fused, s);
     default: return NBHS_EINVAL;
   }
+}
+
+int nbhs_qgemm_multi(int type, int n_w, const void* const* w, const int64_t* rows, float* const* y, int64_t in,
+                     const void* acts, int64_t n, nbhs_stream stream) {
+  return is_k(type) ? NBHS_EINVAL : qgemm_multi(type, n_w, w, rows, y, in, acts, n, stream);
+}
+
+int nbhs_qgemm_k16_multi(int type, int n_w, const void* const* w, const int64_t* rows, float* const* y, int64_t in,
+                         const void* acts, int64_t acts_bytes, int64_t n, nbhs_stream stream) {
+  const int64_t need = nbhs_quant_act_k16_bytes(type, n, in);
+  return need < 0 || acts_bytes < need ? NBHS_EINVAL : qgemm_multi(type, n_w, w, rows, y, in, acts, n, stream);
+}
+
+int nbhs_dequant_rows(int type, const void* w, int64_t rows, int64_t in, const int32_t* ids, int64_t n, float* out,
+                      nbhs_stream stream) {
+  return ids ? dequant_rows(type, w, rows, in, nullptr, ids, n, out, stream) : NBHS_EINVAL;
+}
+
+int nbhs_dequant_rows_host_ids(int type, const void* w, int64_t rows, int64_t in, const int32_t* ids, int64_t n, float* out,
+                               nbhs_stream stream) {
+  return ids && n <= NBHS_EMBED_ARG_IDS ? dequant_rows(type, w, rows, in, ids, nullptr, n, out, stream) : NBHS_EINVAL;
 }
 
 }  // extern "C"
