@@ -33,6 +33,22 @@ def test_embed_bit_exact(backend, dt, d):
     backend.release_weights()
 
 
+@pytest.mark.parametrize("n", [511, 512, 513, 1500])
+@pytest.mark.parametrize("dt", [np.float32, np.float16], ids=["f32", "f16"])
+def test_embed_many_ids(backend, dt, n):
+    """512 ids travel in the launch, more in a device buffer; the buffer of a longer call serves a shorter one next."""
+    rng = np.random.default_rng(n)
+    d = 200
+    table = rng.standard_normal((300, d)).astype(dt)
+    for ids in (rng.integers(0, 300, n).astype(np.int32), rng.integers(0, 300, n - 1).astype(np.int32)):
+        with Buffers(backend) as B:
+            out = B.alloc(ids.size * d)
+            backend.embed(table, ids, out)
+            got = backend.download(out, (ids.size, d))
+        assert np.array_equal(bits(got), bits(oracle.embed(table, ids)))
+    backend.release_weights()
+
+
 def test_embed_rejects_bad_ids_before_any_work(backend):
     table = np.zeros((10, 8), np.float32)
     with Buffers(backend) as B:
@@ -46,6 +62,26 @@ def test_embed_rejects_bad_ids_before_any_work(backend):
 
 @pytest.mark.parametrize("n,d", [(1, 896), (5, 2048), (512, 2048), (3, 16), (7, 1000)])
 def test_rmsnorm_matches_reference(backend, n, d):
+    rng = np.random.default_rng(n * d)
+    x = (rng.standard_normal((n, d)) * rng.uniform(0.01, 50, (n, 1))).astype(np.float32)
+    w = rng.uniform(0.5, 1.5, d).astype(np.float32)
+    with Buffers(backend) as B:
+        dx, dy = B.upload(x), B.alloc(n * d)
+        backend.rmsnorm(dx, w, dy, n, 1e-5)
+        got = backend.download(dy, (n, d))
+        backend.rmsnorm(dx, w, dx, n, 1e-5)  # in place (x == y) gives the same bits
+        inplace = backend.download(dx, (n, d))
+    ref = oracle.rmsnorm(x, w, 1e-5)
+    u = ulp_diff(got, ref)
+    print(f"rmsnorm n={n} d={d}: {int(np.sum(u > 0))} elements differ, max {int(u.max())} ulp", flush=True)
+    assert int(u.max()) <= 1
+    assert np.array_equal(bits(got), bits(inplace))
+    backend.release_weights()
+
+
+@pytest.mark.parametrize("n,d", [(1, 2047), (2, 2049), (3, 2304), (5, 3072), (1, 10001)])
+def test_rmsnorm_rows_beyond_the_registers(backend, n, d):
+    """Rows about and beyond the 2048 elements that a workgroup holds, the rest read twice; in place as well."""
     rng = np.random.default_rng(n * d)
     x = (rng.standard_normal((n, d)) * rng.uniform(0.01, 50, (n, 1))).astype(np.float32)
     w = rng.uniform(0.5, 1.5, d).astype(np.float32)

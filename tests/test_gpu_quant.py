@@ -80,6 +80,21 @@ def test_quant_embed_bit_exact(backend, t):
     backend.release_weights()
 
 
+@pytest.mark.parametrize("n", [511, 512, 513, 1500])
+@pytest.mark.parametrize("t", TYPES, ids=[U.NAMES[t] for t in TYPES])
+def test_quant_embed_many_ids(backend, t, n):
+    """512 ids travel in the launch, more in a device buffer; rows of one workgroup and more."""
+    d = 512 if oracle.block_elems(t) == 256 else 288
+    table = U.random_qmat(t, 50, d, seed=90 + t)
+    ids = np.random.default_rng(n).integers(0, 50, n).astype(np.int32)
+    with Buffers(backend) as B:
+        out = B.alloc(n * d)
+        backend.embed(table, ids, out)
+        got = backend.download(out, (n, d))
+    assert np.array_equal(bits(got), bits(np.asarray(table)[ids]))
+    backend.release_weights()
+
+
 @pytest.mark.parametrize("n", [2, 100])
 def test_quant_non_finite_activations(backend, n):
     """A NaN in an activation block makes its scale NaN (quant.cpp:37-49, 273-303): every output that reads the
@@ -187,8 +202,8 @@ def test_quant_tiled_k_both_kernels(backend, t):
 
 @pytest.mark.parametrize("n", [17, 80, 130])
 def test_quant_tiled_k_types_mixed(backend, n):
-    """Prefill-sized calls over K-type weights, which run the int8 matrix-core kernel on residue-major Q8_K
-    activations, mixed in one call with a Q8_0 weight (the legacy tiled kernel on Q8_0 activations): the
+    """Prefill-sized calls over K-type weights, which run the fp16 matrix-core kernels on activations in an operand form of
+    their own, mixed in one call with a Q8_0 weight (the legacy tiled kernel on Q8_0 activations): the
     activations are quantized once per layout, in the order the types come. Row counts that end inside a 16-row
     tile, three super-blocks per row, activation rows that end inside a 64-row tile. Every output bit-exact."""
     in_ = 768
@@ -278,13 +293,14 @@ def test_quant_single_row_over_many_rows(backend, t):
 @pytest.mark.parametrize("nb", [1, 2, 3, 4, 5, 6, 7, 13])
 @pytest.mark.parametrize("t", KTYPES, ids=[U.NAMES[t] for t in KTYPES])
 def test_quant_tiled_k_super_block_counts(backend, t, nb, extreme):
-    """The 64 x 32 K kernel over every length of its unrolled super-block loop (six per trip: one trip cut short at
-    each point, a whole one, two and a rest), rows and activation rows that end inside a tile, row counts that are and
-    are not a multiple of four (vector stores). `extreme`: the operands whose exact sums come closest to the fp32
+    """The tiled K kernels over every length of the 64 x 32 one's unrolled super-block loop (six per trip: one trip cut
+    short at each point, a whole one, two and a rest), rows and activation rows that end inside a tile: 2497 and 2500
+    weight rows in 64 x 32 tiles (2500, a multiple of four, by vector stores), 1300 in 16 x 32 ones, whose waves share
+    the super-blocks. `extreme`: the operands whose exact sums come closest to the fp32
     accumulator's 2^24 - every quant and sub-block scale the largest (Q6_K: -32 times -128 and 31 times 127) against
     activations quantized to +-127. Every output bit-exact."""
     in_ = 256 * nb
-    for rows, n in ((2497, 33), (1300, 61)):
+    for rows, n in ((2497, 33), (2500, 61), (1300, 61)):
         w = U.random_qmat(t, rows, in_, seed=40 + t + nb)
         x = (np.random.default_rng(nb).standard_normal((n, in_)) * 2).astype(np.float32)
         if extreme:
@@ -350,3 +366,23 @@ def test_quant_tiled_legacy_block_counts(backend, t, nb):
         ref = oracle.matmul_q(t, w.raw, in_, rows, x)
         assert np.array_equal(bits(got), bits(ref)), (U.NAMES[t], rows, n, nb)
         backend.release_weights()
+
+
+@pytest.mark.parametrize("t", KTYPES, ids=[U.NAMES[t] for t in KTYPES])
+def test_quant_k_single_row_wide_and_long(backend, t):
+    """One activation row of 65 super-blocks, wider than the K types' kernel for few rows holds, over 16387 weight rows: the
+    general matvec kernel with eight rows to a wave, the last wave cut short. Every output bit-exact (on the first, some
+    middle and the last rows)."""
+    nb, rows = 65, 16387
+    in_, per = 256 * nb, nb * oracle.block_bytes(t)
+    tile = U.random_qmat(t, 301, in_, seed=t).raw
+    w = U.QMat(t, np.tile(tile, -(-rows // 301))[:rows * per], rows, in_)
+    x = (np.random.default_rng(t).standard_normal((1, in_)) * 2).astype(np.float32)
+    with Buffers(backend) as B:
+        dx, dy = B.upload(x), B.alloc(rows)
+        backend.matmul(w, dx, dy, 1)
+        got = backend.download(dy, (1, rows))
+    backend.release_weights()
+    for r0, r1 in ((0, 301), (8000, 8100), (rows - 301, rows)):
+        ref = oracle.matmul_q(t, np.ascontiguousarray(w.raw[r0 * per:r1 * per]), in_, r1 - r0, x)
+        assert np.array_equal(bits(got[:, r0:r1]), bits(ref)), (U.NAMES[t], r0)
