@@ -1140,12 +1140,15 @@ __global__ __launch_bounds__(256) void qgemm_legacy_kernel(QGemmBatch B, QA A, i
 
 // The legacy kernel's tile for a launch: 64 x 64 while 64 x 64 tiles give at least kLegacyMinWgs workgroups
 // (two per CU); else 64 x 32 while those do; else 32 x 32 (more, smaller workgroups: at the QKV shape 16-80 rows
-// run 10-20 % faster than with 64 x 32, and 512 rows 3-5 % slower). A wave of
-// a 32 x 32 tile has one MFMA per block, a chain of LDS read, MFMA and float term; up to kLegacyUnrollWgs workgroups
-// leave a SIMD about two such waves, so four blocks go in flight (Q8_0: the QKV shape at 40 rows, 192 workgroups, 15.0 ->
-// 13.0 us, at 150, 480, 17.1 -> 16.5; feed-forward blocks of 77 rows 896 -> 3584 -> 896 wide 42.6 -> 38.7, 2048 -> 8192
-// -> 2048 86.7 -> 77.4). With more workgroups the registers cost waves: at 300 rows, 960, 23.8 -> 24.6.
-constexpr int64_t kLegacyUnrollWgs = 512;
+// run 10-20 % faster than with 64 x 32, and 512 rows 3-5 % slower). A wave of a 32 x 32 tile has one MFMA per block, a
+// chain of LDS read, MFMA and float term. While a launch leaves a SIMD about one such wave, or two where a block's
+// operands take few registers, four blocks go in flight; beyond, the registers cost waves. One block against four, us a
+// call at 64-256, 280-512 and 560-768 workgroups (o: 2048 -> 2048 wide, down: 8192 -> 2048):
+//   Q8_0  down x 40  41.9 / 34.7   down x 200  49.2 / 46.9   down x 300  59.8 / 62.5
+//   Q5_1  down x 40  60.0 / 54.4   down x 200  74.1 / 72.8   down x 300  95.6 / 91.2
+//   Q4_0  down x 40  43.7 / 39.8   down x 200  52.3 / 53.3   o x 200  18.0 / 18.0   down x 300  64.5 / 69.2
+//   Q5_0  down x 40  53.4 / 51.7   down x 200  68.3 / 72.4   o x 200  22.0 / 23.0   down x 300  88.7 / 97.5
+constexpr int64_t legacy_unroll_wgs(int type) { return type == kQ4_0 || type == kQ5_0 ? 256 : 512; }
 constexpr int64_t kLegacyMinWgs = 512;
 enum LegacyTile { kTile64x64, kTile64x32, kTile32x32 };
 template <int T>
@@ -1157,7 +1160,7 @@ hipError_t launch_legacy(LegacyTile tile, unsigned tiles, int64_t n, hipStream_t
   const dim3 grid{tiles, unsigned((n + 31) / 32)};
   if (tile == kTile64x32)
     return nbhs_timing::launch(NBHS_K_QGEMM, qgemm_legacy_kernel<T, 2>, grid, dim3(256), s, B, A, n);
-  if (int64_t(grid.x) * grid.y <= kLegacyUnrollWgs)
+  if (int64_t(grid.x) * grid.y <= legacy_unroll_wgs(T))
     return nbhs_timing::launch(NBHS_K_QGEMM, qgemm_legacy_kernel<T, 2, 32, 4>, grid, dim3(256), s, B, A, n);
   return nbhs_timing::launch(NBHS_K_QGEMM, qgemm_legacy_kernel<T, 2, 32>, grid, dim3(256), s, B, A, n);
 }
