@@ -696,11 +696,12 @@ __global__ __launch_bounds__(64) void qgemv_kernel(QBatch B, QA A, const float* 
 // lanes' integer lane sums are added exactly by DPP, lane c keeping aux[2 c] and aux[2 c + 1]; their float terms go to
 // the wave's LDS slice and are then added in super-block order, a lane per (row, integer lane) chain: the reference's
 // operations in its order (quant.cpp:118-144, 394-416).
-// It is bound by memory latency at decode sizes: a pass of 16 pairs is 2.3-3.4 KB per wave, so P passes are requested
-// before any is computed. The kernel it replaces gave a lane a whole super-block (64 scattered 128-byte reads an
-// instruction) and had every wave quantize the activations by itself, super-block chunk after chunk. Measured (start
-// to here): 131072 weight rows, K = 2048, Q6_K 72 -> 52 us (4.2 TB/s), Q4_K 57 -> 36; 2048 rows, K = 8192, Q6_K 20 -> 12;
-// 3072 rows, K = 2048, Q4_K 6.4 -> 5.8, three activation rows 14.2 -> 9.5.
+// A pass of 16 pairs is 2.3-3.4 KB per wave, so P passes are requested before any is computed. What bounds it by its
+// counters: VALU issue at many rows (131072 rows, K = 2048, one activation row: the VALU busy 62 % of the time with Q6_K at
+// 4.2 TB/s, 57 % with Q4_K; waves wait 38-41 % of their time to issue and 23-26 % for loads), the loads' latency at few
+// (2048 rows, K = 8192: 48 % for loads). Two activation rows have an instance of their own, whose LDS leaves room for up to
+// four workgroups on a CU; the one for four rows holds two. us a call: 131072 weight rows, K = 2048, Q6_K 48, Q4_K 32; 2048
+// rows, K = 8192, Q6_K 9.9, Q4_K 8.8; 3072 rows, K = 2048, Q4_K 6.1, three activation rows 9.8.
 constexpr int kGemvChunk = 16;  // super-blocks of a pass
 constexpr int kgemv_max_sb(int nt) { return nt == 1 ? 64 : 32; }  // super-blocks of a row, at most (LDS)
 
@@ -1768,32 +1769,77 @@ QW weight_of(int type, const void* w, int64_t rows, int64_t in) {
             reinterpret_cast<const uint16_t*>(base + l.m_off), rows, nb};
 }
 
-// Passes in flight per wave while that leaves the launch half of kKGemvWaves waves, and batches while it leaves all of
-// them (measured with 1024 .. 16384 waves: 131072 rows of Q4_K 48 / 38 / 35 / 40 / 42 us at 1 / 2 / 4 / 8 / 16 x 1024;
-// 16384 rows 9.6 us with four passes in flight and 2048 waves, 10.2 with two and 4096).
-constexpr int64_t kKGemvWaves = 4096;
-template <int T>
-int launch_kgemv(const QBatch& B, const int64_t* rows, int n_w, const float* x, int64_t in, int64_t n, hipStream_t s) {
-  const int64_t nb = in / 256, rp = kGemvChunk / (nb < kGemvChunk ? nb : kGemvChunk);
+// How a call is laid over kgemv_kernel's grid: passes in flight per wave and batches of rows per wave. All workgroups run
+// at once, 1 to as many on a CU as its registers and LDS hold, and the fullest CU sets the time: its workgroups times the
+// rows a wave of theirs takes (batches x rows of a batch, and half a row for quantizing the activations). Few waves on a
+// SIMD and few passes in flight hide less latency; the factors are fitted to 600 calls (2-56 super-blocks, 5120-151936
+// rows, 1-4 activation rows) in each of the layouts, which come out 1.2 % from the best one on average. Against a layout by
+// a number of waves (4096, with as many batches as fill them), whose grid may end in a second round of a few workgroups, us
+// a call: 14336 rows, K = 2048, two activation rows, Q4_K 17.0 -> 13.1; 28672 rows, K = 4096, Q5_K, one 29.6 -> 23.6, two
+// 40.3 -> 34.7; Q4_K, four 60.2 -> 51.2; 16384 rows, K = 2048, one, Q6_K 11.7 -> 11.7. Not caught: 131072 rows of 2
+// super-blocks, four rows, Q6_K 42.0 -> 44.6, where a second round of short workgroups overlaps the first.
+constexpr int64_t kCUs = 256;
+struct KGemvPlan {
+  int passes = 0;
+  int64_t batches = 0;
+  double cost = 0;
+};
+
+// Workgroups of NT, P on a CU.
+template <int T, int NT, int P>
+int kgemv_resident() {
+  static const int v = [] {
+    int b = 0;
+    const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, kgemv_kernel<T, NT, P>, 256, 0);
+    return e == hipSuccess ? std::clamp(b, 1, 4) : 1;
+  }();
+  return v;
+}
+
+template <int T, int NT, int P>
+void plan_kgemv(const int64_t* rows, int n_w, int64_t nb, KGemvPlan& best) {
+  const int64_t rp = kGemvChunk / std::min<int64_t>(nb, kGemvChunk), rb = std::min<int64_t>(P * rp, 8);
+  if (P > 1 && P * rp > 8) return;
+  auto wgs_of = [&](int64_t batches) {
+    int64_t wgs = 0;
+    for (int i = 0; i < n_w; ++i) wgs += (rows[i] + 4 * rb * batches - 1) / (4 * rb * batches);
+    return wgs;
+  };
   int64_t total = 0;
   for (int i = 0; i < n_w; ++i) total += rows[i];
-  const int64_t passes = (total + rp - 1) / rp / kKGemvWaves;  // of each wave, at that size
-  const int p = passes >= 2 && 4 * rp <= 8 ? 4 : passes >= 1 && 2 * rp <= 8 ? 2 : 1;
-  const int64_t rb = std::min<int64_t>(p * rp, 8), batches = std::max<int64_t>(1, total / rb / kKGemvWaves);
+  constexpr double kWaves[] = {0, 1.7, 1.15, 1.075, 1}, kPasses = P == 4 ? 1 : P == 2 ? 1.1 : 1.4;
+  int64_t last = 0;
+  for (int w = kgemv_resident<T, NT, P>(); w >= 1; --w) {
+    int64_t batches = std::max<int64_t>(1, (total + rb * 4 * kCUs * w - 1) / (rb * 4 * kCUs * w));
+    if (batches == last) continue;  // the same layout
+    int64_t wgs = wgs_of(batches);
+    while (wgs > kCUs * w) wgs = wgs_of(++batches);  // (a partial last workgroup of each weight)
+    last = batches;
+    const int64_t per_cu = (wgs + kCUs - 1) / kCUs;
+    const double cost = double(per_cu) * (double(batches * rb) + 0.5) * kWaves[per_cu] * kPasses;
+    if (best.passes == 0 || cost < best.cost) best = KGemvPlan{P, batches, cost};
+  }
+}
+
+template <int T, int NT>
+int launch_kgemv(const QBatch& B, const int64_t* rows, int n_w, const float* x, int64_t in, int64_t n, hipStream_t s) {
+  const int64_t nb = in / 256, rp = kGemvChunk / std::min<int64_t>(nb, kGemvChunk);
+  KGemvPlan plan;
+  plan_kgemv<T, NT, 4>(rows, n_w, nb, plan);
+  plan_kgemv<T, NT, 2>(rows, n_w, nb, plan);
+  plan_kgemv<T, NT, 1>(rows, n_w, nb, plan);
+  if (plan.batches > INT32_MAX) return NBHS_EINVAL;
+  const int64_t wg_rows = 4 * std::min<int64_t>(plan.passes * rp, 8) * plan.batches;
   QBatch b = B;
   int64_t wgs = 0;
-  for (int i = 0; i < n_w; ++i) b.wave0[i] = wgs, wgs += (rows[i] + 4 * rb * batches - 1) / (4 * rb * batches);
-  if (wgs >= (int64_t(1) << 31) || batches > INT32_MAX) return NBHS_EINVAL;
+  for (int i = 0; i < n_w; ++i) b.wave0[i] = wgs, wgs += (rows[i] + wg_rows - 1) / wg_rows;
   const dim3 grid{unsigned(wgs), 1, 1}, block{256, 1, 1};
-  auto go = [&](auto nt, auto pc) {
-    return nbhs_timing::launch(NBHS_K_QGEMV, kgemv_kernel<T, decltype(nt)::value, decltype(pc)::value>, grid, block, s, b,
-                               x, in, int(n), int(batches));
+  auto go = [&](auto kernel) {
+    return nbhs_timing::launch(NBHS_K_QGEMV, kernel, grid, block, s, b, x, in, int(n), int(plan.batches));
   };
-  using I1 = std::integral_constant<int, 1>;
-  using I2 = std::integral_constant<int, 2>;
-  using I4 = std::integral_constant<int, 4>;
-  if (n == 1) return p == 4 ? go(I1{}, I4{}) : p == 2 ? go(I1{}, I2{}) : go(I1{}, I1{});
-  return p == 4 ? go(I4{}, I4{}) : p == 2 ? go(I4{}, I2{}) : go(I4{}, I1{});
+  return plan.passes == 4   ? go(kgemv_kernel<T, NT, 4>)
+         : plan.passes == 2 ? go(kgemv_kernel<T, NT, 2>)
+                            : go(kgemv_kernel<T, NT, 1>);
 }
 
 template <int T>
@@ -1802,7 +1848,10 @@ int launch_gemv(const QBatch& B, const int64_t* rows, int n_w, const QA& A, cons
   int64_t total = 0;
   for (int i = 0; i < n_w; ++i) total += rows[i];
   if constexpr (is_k(T)) {
-    if (fused && in / 256 <= kgemv_max_sb(n == 1 ? 1 : 4)) return launch_kgemv<T>(B, rows, n_w, x, in, n, s);
+    if (fused && in / 256 <= kgemv_max_sb(int(n)))
+      return n == 1   ? launch_kgemv<T, 1>(B, rows, n_w, x, in, n, s)
+             : n == 2 ? launch_kgemv<T, 2>(B, rows, n_w, x, in, n, s)
+                      : launch_kgemv<T, 4>(B, rows, n_w, x, in, n, s);
   }
   const bool wide = fused && n == 1 && total >= kWideRows;
   const int rw = rows_per_wave(is_k(T), fused ? (n == 1 ? 1 : 4) : (n <= 4 ? 4 : 16), wide);

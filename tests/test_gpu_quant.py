@@ -368,6 +368,32 @@ def test_quant_tiled_legacy_block_counts(backend, t, nb):
         backend.release_weights()
 
 
+@pytest.mark.parametrize("n", [1, 2, 3])
+@pytest.mark.parametrize("t", KTYPES, ids=[U.NAMES[t] for t in KTYPES])
+def test_quant_k_few_rows_layouts(backend, t, n):
+    """Few activation rows over enough weight rows for one, two and four passes in flight and one to several batches a wave,
+    alone and as three weights that each end inside a workgroup. With one row, both sides of the sizes at which Q4_K and Q5_K
+    take the general matvec kernel (16384-32768 weight rows; 6-8 and 16-24 super-blocks). Every output bit-exact."""
+    cases = [(8, (16383,)), (8, (16384,)), (6, (32768,)), (7, (32769,)), (5, (16384,)), (9, (16390,)), (16, (16390,)),
+             (24, (16384,)), (25, (16384,)), (8, (70001,)), (4, (5001, 1003, 999)), (16, (9001, 2001, 2003)),
+             (32, (4099, 1, 1025))]
+    bb = oracle.block_bytes(t)
+    for nb, rows in cases:
+        in_, per = 256 * nb, nb * bb
+        tile = U.random_qmat(t, 61, in_, seed=nb + t).raw
+        ws = [U.QMat(t, np.tile(tile, -(-r // 61))[:r * per], r, in_) for r in rows]
+        x = (np.random.default_rng(nb).standard_normal((n, in_)) * 2).astype(np.float32)
+        with Buffers(backend) as B:
+            dx, ys = B.upload(x), [B.alloc(n * r) for r in rows]
+            backend.matmul_multi(ws, dx, ys, n)
+            got = [backend.download(y, (n, r)) for y, r in zip(ys, rows)]
+        backend.release_weights()
+        ref = oracle.matmul_q(t, tile, in_, 61, x)
+        for g, r in zip(got, rows):  # every row is one of the tile's 61
+            want = np.tile(ref, (1, -(-r // 61)))[:, :r]
+            assert np.array_equal(bits(g), bits(want)), (U.NAMES[t], nb, rows, r, n)
+
+
 @pytest.mark.parametrize("t", KTYPES, ids=[U.NAMES[t] for t in KTYPES])
 def test_quant_k_single_row_wide_and_long(backend, t):
     """One activation row of 65 super-blocks, wider than the K types' kernel for few rows holds, over 16387 weight rows: the
