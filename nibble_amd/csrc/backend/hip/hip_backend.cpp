@@ -14,8 +14,10 @@ namespace nibble::hip {
 namespace {
 
 // Calls with at most this many query rows take the fp32 split-context kernel (decode, short appends).
-// K-type calls of more rows than these take the tiled kernels (the small-call one first): measured faster from
-// there on at the QKV shape than the 16-row gemv launches
+// K-type calls of more rows than these take the tiled kernels (the small-call one first). us a call, 16-row gemv against
+// tiled: Q6_K, QKV of 2048, 5 rows 20.0 / 10.9, 8 rows 28.1 / 11.3. Q4_K, QKV, 5 rows 10.5 / 10.3, 8 rows 13.3 / 10.7;
+// 8192 -> 2048, 5 rows 26.6 / 29.4, 8 rows 36.9 / 31.0; Q5_K likewise: for these two the tiled kernels are ahead from 6
+// rows on already, and at 5 rows where the weights are many (2 x 8192 rows 33.3 / 13.9).
 constexpr int64_t kKTiledMinRows = 8, kQ6KTiledMinRows = 4;
 constexpr int64_t kDecodeMaxRows = NBHS_DECODE_MAX_ROWS;
 constexpr size_t kGemmMaxWeights = NBHS_GEMM_MAX_WEIGHTS;

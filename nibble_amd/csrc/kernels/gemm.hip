@@ -158,16 +158,16 @@ __global__ __launch_bounds__(kSplitThreads) void split_acts_kernel(const float* 
 // while the other waits.
 //  * 64 x 64 tiles with a 3-stage ring while all of them run at once, two to a CU.
 //  * 64 x 128 tiles with a 2-stage ring from kWideMinTiles tiles of 64 x 64 on: each activation byte fetched from L2 serves
-//    twice the products, and no few workgroups are left for a second round. About the line, 64 x 64 against 64 x 128: 4096
-//    weight rows x 448, K = 4096, 448 tiles, 51.5 us a call against 54.2; 5120 x 448, K = 2048, 560 tiles, 41.6 against
-//    36.3; 3072 x 704, K = 8192, 528 tiles, 141 against 116; 2048 x 1152, K = 8192, 576 tiles, 148 against 125.
+//    twice the products, and no few workgroups are left for a second round. About the line, 64 x 64 against 64 x 128: 2048
+//    weight rows x 512, K = 8192, 256 tiles, 68 us a call against 85; 4096 x 448, K = 4096, 448 tiles, 52.2 against 52.7;
+//    3072 x 704, K = 8192, 528 tiles, 152 against 123; 5120 x 448, K = 2048, 560 tiles, 43.4 against 39.4.
 //  * 128 x 128 tiles of 32-deep slices with a 3-stage ring where a row of tiles is so long that its workgroups share few
 //    weight tiles among themselves and every row of tiles reads the weights again: half as many rows of tiles then, from
 //    kHugeMinCols tiles of 128 weight rows and kHugeMinTiles tiles on, if they do not add an empty half row of tiles
 //    (an odd number of 64-row ones), and from kHugeAllCols on always. 64 x 128 against 128 x 128: 110000 weight rows x 128,
 //    K = 2048, 228 us a call against 174; 57344 x 512, K = 8192, 1395 against 1203; 32768 x 512, K = 2048, 169 against 165;
 //    x 448, an odd number, 149 against 157; 20480 x 640, K = 1024, 800 tiles, 73.9 against 75.8, x 768, 960 tiles, 83.2
-//    against 82.2; 16384 x 2048, K = 2048, 312 against 316.
+//    against 82.2; 16384 x 2048, K = 2048, 312 against 316; 28672 x 640, K = 4096, 373 against 383, x 1024 560 against 540.
 // Tiles whose four waves split K and not the outputs (half the LDS reads; one workgroup per CU with a ring of 4-6 slices,
 // the waves' sums added at the end) were no faster: QKV 22.7 us, 16384 x 512 96 us - what the deeper ring gains goes to
 // each workgroup's fixed part, which nothing overlaps.
@@ -177,10 +177,10 @@ constexpr int kHugeBM = 128, kHugeBK = 32, kHugeStages = 3;
 constexpr int64_t kWideMinTiles = 513, kHugeMinCols = 160, kHugeMinTiles = 960, kHugeAllCols = 512;
 // K ranges of a weight whose 64 x 64 tiles are too few to fill the CUs and each walk the whole K: up to kMaxSplit
 // ranges, doubling while the weight's tiles times its ranges stay within kSplitWgs, of at least kFewMinSlices slices in
-// calls of up to kFewMaxRows activation rows (QKV shape, K = 2048, 3072 weight rows: 12-64 rows 27-29 -> 15-19 us per
-// call, 65-128 rows 29-30 -> 19-22) and kMinSlices in longer ones (K = 8192, 2048 weight rows x 140, after a
-// gate + up that is not split: 130 -> 92 us for the block, against 128 x 128 tiles in K ranges). A target of
-// 512 workgroups gained 2-4 us at 192-256 QKV rows but cost gate + up 4-10 us at 32-128 rows. A split weight's partial
+// calls of up to kFewMaxRows activation rows and kMinSlices in longer ones. us a call without and with them: 2048 weight
+// rows, K = 8192, x 24 57.3 / 19.6, x 128 59.8 / 28.2, x 140 60.1 / 38.6, x 256 60.9 / 42.1 (x 512 makes 256 tiles, so no
+// ranges, 65); QKV, 3072 rows, K = 2048, x 24 18.6 / 14.2, x 64 19.1 / 16.8. Where a weight alone makes half of kSplitWgs
+// tiles they cost: QKV x 128 19.8 / 22.1, gate + up of 2 x 8192 rows x 64 22.8 / 28.1. A split weight's partial
 // sums are thus at most kSplitWgs tiles of kBM x kSmallBN; the workspace holds those of kMaxWeights weights (32 MB).
 constexpr int kFewMaxRows = 128, kMaxSplit = 8, kFewMinSlices = 4, kMinSlices = 32;
 constexpr int64_t kSplitWgs = 256;

@@ -697,9 +697,9 @@ __global__ __launch_bounds__(64) void qgemv_kernel(QBatch B, QA A, const float* 
 // the wave's LDS slice and are then added in super-block order, a lane per (row, integer lane) chain: the reference's
 // operations in its order (quant.cpp:118-144, 394-416).
 // A pass of 16 pairs is 2.3-3.4 KB per wave, so P passes are requested before any is computed. What bounds it by its
-// counters: VALU issue at many rows (131072 rows, K = 2048, one activation row: the VALU busy 62 % of the time with Q6_K at
-// 4.2 TB/s, 57 % with Q4_K; waves wait 38-41 % of their time to issue and 23-26 % for loads), the loads' latency at few
-// (2048 rows, K = 8192: 48 % for loads). Two activation rows have an instance of their own, whose LDS leaves room for up to
+// counters: VALU issue at many rows (131072 rows, K = 2048, one activation row: the VALU busy 66 % of the time with Q6_K at
+// 4.6 TB/s, 56 % with Q4_K; waves wait 35-43 % of their time to issue and 26-31 % for loads), the loads' latency at few
+// (2048 rows, K = 8192: the VALU busy 18 %, 46 % of the time waiting for loads). Two activation rows have an instance of their own, whose LDS leaves room for up to
 // four workgroups on a CU; the one for four rows holds two. us a call: 131072 weight rows, K = 2048, Q6_K 48, Q4_K 32; 2048
 // rows, K = 8192, Q6_K 9.9, Q4_K 8.8; 3072 rows, K = 2048, Q4_K 6.1, three activation rows 9.8.
 constexpr int kGemvChunk = 16;  // super-blocks of a pass
@@ -772,7 +772,8 @@ __global__ __launch_bounds__(256) void kgemv_kernel(QBatch B, const float* __res
   };
   load_pass(r00, 0);
   // quantize_row_q8_K (quant.cpp:273-303), the same bits either way: few super-blocks a wave each, four elements per
-  // lane; many eight lanes each, 32 elements per lane
+  // lane; many eight lanes each, 32 elements per lane. A wave each against eight lanes each, us a call with 2048-4096 weight
+  // rows: 8 super-blocks 5.4 / 6.4, 16 (two rows of 8) 7.0 / 6.9, 24 8.8 / 7.5, 32 11.3 / 8.8.
   if (n * nb <= 16) {
     for (int i = wave; i < n * nb; i += 4) {
       const int t = i / nb, sb = i - t * nb, kk = lane >> 3, w = lane & 7;
@@ -1174,7 +1175,7 @@ hipError_t launch_legacy(LegacyTile tile, unsigned tiles, int64_t n, hipStream_t
 // two high bits h, whose MFMAs share an accumulator. Every product and every partial sum is an integer below 2^24
 // (at most 32 * 4096 * 127), so the fp32 accumulator holds float(aux[w]) exactly, whatever the order: no integer
 // slices to combine and no conversion on the VALU, which the float sums bound (per output and residue a product and
-// an addition are left; the int8 form it replaces took two or more MFMAs and four or more VALU operations).
+// an addition are left; int8 operands take two or more MFMAs and four or more VALU operations).
 // The minimum term's sumi = sum_k m_k b_k (b_k: the sub-block's quant sum, |b_k| <= 4064, m_k <= 63) is one
 // v_mfma_f32_16x16x16_f16 over b_k = 64 (b_k >> 6) + (b_k & 63) against (m_k, 64 m_k), likewise exact.
 // The float arithmetic that follows is the reference's per output and block: d = fp16(d_w) * d_a, sums[w] +=
@@ -1308,10 +1309,12 @@ constexpr int vm_lds_wait(int n) { return (n & 15) | (7 << 4) | (0 << 8) | ((n >
 // super-block (scales, d and dmin; the activation rows' d and sum digits) are loaded into registers, each by one wave
 // and each value by one lane, during this super-block and stored to LDS at its end: the L1's rate of lane requests, not
 // bytes, bounded the kernel when every lane loaded the values that it uses (Q4_K, 17408 weight rows x 512 activation
-// rows, K = 2048: 123 us, 118 without the sums; this form 95). What bounds it now is VALU issue (271 operations per
-// wave and super-block, 128 of them the sums) with three waves per SIMD between the loads' latencies. Tiles of 16 x 64
-// and 32 x 32 per wave share an operand build among more sums but take two waves per SIMD and spill: 109 us.
-// Against the int8-slice kernel it replaces: Q4_K QKV (3072 rows x 512, K = 2048) 49 -> 20 us, Q6_K 67 -> 25.
+// rows, K = 2048: 123 us, 118 without the sums; this form 95). What bounds it is VALU issue (316 operations per wave and
+// super-block, 128 of them the sums) with three waves per SIMD between the loads' latencies: by the counters the VALU is
+// busy 78 % of the time at 16384 weight rows x 512 and 48 % at 3072, the matrix cores 18 and 11 %. Tiles of 16 x 64 and 32
+// x 32 per wave share an operand build among more sums but take two waves per SIMD and spill: 109 us. A layer's QKV (3072
+// rows x 512, K = 2048, 16 layers' weights in turn), with int8 slices as operands and with this form: Q4_K 43 and 22 us
+// the kernel, 48.7 and 27.9 with the quantization; Q6_K 61.5 and 27.6, 67.3 and 33.3. (Q5_K spills 12 bytes a lane.)
 template <int T>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void qgemm_k_kernel(QGemmBatch B, QA A,
                                                                                              int64_t n) {
@@ -1749,8 +1752,8 @@ __device__ __forceinline__ float dequant_one(const QW& W, int64_t wb, int e) {
   }
 }
 
-// Row blockIdx.y's elements. (A thread per block, which this replaces, took 40 us for one row of Q6_K, K = 2048: eight
-// threads, 256 dependent loads and stores each; now 5.)
+// Row blockIdx.y's elements: one row of Q6_K, K = 2048, 5 us (with a thread per block, eight threads of 256 dependent
+// loads and stores each, 40).
 template <int T>
 __global__ __launch_bounds__(256) void dequant_rows_kernel(QW W, EmbedIds ids, const int32_t* __restrict__ far_ids,
                                                            int64_t row0, float* __restrict__ out) {
@@ -1846,9 +1849,9 @@ int launch_kgemv(const QBatch& B, const int64_t* rows, int n_w, const float* x, 
 // fill that kernel's chunks of 8 as well as kgemv_kernel's of 16 (6-8, or 16-24): its 2048-4096 waves of eight rows then
 // all run at once, and a lane that unpacks a whole super-block adds its terms itself. us a call, qgemv_kernel against
 // kgemv_kernel: Q4_K, 16384 rows, K = 2048, 8.8 / 9.8; 28672 rows, K = 4096, 20.3 / 22.8; Q5_K, 17920 rows, K = 1536, 10.4 /
-// 12.3; 28672 rows, K = 5120, 32.1 / 36.5. Beyond the lines kgemv_kernel takes 0.7 of the time at 14336 rows (too few
+// 12.3; 28672 rows, K = 5120, 32.5 / 36.8. Beyond the lines kgemv_kernel takes 0.7 of the time at 14336 rows (too few
 // waves), 0.75-0.92 at 36864 (a second round), 0.9-1 at 9 and 12 super-blocks; Q6_K's unpacking keeps a lane too long
-// (12.7 / 11.7 at 16384 rows, K = 2048).
+// (12.7 / 11.6 at 16384 rows, K = 2048).
 constexpr bool wide_row_to_qgemv(int type, int64_t nb, int64_t rows) {
   return type != kQ6_K && rows >= kWideRows && rows <= 2 * kWideRows && ((nb >= 6 && nb <= 8) || (nb >= 16 && nb <= 24));
 }

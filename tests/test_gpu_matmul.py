@@ -337,7 +337,7 @@ def test_f16_gemm_split_k_groups(backend, n, in_, rows):
 
 @pytest.mark.parametrize("n", [9, 12, 16, 17, 40, 64, 96, 128])
 def test_f16_gemm_few_rows_k_ranges(backend, n):
-    """Calls of few activation rows (at most 64) give few 64 x 64 tiles, so each weight takes K ranges of 64 x 64
+    """Calls of few activation rows (at most 128) give few 64 x 64 tiles, so each weight takes K ranges of 64 x 64
     tiles (up to 8, partials summed in range order): 300 and 40 rows at in = 2048 (8 ranges of 4 slices), and a
     100-row weight at in = 1000 (K padded to 1024: ranges of 4 slices, the last one partial), in one call. Within the
     summation bound and against the restated reference, and matmul_multi equals separate calls bit for bit."""
