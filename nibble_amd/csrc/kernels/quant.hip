@@ -1845,24 +1845,13 @@ int launch_kgemv(const QBatch& B, const int64_t* rows, int n_w, const float* x, 
                             : go(kgemv_kernel<T, NT, 1>);
 }
 
-// One activation row of Q4_K or Q5_K against 16384-32768 weight rows stays with qgemv_kernel where the row's super-blocks
-// fill that kernel's chunks of 8 as well as kgemv_kernel's of 16 (6-8, or 16-24): its 2048-4096 waves of eight rows then
-// all run at once, and a lane that unpacks a whole super-block adds its terms itself. us a call, qgemv_kernel against
-// kgemv_kernel: Q4_K, 16384 rows, K = 2048, 8.8 / 9.8; 28672 rows, K = 4096, 20.3 / 22.8; Q5_K, 17920 rows, K = 1536, 10.4 /
-// 12.3; 28672 rows, K = 5120, 32.5 / 36.8. Beyond the lines kgemv_kernel takes 0.7 of the time at 14336 rows (too few
-// waves), 0.75-0.92 at 36864 (a second round), 0.9-1 at 9 and 12 super-blocks; Q6_K's unpacking keeps a lane too long
-// (12.7 / 11.6 at 16384 rows, K = 2048).
-constexpr bool wide_row_to_qgemv(int type, int64_t nb, int64_t rows) {
-  return type != kQ6_K && rows >= kWideRows && rows <= 2 * kWideRows && ((nb >= 6 && nb <= 8) || (nb >= 16 && nb <= 24));
-}
-
 template <int T>
 int launch_gemv(const QBatch& B, const int64_t* rows, int n_w, const QA& A, const float* x, int64_t in, int64_t n,
                 bool fused, hipStream_t s) {
   int64_t total = 0;
   for (int i = 0; i < n_w; ++i) total += rows[i];
   if constexpr (is_k(T)) {
-    if (fused && in / 256 <= kgemv_max_sb(int(n)) && !(n == 1 && wide_row_to_qgemv(T, in / 256, total)))
+    if (fused && in / 256 <= kgemv_max_sb(int(n)))
       return n == 1   ? launch_kgemv<T, 1>(B, rows, n_w, x, in, n, s)
              : n == 2 ? launch_kgemv<T, 2>(B, rows, n_w, x, in, n, s)
                       : launch_kgemv<T, 4>(B, rows, n_w, x, in, n, s);

@@ -372,8 +372,7 @@ def test_quant_tiled_legacy_block_counts(backend, t, nb):
 @pytest.mark.parametrize("t", KTYPES, ids=[U.NAMES[t] for t in KTYPES])
 def test_quant_k_few_rows_layouts(backend, t, n):
     """Few activation rows over enough weight rows for one, two and four passes in flight and one to several batches a wave,
-    alone and as three weights that each end inside a workgroup. With one row, both sides of the sizes at which Q4_K and Q5_K
-    take the general matvec kernel (16384-32768 weight rows; 6-8 and 16-24 super-blocks). Every output bit-exact."""
+    alone and as three weights that each end inside a workgroup. Every output bit-exact."""
     cases = [(8, (16383,)), (8, (16384,)), (6, (32768,)), (7, (32769,)), (5, (16384,)), (9, (16390,)), (16, (16390,)),
              (24, (16384,)), (25, (16384,)), (8, (70001,)), (4, (5001, 1003, 999)), (16, (9001, 2001, 2003)),
              (32, (4099, 1, 1025))]
