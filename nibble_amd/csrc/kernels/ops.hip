@@ -69,42 +69,56 @@ __device__ __forceinline__ double wave_sum_f64(double v) {
 }
 
 // One workgroup per row of d elements. A row is a chain of latencies (its loads, the sum over the workgroup, a square
-// root and two divisions in double), so its elements stay in registers (up to kNormHeld per thread) and every thread
-// finishes the sum by itself: one barrier, no second trip for the scale. One row of 2048: 5.8 -> 4.6 us.
-constexpr int kNormHeld = 8;
+// root and two divisions in double), so its elements stay in registers (up to HELD per thread) and every thread finishes
+// the sum by itself: one barrier, no second trip for the scale. One row of 2048: 5.8 -> 4.6 us. Where many short rows keep
+// the CUs busy, that arithmetic done by all four waves is the time itself: from kNormMany rows of at most kNormShort elements
+// a thread on, one wave does it (ONE) and a second barrier hands the scale on. Every thread against one wave, us: 8192 rows
+// of 64 10.0 / 5.2, of 512 11.8 / 7.3, 2048 rows of 512 4.5 / 3.3, 512 rows 3.3 both; rows of 896 are bound by memory (8192
+// of them 14.6, 16.4 in the form with a second trip for the scale).
+constexpr int kNormHeld = 8, kNormShort = 2, kNormMany = 1024;
+template <int HELD, bool ONE>
 __global__ __launch_bounds__(kThreads) void rmsnorm_kernel(const float* __restrict__ x, const float* __restrict__ w,
                                                            float* __restrict__ y, int64_t d, float eps) {
   __shared__ double part[kThreads / 64];
+  __shared__ double shared_scale;
   const int64_t t = blockIdx.x;
   const float* xt = x + t * d;
-  float held[kNormHeld], wt[kNormHeld];
+  float held[HELD], wt[HELD];
 #pragma unroll
-  for (int c = 0; c < kNormHeld; ++c) {
+  for (int c = 0; c < HELD; ++c) {
     const int64_t i = threadIdx.x + int64_t(c) * kThreads;
     held[c] = i < d ? xt[i] : 0.f;
     wt[c] = i < d ? w[i] : 0.f;
   }
   double ss = 0.0;
 #pragma unroll
-  for (int c = 0; c < kNormHeld; ++c) ss = __dadd_rn(ss, __dmul_rn(double(held[c]), double(held[c])));
-  for (int64_t i = threadIdx.x + kNormHeld * kThreads; i < d; i += kThreads) {
+  for (int c = 0; c < HELD; ++c) ss = __dadd_rn(ss, __dmul_rn(double(held[c]), double(held[c])));
+  for (int64_t i = threadIdx.x + HELD * kThreads; i < d; i += kThreads) {
     const double v = double(xt[i]);
     ss = __dadd_rn(ss, __dmul_rn(v, v));
   }
   ss = wave_sum_f64(ss);
   if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = ss;
   __syncthreads();
-  double s = 0.0;
+  double scale;
+  if (!ONE || threadIdx.x < 64) {
+    double s = 0.0;
 #pragma unroll
-  for (int i = 0; i < kThreads / 64; ++i) s = __dadd_rn(s, part[i]);
-  const double scale = __ddiv_rn(1.0, __dsqrt_rn(__dadd_rn(__ddiv_rn(s, double(d)), double(eps))));
+    for (int i = 0; i < kThreads / 64; ++i) s = __dadd_rn(s, part[i]);
+    scale = __ddiv_rn(1.0, __dsqrt_rn(__dadd_rn(__ddiv_rn(s, double(d)), double(eps))));
+    if (ONE && threadIdx.x == 0) shared_scale = scale;
+  }
+  if constexpr (ONE) {
+    __syncthreads();
+    scale = shared_scale;
+  }
   float* yt = y + t * d;
 #pragma unroll
-  for (int c = 0; c < kNormHeld; ++c) {
+  for (int c = 0; c < HELD; ++c) {
     const int64_t i = threadIdx.x + int64_t(c) * kThreads;
     if (i < d) yt[i] = float(__dmul_rn(__dmul_rn(double(held[c]), scale), double(wt[c])));
   }
-  for (int64_t i = threadIdx.x + kNormHeld * kThreads; i < d; i += kThreads)
+  for (int64_t i = threadIdx.x + HELD * kThreads; i < d; i += kThreads)
     yt[i] = float(__dmul_rn(__dmul_rn(double(xt[i]), scale), double(w[i])));
 }
 
@@ -151,8 +165,12 @@ int nbhs_embed_host_ids(int f16, const void* table, const int32_t* ids, int64_t 
 
 int nbhs_rmsnorm_f32(const float* x, const float* w, float* y, int64_t n, int64_t d, float eps, nbhs_stream s) {
   if (!x || !w || !y || n <= 0 || d <= 0 || n >= (int64_t(1) << 31)) return NBHS_EINVAL;
-  return nbhs_timing::launch(NBHS_K_RMSNORM, rmsnorm_kernel, dim3(unsigned(n)), dim3(kThreads),
-                             reinterpret_cast<hipStream_t>(s), x, w, y, d, eps);
+  const hipStream_t st = reinterpret_cast<hipStream_t>(s);
+  if (d <= kNormShort * kThreads && n >= kNormMany)
+    return nbhs_timing::launch(NBHS_K_RMSNORM, rmsnorm_kernel<kNormShort, true>, dim3(unsigned(n)), dim3(kThreads), st, x, w,
+                               y, d, eps);
+  return nbhs_timing::launch(NBHS_K_RMSNORM, rmsnorm_kernel<kNormHeld, false>, dim3(unsigned(n)), dim3(kThreads), st, x, w, y,
+                             d, eps);
 }
 
 int nbhs_add_f32(float* x, const float* y, int64_t count, nbhs_stream s) {

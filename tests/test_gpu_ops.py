@@ -99,6 +99,26 @@ def test_rmsnorm_rows_beyond_the_registers(backend, n, d):
     backend.release_weights()
 
 
+@pytest.mark.parametrize("n,d", [(1023, 512), (1024, 512), (1024, 513), (1025, 64), (2000, 300), (1100, 1)])
+def test_rmsnorm_many_short_rows(backend, n, d):
+    """Many rows of at most 512 elements, whose scale one wave computes for the workgroup, and both sides of that rule."""
+    rng = np.random.default_rng(n * d)
+    x = (rng.standard_normal((n, d)) * rng.uniform(0.01, 50, (n, 1))).astype(np.float32)
+    w = rng.uniform(0.5, 1.5, d).astype(np.float32)
+    with Buffers(backend) as B:
+        dx, dy = B.upload(x), B.alloc(n * d)
+        backend.rmsnorm(dx, w, dy, n, 1e-5)
+        got = backend.download(dy, (n, d))
+        backend.rmsnorm(dx, w, dx, n, 1e-5)  # in place (x == y) gives the same bits
+        inplace = backend.download(dx, (n, d))
+    ref = oracle.rmsnorm(x, w, 1e-5)
+    u = ulp_diff(got, ref)
+    print(f"rmsnorm n={n} d={d}: {int(np.sum(u > 0))} elements differ, max {int(u.max())} ulp", flush=True)
+    assert int(u.max()) <= 1
+    assert np.array_equal(bits(got), bits(inplace))
+    backend.release_weights()
+
+
 @pytest.mark.parametrize("count", [1, 1000, 8192 * 5 + 3])
 def test_add_and_silu_mul(backend, count):
     rng = np.random.default_rng(count)
