@@ -1719,49 +1719,83 @@ hipError_t launch_k(bool small, unsigned tiles, hipStream_t s, const QGemmBatch&
   return nbhs_timing::launch(NBHS_K_QGEMM, qgemm_k_kernel<T>, grid, dim3(256), s, B, A, n);
 }
 
-// ---- dequantization (quant.cpp:157-242), one thread per output element ----
+// ---- dequantization (quant.cpp:157-242), four output elements per thread ----
 
 // The ids of a call that fit a kernel argument travel in it: no copy to the device, no wait for the stream.
 struct EmbedIds {
   int32_t id[NBHS_EMBED_ARG_IDS];
 };
 
-// Element e of block wb of the weight: the reference's expression for it.
+// Elements e .. e + 3 (e % 4 == 0) of block wb of the weight: the reference's expression for each.
 template <int T>
-__device__ __forceinline__ float dequant_one(const QW& W, int64_t wb, int e) {
+__device__ __forceinline__ floatx4_t dequant_four(const QW& W, int64_t wb, int e) {
   const float d = h2f(W.d[wb]);
-  if constexpr (T == kQ8_0) {
-    return __fmul_rn(float(reinterpret_cast<const int8_t*>(W.q)[wb * 32 + e]), d);
-  } else if constexpr (T == kQ4_0 || T == kQ5_0 || T == kQ5_1) {
-    int q = (W.q[wb * 16 + (e & 15)] >> (e < 16 ? 0 : 4)) & 0x0F;
-    if constexpr (T != kQ4_0) q |= ((reinterpret_cast<const uint32_t*>(W.h)[wb] >> e) & 1u) << 4;
-    if constexpr (T == kQ5_1) return __fadd_rn(__fmul_rn(float(q), d), h2f(W.m[wb]));
-    return __fmul_rn(float(q - (T == kQ4_0 ? 8 : 16)), d);
-  } else if constexpr (T == kQ4_K || T == kQ5_K) {
-    const int k = e >> 5, p = residue_pos(e & 31);
-    int sc, m;
-    scale_min_k4(k, W.s + wb * 16, sc, m);
-    int q = (W.q[wb * 128 + 32 * (k >> 1) + p] >> (4 * (k & 1))) & 0xF;
-    if constexpr (T == kQ5_K) q += ((W.h[wb * 32 + p] >> k) & 1) ? 16 : 0;
-    return __fsub_rn(__fmul_rn(__fmul_rn(d, float(sc)), float(q)), __fmul_rn(h2f(W.m[wb]), float(m)));
-  } else {  // Q6_K
-    const int k = e >> 5, h = k >> 2, g = k & 3, p = residue_pos(e & 31);
-    const int q = (((W.q[wb * 128 + 64 * h + 32 * (g & 1) + p] >> ((g >> 1) * 4)) & 0xF) |
-                   (((W.h[wb * 64 + 32 * h + p] >> (2 * g)) & 3) << 4)) - 32;
-    return __fmul_rn(__fmul_rn(d, float(reinterpret_cast<const int8_t*>(W.s)[wb * 16 + (e >> 4)])), float(q));
+  floatx4_t v;
+  if constexpr (T == kQ8_0 || T == kQ4_0 || T == kQ5_0 || T == kQ5_1) {
+    const uint32_t w = *reinterpret_cast<const uint32_t*>(W.q + (T == kQ8_0 ? wb * 32 + e : wb * 16 + (e & 15)));
+    uint32_t h = 0;
+    if constexpr (T == kQ5_0 || T == kQ5_1) h = reinterpret_cast<const uint32_t*>(W.h)[wb] >> e;
+    float m = 0.f;
+    if constexpr (T == kQ5_1) m = h2f(W.m[wb]);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      if constexpr (T == kQ8_0) {
+        v[j] = __fmul_rn(float(int8_t(w >> (8 * j))), d);
+      } else {
+        int q = (w >> (8 * j + (e < 16 ? 0 : 4))) & 0x0F;
+        if constexpr (T != kQ4_0) q |= ((h >> j) & 1u) << 4;
+        v[j] = T == kQ5_1 ? __fadd_rn(__fmul_rn(float(q), d), m) : __fmul_rn(float(q - (T == kQ4_0 ? 8 : 16)), d);
+      }
+    }
+  } else {
+    // byte i of words w .. w + 3 of sub-block k's residue-ordered group
+    const int k = e >> 5, w = e & 7, i = (e >> 3) & 3;
+    if constexpr (T == kQ4_K || T == kQ5_K) {
+      int sc, mn;
+      scale_min_k4(k, W.s + wb * 16, sc, mn);
+      const u32x4_t qw = *reinterpret_cast<const u32x4_t*>(W.q + wb * 128 + 32 * (k >> 1) + 4 * w);
+      u32x4_t hw;
+      if constexpr (T == kQ5_K) hw = *reinterpret_cast<const u32x4_t*>(W.h + wb * 32 + 4 * w);
+      const float ds = __fmul_rn(d, float(sc)), ms = __fmul_rn(h2f(W.m[wb]), float(mn));
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        int q = (qw[j] >> (8 * i + 4 * (k & 1))) & 0xF;
+        if constexpr (T == kQ5_K) q += ((hw[j] >> (8 * i + k)) & 1) ? 16 : 0;
+        v[j] = __fsub_rn(__fmul_rn(ds, float(q)), ms);
+      }
+    } else {  // Q6_K
+      const int h = k >> 2, g = k & 3;
+      const u32x4_t qw = *reinterpret_cast<const u32x4_t*>(W.q + wb * 128 + 64 * h + 32 * (g & 1) + 4 * w);
+      const u32x4_t hw = *reinterpret_cast<const u32x4_t*>(W.h + wb * 64 + 32 * h + 4 * w);
+      const float ds = __fmul_rn(d, float(reinterpret_cast<const int8_t*>(W.s)[wb * 16 + (e >> 4)]));
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int q = int(((qw[j] >> (8 * i + 4 * (g >> 1))) & 0xF) | (((hw[j] >> (8 * i + 2 * g)) & 3) << 4)) - 32;
+        v[j] = __fmul_rn(ds, float(q));
+      }
+    }
   }
+  return v;
 }
 
-// Row blockIdx.y's elements: one row of Q6_K, K = 2048, 5 us (with a thread per block, eight threads of 256 dependent
-// loads and stores each, 40).
+// Row blockIdx.y's elements, four a thread: word loads and 16-byte stores, a block's scales once. us for one row of Q6_K,
+// K = 2048, 5 (with a thread per block, eight threads of 256 dependent loads and stores each, 40); 4096 rows, K = 4096, Q8_0
+// 27, Q4_K 31, Q6_K 29 (with a thread per element 44, 58 and 54).
 template <int T>
 __global__ __launch_bounds__(256) void dequant_rows_kernel(QW W, EmbedIds ids, const int32_t* __restrict__ far_ids,
-                                                           int64_t row0, float* __restrict__ out) {
+                                                           int64_t row0, float* __restrict__ out, int vec) {
   constexpr int be = int(block_elems(T));
-  const int64_t in = W.nb * be, i = int64_t(blockIdx.x) * 256 + threadIdx.x, t = row0 + blockIdx.y;
+  const int64_t in = W.nb * be, i = 4 * (int64_t(blockIdx.x) * 256 + threadIdx.x), t = row0 + blockIdx.y;
   if (i >= in) return;
-  const int64_t id = far_ids ? far_ids[t] : ids.id[blockIdx.y];
-  out[t * in + i] = dequant_one<T>(W, id * W.nb + i / be, int(i % be));
+  const int64_t id = far_ids ? far_ids[t] : ids.id[blockIdx.y], wb = id * W.nb + i / be;
+  const floatx4_t v = dequant_four<T>(W, wb, int(i % be));
+  float* const o = out + t * in + i;
+  if (vec) {
+    *reinterpret_cast<floatx4_t*>(o) = v;
+  } else {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) o[j] = v[j];
+  }
 }
 
 QW weight_of(int type, const void* w, int64_t rows, int64_t in) {
@@ -1879,12 +1913,13 @@ int launch_gemv(const QBatch& B, const int64_t* rows, int n_w, const QA& A, cons
 template <int T>
 int launch_dequant(const QW& W, const int32_t* host_ids, const int32_t* ids, int64_t n, float* out, hipStream_t s) {
   const int64_t in = W.nb * block_elems(T);
+  const int vec = reinterpret_cast<uintptr_t>(out) % 16 == 0 ? 1 : 0;  // (a row is whole blocks: multiples of 32 floats)
   EmbedIds arg{};
   if (host_ids) std::copy(host_ids, host_ids + n, arg.id);
   for (int64_t t0 = 0; t0 < n; t0 += 65535) {
-    const dim3 grid{unsigned((in + 255) / 256), unsigned(std::min<int64_t>(n - t0, 65535))};
+    const dim3 grid{unsigned((in + 1023) / 1024), unsigned(std::min<int64_t>(n - t0, 65535))};
     const hipError_t e = nbhs_timing::launch(NBHS_K_ELEMENTWISE, dequant_rows_kernel<T>, grid, dim3(256), s, W, arg,
-                                             host_ids ? nullptr : ids, t0, out);
+                                             host_ids ? nullptr : ids, t0, out, vec);
     if (e != hipSuccess) return e;
   }
   return hipSuccess;

@@ -83,16 +83,18 @@ def test_quant_embed_bit_exact(backend, t):
 @pytest.mark.parametrize("n", [511, 512, 513, 1500])
 @pytest.mark.parametrize("t", TYPES, ids=[U.NAMES[t] for t in TYPES])
 def test_quant_embed_many_ids(backend, t, n):
-    """512 ids travel in the launch, more in a device buffer; rows of one workgroup and more."""
-    d = 512 if oracle.block_elems(t) == 256 else 288
-    table = U.random_qmat(t, 50, d, seed=90 + t)
-    ids = np.random.default_rng(n).integers(0, 50, n).astype(np.int32)
-    with Buffers(backend) as B:
-        out = B.alloc(n * d)
-        backend.embed(table, ids, out)
-        got = backend.download(out, (n, d))
-    assert np.array_equal(bits(got), bits(np.asarray(table)[ids]))
-    backend.release_weights()
+    """512 ids travel in the launch, more in a device buffer; rows of part of a workgroup, one and more; an output that is
+    16-byte aligned (vector stores) and one that is not."""
+    for d in (512, 1280) if oracle.block_elems(t) == 256 else (288, 1056):
+        table = U.random_qmat(t, 50, d, seed=90 + t)
+        ids = np.random.default_rng(n).integers(0, 50, n).astype(np.int32)
+        with Buffers(backend) as B:
+            buf = B.alloc(n * d + 3)
+            for out in (buf, buf.at(3)):
+                backend.embed(table, ids, out)
+                got = backend.download(out, (n, d))
+                assert np.array_equal(bits(got), bits(np.asarray(table)[ids]))
+        backend.release_weights()
 
 
 @pytest.mark.parametrize("n", [2, 100])
