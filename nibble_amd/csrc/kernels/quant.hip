@@ -697,9 +697,9 @@ __global__ __launch_bounds__(64) void qgemv_kernel(QBatch B, QA A, const float* 
 // the wave's LDS slice and are then added in super-block order, a lane per (row, integer lane) chain: the reference's
 // operations in its order (quant.cpp:118-144, 394-416).
 // A pass of 16 pairs is 2.3-3.4 KB per wave, so P passes are requested before any is computed. What bounds it by its
-// counters: VALU issue at many rows (131072 rows, K = 2048, one activation row: the VALU busy 66 % of the time with Q6_K at
-// 4.6 TB/s, 56 % with Q4_K; waves wait 35-43 % of their time to issue and 26-31 % for loads), the loads' latency at few
-// (2048 rows, K = 8192: the VALU busy 18 %, 46 % of the time waiting for loads). Two activation rows have an instance of their own, whose LDS leaves room for up to
+// counters: VALU issue at many rows (131072 rows, K = 2048, one activation row: the VALU busy 67 % of the time with Q6_K at
+// 4.5 TB/s, 58 % with Q4_K; waves wait 35-42 % of their time to issue and 26-30 % for loads), the loads' latency at few
+// (2048 rows, K = 8192: the VALU busy 18 %, 47 % of the time waiting for loads). Two activation rows have an instance of their own, whose LDS leaves room for up to
 // four workgroups on a CU; the one for four rows holds two. us a call: 131072 weight rows, K = 2048, Q6_K 48, Q4_K 32; 2048
 // rows, K = 8192, Q6_K 9.9, Q4_K 8.8; 3072 rows, K = 2048, Q4_K 6.1, three activation rows 9.8.
 constexpr int kGemvChunk = 16;  // super-blocks of a pass
