@@ -699,9 +699,10 @@ __global__ __launch_bounds__(64) void qgemv_kernel(QBatch B, QA A, const float* 
 // A pass of 16 pairs is 2.3-3.4 KB per wave, so P passes are requested before any is computed. What bounds it by its
 // counters: VALU issue at many rows (131072 rows, K = 2048, one activation row: the VALU busy 67 % of the time with Q6_K at
 // 4.5 TB/s, 58 % with Q4_K; waves wait 35-42 % of their time to issue and 26-30 % for loads), the loads' latency at few
-// (2048 rows, K = 8192: the VALU busy 18 %, 47 % of the time waiting for loads). Two activation rows have an instance of their own, whose LDS leaves room for up to
-// four workgroups on a CU; the one for four rows holds two. us a call: 131072 weight rows, K = 2048, Q6_K 48, Q4_K 32; 2048
-// rows, K = 8192, Q6_K 9.9, Q4_K 8.8; 3072 rows, K = 2048, Q4_K 6.1, three activation rows 9.8.
+// (2048 rows, K = 8192: the VALU busy 18 %, 47 % of the time waiting for loads). Two activation rows have an instance of
+// their own, whose LDS leaves room for up to four workgroups on a CU; the one for four rows holds two. us a call: 131072
+// weight rows, K = 2048, Q6_K 48, Q4_K 32; 2048 rows, K = 8192, Q6_K 9.9, Q4_K 8.8; 3072 rows, K = 2048, Q4_K 6.1, three
+// activation rows 9.8.
 constexpr int kGemvChunk = 16;  // super-blocks of a pass
 constexpr int kgemv_max_sb(int nt) { return nt == 1 ? 64 : 32; }  // super-blocks of a row, at most (LDS)
 
